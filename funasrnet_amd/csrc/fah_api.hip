@@ -353,8 +353,10 @@ struct fah_weight {
   bool half_scales = true;
   DeviceBuffer q, s;
   int group_rows = 1;
-  // FP32 weight (Weight.Values): `f` holds [rows][cols] floats, q/s unused.
+  // FP32 weight (Weight.Values): `f` holds [rows][cols] floats and their bf16
+  // planes (fah::f32_weight_bytes), q/s unused.
   bool f32 = false;
+  bool splittable = false;
   DeviceBuffer f;
 };
 
@@ -1580,7 +1582,14 @@ int fah_weight_f32_upload(fah_context* h, const float* values, int rows, int col
     w->rows = rows;
     w->cols = cols;
     w->f32 = true;
-    upload(w->f, values, (size_t)rows * cols * 4, c->stream);
+    w->f.allocate(fah::f32_weight_bytes(rows, cols));
+    check(hipMemcpyAsync(w->f.ptr, values, (size_t)rows * cols * 4, hipMemcpyHostToDevice, c->stream), "H2D weight");
+    check(fah::launch_f32_split(w->f.as<float>(), rows, cols, c->stream), "split weight");
+    int outside = 0;
+    check(hipMemcpyAsync(&outside, fah::f32_weight_outside(w->f.as<float>(), rows, cols), 4, hipMemcpyDeviceToHost, c->stream),
+          "D2H range");
+    check(hipStreamSynchronize(c->stream), "hipStreamSynchronize");
+    w->splittable = outside == 0;
     *out = w.release();
     return FAH_OK;
   });
@@ -1776,7 +1785,7 @@ int fah_linear_many(fah_context* h, const float* input, int frames, const fah_we
       size_t at = 0;
       for (int i = 0; i < count; ++i) {
         check(fah::launch_f32_linear(c->in.as<float>(), weights[i]->f.as<float>(), nullptr, c->out.as<float>() + at,
-                                     frames, weights[i]->rows, cols, false, c->stream),
+                                     frames, weights[i]->rows, cols, false, weights[i]->splittable, c->stream),
               "f32 linear");
         at += (size_t)frames * weights[i]->rows;
       }
@@ -1840,7 +1849,7 @@ int fah_linear(fah_context* h, const float* input, int frames, const fah_weight*
     }
     meter.kernels_begin();
     check(fah::launch_f32_linear(c->in.as<float>(), w->f.as<float>(), dbias, c->out.as<float>(), frames, w->rows,
-                                 w->cols, false, c->stream),
+                                 w->cols, false, w->splittable, c->stream),
           "f32 linear");
     meter.kernels_end();
     check(hipMemcpyAsync(output, c->out.ptr, out_bytes, hipMemcpyDeviceToHost, c->stream), "D2H output");
@@ -1862,7 +1871,7 @@ int fah_linear_device(fah_context* h, const float* x, int frames, const fah_weig
     if (c->disposed) return fail(FAH_ERROR_DISPOSED, "context disposed");
     check(hipSetDevice(c->device), "hipSetDevice");
     DeviceWork work(*c);
-    check(fah::launch_f32_linear(x, w->f.as<float>(), bias, out, frames, w->rows, w->cols, false, c->stream),
+    check(fah::launch_f32_linear(x, w->f.as<float>(), bias, out, frames, w->rows, w->cols, false, w->splittable, c->stream),
           "f32 linear");
     return FAH_OK;
   });
@@ -1902,9 +1911,9 @@ int fah_relu_projection(fah_context* h, const float* input, int frames, const fa
     float* dout = reinterpret_cast<float*>(c->out.as<char>() + mid_bytes);
     // The intermediate stays on the device (IReluProjectionBackend.cs:4-16).
     meter.kernels_begin();
-    check(fah::launch_f32_linear(c->in.as<float>(), first->f.as<float>(), d1, mid, frames, H, K, true, c->stream),
+    check(fah::launch_f32_linear(c->in.as<float>(), first->f.as<float>(), d1, mid, frames, H, K, true, first->splittable, c->stream),
           "f32 linear + ReLU");
-    check(fah::launch_f32_linear(mid, second->f.as<float>(), d2, dout, frames, N, H, false, c->stream), "f32 linear");
+    check(fah::launch_f32_linear(mid, second->f.as<float>(), d2, dout, frames, N, H, false, second->splittable, c->stream), "f32 linear");
     meter.kernels_end();
     check(hipMemcpyAsync(output, dout, out_bytes, hipMemcpyDeviceToHost, c->stream), "D2H output");
     work.release();  // enqueued: other contexts may enqueue while this stream drains

@@ -22,276 +22,422 @@ namespace {
 
 typedef float floatx4 __attribute__((ext_vector_type(4)));
 
-// ---- GEMM on fp32 MFMA --------------------------------------------------------
-// out[f][n] = sum_k x[f][k] * w[n][k] (+ bias[n]) (ReLU), any M (frames), N,
-// K with K % 4 == 0 and 16-byte aligned rows. Four waves in a 2 x 2 grid,
-// each a (16 BI) x (16 BJ) tile of v_mfma_f32_16x16x4f32 blocks; workgroup
-// tile (32 BI) x (32 BJ); K in tiles of GK staged in two LDS buffers as
-// row-major [row][GK + 4] (16-byte loads and stores; the next tile's global
-// loads sit in registers while the current one is multiplied, then go to
-// the other buffer, one barrier per tile). Lane layout of 16x16x4: A[i][k]
-// from lane i + 16k, B[k][j] from lane j + 16k, D[4q + r][j] in lane j + 16q
-// (r < 4). In substep s of a K tile, lane group q multiplies k =
-// (GK / 4) q + s, so each lane reads its GK / 4 values of a row as 16-byte
-// LDS reads. One order per shape: the same bits whichever entry point runs it.
-#ifndef FAH_GK
-#define FAH_GK 64
-#endif
-constexpr int kGK = FAH_GK;
+// ---- GEMM: FP32 products on the bf16 matrix cores --------------------------------
+// out[f][n] = sum_k x[f][k] * w[n][k] (+ bias[n]) (ReLU), any M (frames), N, K.
+//
+// What bounds it: fp32 MFMA does 256 flop a cycle and CU, bf16 MFMA 4,096.
+// Every fp32 value is the exact sum of three bf16 values (each the rest
+// rounded to nearest: 8 + 8 + 8 significand bits), so a product of two is the
+// sum of nine bf16 products that fp32 holds exactly; the six largest are
+// formed (a0 b0, a0 b1, a1 b0, a1 b1, a0 b2, a2 b0), the other three are below
+// 2^-25 of the product, half an ulp of its fp32 rounding. Six bf16 MFMAs of 16
+// k take 6 x 32 cycles for a 32 x 32 tile where fp32 ones take 4 x 4 x 32, and
+// round the sum six times for 16 k instead of sixteen times.
+//
+// Layout: a workgroup of WN x KS waves takes 32 TI frames and 32 TJ WN rows in
+// v_mfma_f32_32x32x16_bf16 tiles, each wave all the frames and 32 TJ rows, K in
+// tiles of 32 KB k of which wave group ks takes the 16-k steps ks HS .. ks HS +
+// HS - 1; the groups' sums are added in LDS in order. The weight's planes were
+// laid out at upload in the lanes' own order, so a wave reads its operands
+// straight from memory, 1 KB at a time (through LDS they took 22.8 us where
+// this takes 20.4 for 1000 x 512 -> 2048: LDS reads, then L1 fills of half
+// lines). A thread loads 8 k of a frame (32 bytes), splits them and writes 16
+// bytes to each of three LDS planes, in the shadow of the previous tile's MFMAs;
+// 16-byte chunks are placed so that the rows of an operand read and of a write
+// fall on distinct banks (SQ_LDS_BANK_CONFLICT 0). Two LDS buffers, one barrier
+// a tile. Results leave by non-temporal stores (18.3 -> 17.6 us: the write-back
+// at the kernel's end shortens). Operand lane layout: row l % 32, k 8 (l / 32)
+// .. + 7; result register r of lane l: row 8 (r / 4) + 4 (l / 32) + r % 4,
+// column l % 32.
+//
+// Measured against the fp32 MFMA kernel before it (fp32 sums of 64 x 64 tiles),
+// us: 1000 x 512 -> 2048 25.3 -> 19.5, 333 x 560 -> 1536 17.2 -> 11.8, 4000 x
+// 2048 -> 512 84.7 -> 54.1, 300 x 1023 -> 700 170 -> 19.2; error against 64 bits
+// (2-norm) 4.0e-7 -> 0.97e-7, 4.2e-7 -> 1.0e-7, 8.1e-7 -> 1.9e-7, 5.7e-7 ->
+// 1.0e-7. Of the 19.5, the MFMAs take 6.2 (at the 2.0 GHz seen), the 8 MB of
+// stores 3, the launch, first loads and epilogue the rest.
+//
+// Range: a weight is split only if its values are at most kSplitMost in
+// magnitude and no row but a zero one lies below kSplitRowLeast (checked once,
+// at upload). What bf16 planes cannot hold of a frame is then below 2^-126
+// 2^20 K in a sum. Frames with infinities, NaN or values that round past the
+// largest bf16 make sums infinite or NaN; a workgroup that finds such a sum,
+// one below kSplitLow, or zeros and frames with values below kSplitTiny, forms
+// its tile again on fp32 MFMA (tile_f32).
+constexpr uint32_t kSplitLow = 0x1c800000u;      // 2^-70
+constexpr uint32_t kSplitTiny = 0x0d800000u;     // 2^-100
+constexpr uint32_t kSplitMost = 0x49800000u;     // 2^20
+constexpr uint32_t kSplitRowLeast = 0x17800000u; // 2^-80
 
-template <int BI, int BJ, bool RELU>
-__global__ __launch_bounds__(256) void f32_gemm_kernel(const float* __restrict__ x, const float* __restrict__ w,
-                                                       const float* __restrict__ bias, float* __restrict__ out, int M,
-                                                       int N, int K) {
-  constexpr int TM = 32 * BI, TN = 32 * BJ;              // workgroup tile
-  constexpr int ROW = kGK + 4, KQ = kGK / 4;              // LDS row (floats); k values per lane group
-  constexpr int PER_ROW = kGK / 4, ROWS = 256 / PER_ROW;  // 16-byte loads per row; rows per pass
-  constexpr int LA = TM / ROWS, LB = TN / ROWS;           // 16-byte loads per thread and operand
-  static_assert(LA >= 1 && LB >= 1 && TM % ROWS == 0 && TN % ROWS == 0, "whole load passes");
-  __shared__ __attribute__((aligned(16))) float a_s[2][TM * ROW];
-  __shared__ __attribute__((aligned(16))) float b_s[2][TN * ROW];
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef float floatx2 __attribute__((ext_vector_type(2)));
+typedef float floatx16 __attribute__((ext_vector_type(16)));
+
+__device__ __forceinline__ uint32_t pack_bf16(float a, float b) {
+  const floatx2 v = {a, b};
+  uint32_t r = __builtin_bit_cast(uint32_t, __builtin_convertvector(v, bf16x2));
+  asm("" : "+v"(r));  // (one conversion: the halves are taken from the packed word)
+  return r;
+}
+
+// Eight floats as three planes of eight bf16.
+__device__ __forceinline__ void split8(const float* v, uint4* p) {
+  uint32_t w[3][4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    float a = v[2 * i], b = v[2 * i + 1];
+#pragma unroll
+    for (int s = 0; s < 3; ++s) {
+      const uint32_t h = pack_bf16(a, b);
+      w[s][i] = h;
+      if (s < 2) {
+        a -= u2f(h << 16);
+        b -= u2f(h & 0xffff0000u);
+      }
+    }
+  }
+#pragma unroll
+  for (int s = 0; s < 3; ++s) p[s] = make_uint4(w[s][0], w[s][1], w[s][2], w[s][3]);
+}
+
+// Planes of a weight, in the order the GEMM's lanes hold them: for each 32
+// rows and 16 k a fragment of [plane 3][lane 64] 16-byte pieces, lane l holding
+// row l % 32, k 8 (l / 32) .. + 7. Rows are padded to 32 with the last one (no zero
+// sums that the matrix does not have), k with zeros to 128.
+__host__ __device__ inline int split_k16(int K) { return ((K + 127) & ~127) / 16; }
+__host__ __device__ inline int64_t split_pieces(int64_t rows, int K) { return (rows + 31) / 32 * split_k16(K) * 192; }
+
+__global__ __launch_bounds__(256) void f32_split_planes_kernel(const float* __restrict__ w, int64_t rows, int K,
+                                                               uint4* __restrict__ planes) {
+  const int64_t fragments = (rows + 31) / 32 * split_k16(K), total = fragments * 64;
+  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < total; i += (int64_t)gridDim.x * 256) {
+    const int lane = (int)(i & 63);
+    const int64_t fragment = i >> 6, r = min(fragment / split_k16(K) * 32 + (lane & 31), rows - 1);
+    const int k = (int)(fragment % split_k16(K)) * 16 + 8 * (lane >> 5);
+    float v[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) v[e] = k + e < K ? w[r * K + k + e] : 0.0f;
+    uint4 p[3];
+    split8(v, p);
+#pragma unroll
+    for (int s = 0; s < 3; ++s) planes[fragment * 192 + 64 * s + lane] = p[s];
+  }
+}
+
+// Sets *outside for a weight that is not to be split (one wave a row).
+__global__ __launch_bounds__(256) void f32_split_range_kernel(const float* __restrict__ w, int64_t rows, int K,
+                                                              int* outside) {
+  const int lane = threadIdx.x & 63;
+  for (int64_t r = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6); r < rows; r += (int64_t)gridDim.x * 4) {
+    uint32_t most = 0u;
+    for (int k = lane; k < K; k += 64) most = max(most, f2u(w[r * K + k]) & 0x7fffffffu);
+#pragma unroll
+    for (int m = 32; m >= 1; m >>= 1) most = max(most, (uint32_t)__shfl_xor((int)most, m, 64));
+    if (lane == 0 && (most > kSplitMost || (most != 0u && most < kSplitRowLeast))) *outside = 1;
+  }
+}
+
+// Eight k of a row from k on, clamped into the row: what lies past K meets the
+// weight planes' zeros. VEC: K % 4 == 0 and 16-byte aligned rows.
+template <bool VEC>
+__device__ __forceinline__ void load8(const float* row, int k, int K, float* v) {
+  if (VEC) {
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const float4 q = *reinterpret_cast<const float4*>(row + min(k + 4 * h, K - 4));
+      v[4 * h] = q.x;
+      v[4 * h + 1] = q.y;
+      v[4 * h + 2] = q.z;
+      v[4 * h + 3] = q.w;
+    }
+  } else {
+#pragma unroll
+    for (int i = 0; i < 8; ++i) v[i] = row[min(k + i, K - 1)];
+  }
+}
+
+__device__ __forceinline__ void store_linear(float v, const float* bias, float* out, int f, int n, int M, int N,
+                                             bool relu) {
+  if (f < M && n < N) {
+    v = v + (bias ? bias[n] : 0.0f);
+    if (relu) v = v < 0.0f ? 0.0f : v;
+    out[(size_t)f * N + n] = v;
+  }
+}
+
+// A TM x TN tile on fp32 MFMA, any K and alignment: K in steps of 32 staged in
+// LDS, one float per thread and row; wave w takes the 16 x 16 blocks w, w + WAVES,
+// ... Lane layout of 16x16x4: A[i][k] from lane i + 16k, B[k][j] from lane
+// j + 16k, D[4q + r][j] in lane j + 16q.
+template <int TM, int TN, int WAVES>
+__device__ __forceinline__ void tile_f32(char* smem, const float* x, const float* w, const float* bias, float* out, int M,
+                                      int N, int K, int f0, int n0, bool relu) {
+  constexpr int PAD = 33, BLOCKS = (TM / 16) * (TN / 16), PER = BLOCKS / WAVES, NT = 64 * WAVES;
+  static_assert(BLOCKS % WAVES == 0, "whole blocks a wave");
+  float* s = reinterpret_cast<float*>(smem);  // [TM + TN][PAD]
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-  const int f0 = blockIdx.y * TM, n0 = blockIdx.x * TN;
-  const int wm = (wave >> 1) * 16 * BI, wn = (wave & 1) * 16 * BJ;
-  const int li = lane & 15, lq = lane >> 4;
-  floatx4 acc[BI][BJ];
+  floatx4 acc[PER];
 #pragma unroll
-  for (int i = 0; i < BI; ++i)
+  for (int b = 0; b < PER; ++b) acc[b] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+  for (int k0 = 0; k0 < K; k0 += 32) {
+    __syncthreads();
+    const int k = k0 + (tid & 31);
+    for (int r = tid >> 5; r < TM + TN; r += NT / 32) {
+      const int f = f0 + r, n = n0 + r - TM;
+      float v = 0.0f;
+      if (k < K) {
+        if (r < TM) v = f < M ? x[(size_t)f * K + k] : 0.0f;
+        else v = n < N ? w[(size_t)n * K + k] : 0.0f;
+      }
+      s[r * PAD + (tid & 31)] = v;
+    }
+    __syncthreads();
+    for (int ks = 0; ks < 32; ks += 4) {
+      const int kk = ks + (lane >> 4);
 #pragma unroll
-    for (int j = 0; j < BJ; ++j) acc[i][j] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
-  // Global loads: thread t takes row t / PER_ROW (+ ROWS per further load),
-  // the 16 bytes at k = 4 (t % PER_ROW) of the tile; rows past the edge and
-  // k past K read as zero.
-  const int lr = tid / PER_ROW, lc = 4 * (tid % PER_ROW);
-  float4 ra[LA], rb[LB];
-  auto fetch = [&](int k0) {
-    const int k = k0 + lc;
+      for (int b = 0; b < PER; ++b) {
+        const int blk = wave + WAVES * b, bi = blk % (TM / 16), bj = blk / (TM / 16);
+        acc[b] = __builtin_amdgcn_mfma_f32_16x16x4f32(s[(16 * bi + (lane & 15)) * PAD + kk],
+                                                      s[(TM + 16 * bj + (lane & 15)) * PAD + kk], acc[b], 0, 0, 0);
+      }
+    }
+  }
 #pragma unroll
-    for (int u = 0; u < LA; ++u) {
-      const int f = f0 + lr + ROWS * u;
-      ra[u] = (f < M && k < K) ? *reinterpret_cast<const float4*>(x + (size_t)f * K + k) : make_float4(0.f, 0.f, 0.f, 0.f);
+  for (int b = 0; b < PER; ++b) {
+    const int blk = wave + WAVES * b, bi = blk % (TM / 16), bj = blk / (TM / 16);
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+      store_linear(acc[b][r], bias, out, f0 + 16 * bi + 4 * (lane >> 4) + r, n0 + 16 * bj + (lane & 15), M, N, relu);
+  }
+}
+
+// 16-byte slot of chunk c of row r in a plane of rows of CH chunks (4 or 8).
+template <int CH>
+__device__ __forceinline__ int split_slot(int row, int chunk) {
+  const int swz = CH == 8 ? row & 7 : ((row >> 1) & 3) ^ ((row >> 3) & 1);
+  return (row * CH + (chunk ^ swz)) * 16;
+}
+
+template <int WN, int KS, int TI, int TJ, int KB, int D, bool VEC>
+__global__ __launch_bounds__(64 * WN * KS) void f32_split_gemm_kernel(
+    const float* __restrict__ x, const float* __restrict__ w, const uint4* __restrict__ planes,
+    const float* __restrict__ bias, float* __restrict__ out, int M, int N, int K, int relu, int splittable) {
+  constexpr int TM = 32 * TI, TN = 32 * TJ * WN, WAVES = WN * KS, NT = 64 * WAVES, KT = 32 * KB;
+  constexpr int CH = KT / 8, PLANE = TM * KT * 2, BUF = 3 * PLANE, UA = TM * CH / NT, HS = 2 * KB / KS;
+  static_assert(D % 2 == 0 && 128 % (D * KT) == 0, "two LDS buffers; planes padded to whole groups of D tiles");
+  static_assert(UA >= 1 && UA * NT == TM * CH && HS * KS == 2 * KB, "whole units a thread, whole 16-k steps a wave");
+  constexpr int kReduce = (KS - 1) * WN * TI * TJ * 4096;  // partial tiles of the other wave groups
+  constexpr int kFallback = (TM + TN) * 33 * 4;
+  constexpr int kMax = kReduce > kFallback ? kReduce : kFallback, kLds = 2 * BUF > kMax ? 2 * BUF : kMax;
+  __shared__ __attribute__((aligned(16))) char smem[kLds];
+  __shared__ int unsure_s;
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, l32 = lane & 31, lk = lane >> 5;
+  const int ks = wave / WN, wn = wave % WN;
+  // Workgroups are dealt to the eight XCDs in turn: each XCD takes a run of
+  // consecutive tiles, frames fastest, so that its L2 holds few weight rows.
+  const int mt = (M + TM - 1) / TM, tiles = gridDim.x, xcd = blockIdx.x & 7, q8 = tiles >> 3, r8 = tiles & 7;
+  const int tile = xcd * q8 + min(xcd, r8) + (blockIdx.x >> 3);
+  const int f0 = (tile % mt) * TM, n0 = (tile / mt) * TN;
+  auto split_tile = [&]() -> bool {
+    // Frames past the end repeat the last one, row blocks past the end the
+    // last block (neither is stored).
+    const float* asrc[UA];
+    int aat[UA];
+#pragma unroll
+    for (int u = 0; u < UA; ++u) {
+      const int unit = tid + NT * u, row = unit / CH;
+      asrc[u] = x + (size_t)min(f0 + row, M - 1) * K;
+      aat[u] = split_slot<CH>(row, unit % CH);
+    }
+    const int k16 = split_k16(K), steps = (K + D * KT - 1) / (D * KT) * D, kc = 8 * (tid % CH);
+    const uint4* bsrc[TJ];
+#pragma unroll
+    for (int j = 0; j < TJ; ++j)
+      bsrc[j] = planes + ((size_t)min(n0 / 32 + TJ * wn + j, (N - 1) / 32) * k16 + ks * HS) * 192 + lane;
+    struct Regs {
+      float a[UA][8];
+      uint4 b[TJ][HS][3];
+    } r[D];
+    auto fetch_a = [&](Regs& r, int t) {
+      t = min(t, steps - 1);
+#pragma unroll
+      for (int u = 0; u < UA; ++u) load8<VEC>(asrc[u], KT * t + kc, K, r.a[u]);
+    };
+    auto fetch_b = [&](Regs& r, int t) {
+      t = min(t, steps - 1);
+#pragma unroll
+      for (int j = 0; j < TJ; ++j)
+#pragma unroll
+        for (int h = 0; h < HS; ++h)
+#pragma unroll
+          for (int s = 0; s < 3; ++s) r.b[j][h][s] = bsrc[j][(size_t)(2 * KB * t + h) * 192 + 64 * s];
+    };
+    auto stage = [&](Regs& r, int buf) {
+#pragma unroll
+      for (int u = 0; u < UA; ++u) {
+        uint4 p[3];
+        split8(r.a[u], p);
+#pragma unroll
+        for (int s = 0; s < 3; ++s) *reinterpret_cast<uint4*>(smem + buf * BUF + s * PLANE + aat[u]) = p[s];
+      }
+    };
+    // The large products a0 b0 and the five corrections have sums of their own:
+    // the first is rounded once for 16 k, the others are small.
+    floatx16 acc[TI][TJ], rest[TI][TJ];
+#pragma unroll
+    for (int i = 0; i < TI; ++i)
+#pragma unroll
+      for (int j = 0; j < TJ; ++j) acc[i][j] = rest[i][j] = floatx16{};
+    struct Frags {
+      bf16x8 a[TI][3];
+    } g0, g1;
+    auto read = [&](Frags& g, int buf, int h) {
+      const char* base = smem + buf * BUF;
+#pragma unroll
+      for (int i = 0; i < TI; ++i)
+#pragma unroll
+        for (int s = 0; s < 3; ++s)
+          g.a[i][s] = *reinterpret_cast<const bf16x8*>(base + s * PLANE +
+                                                       split_slot<CH>(32 * i + l32, 2 * (ks * HS + h) + lk));
+    };
+    auto multiply = [&](Frags& g, Regs& r, int h) {
+      constexpr int pa[6] = {2, 0, 1, 0, 1, 0}, pb[6] = {0, 2, 1, 0, 0, 1};
+#pragma unroll
+      for (int p = 0; p < 6; ++p)
+#pragma unroll
+        for (int i = 0; i < TI; ++i)
+#pragma unroll
+          for (int j = 0; j < TJ; ++j) {
+            floatx16& sum = p == 3 ? acc[i][j] : rest[i][j];
+            sum = __builtin_amdgcn_mfma_f32_32x32x16_bf16(g.a[i][pa[p]], __builtin_bit_cast(bf16x8, r.b[j][h][pb[p]]), sum, 0,
+                                                          0, 0);
+          }
+    };
+    // The weights of tiles t + 1 .. t + D - 1 and the frames of tiles t + 2 .. t + D
+    // are in registers or on their way while tile t is multiplied (four tiles
+    // measured like two). Tiles past the end meet the weight planes' zeros.
+    auto step = [&](Regs& cur, Regs& next, int t, int buf) {
+      read(g0, buf, 0);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int h = 0; h < HS; ++h) {
+        Frags& g = h & 1 ? g1 : g0;
+        Frags& o = h & 1 ? g0 : g1;
+        if (h + 1 < HS) read(o, buf, h + 1);
+        __builtin_amdgcn_sched_barrier(0);
+        if (h == 0) stage(next, buf ^ 1);
+        if (h == HS - 1) fetch_a(next, t + 1 + D);
+        multiply(g, cur, h);
+        if (h == 0) {
+#pragma unroll
+          for (int i = 0; i < 6 * TI * TJ; ++i) {
+            __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
+            __builtin_amdgcn_sched_group_barrier(0x2, (44 * UA + 6 * TI * TJ - 1) / (6 * TI * TJ), 0);
+          }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      fetch_b(cur, t + D);
+      lds_barrier();
+    };
+#pragma unroll
+    for (int d = 0; d < D; ++d) {
+      fetch_a(r[d], d);
+      fetch_b(r[d], d);
+    }
+    stage(r[0], 0);
+    fetch_a(r[0], D);
+    if (tid == 0) unsure_s = 0;
+    lds_barrier();
+    for (int t = 0; t < steps; t += D) {
+#pragma unroll
+      for (int d = 0; d < D; ++d) step(r[d], r[(d + 1) % D], t + d, d & 1);
     }
 #pragma unroll
-    for (int u = 0; u < LB; ++u) {
-      const int n = n0 + lr + ROWS * u;
-      rb[u] = (n < N && k < K) ? *reinterpret_cast<const float4*>(w + (size_t)n * K + k) : make_float4(0.f, 0.f, 0.f, 0.f);
+    for (int i = 0; i < TI; ++i)
+#pragma unroll
+      for (int j = 0; j < TJ; ++j)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) acc[i][j][e] += rest[i][j][e];
+    if (KS > 1) {
+      // (The loop's last barrier is past every read of the staging buffers.)
+      float* part = reinterpret_cast<float*>(smem) + (size_t)wn * TI * TJ * 1024 + lane;
+      constexpr size_t kGroup = (size_t)WN * TI * TJ * 1024;
+      if (ks > 0) {
+#pragma unroll
+        for (int i = 0; i < TI; ++i)
+#pragma unroll
+          for (int j = 0; j < TJ; ++j)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) part[(ks - 1) * kGroup + (i * TJ + j) * 1024 + r * 64] = acc[i][j][r];
+      }
+      lds_barrier();
+      if (ks == 0) {
+#pragma unroll
+        for (int g = 0; g < KS - 1; ++g)
+#pragma unroll
+          for (int i = 0; i < TI; ++i)
+#pragma unroll
+            for (int j = 0; j < TJ; ++j)
+#pragma unroll
+              for (int r = 0; r < 16; ++r) acc[i][j][r] += part[g * kGroup + (i * TJ + j) * 1024 + r * 64];
+      }
     }
-  };
-  auto stage = [&](int buf) {
+    // Magnitudes less one (zero wraps): the largest and the smallest.
+    uint32_t most = 0u, least = 0xffffffffu;
+    if (ks == 0) {
 #pragma unroll
-    for (int u = 0; u < LA; ++u) *reinterpret_cast<float4*>(&a_s[buf][(lr + ROWS * u) * ROW + lc]) = ra[u];
+      for (int i = 0; i < TI; ++i)
 #pragma unroll
-    for (int u = 0; u < LB; ++u) *reinterpret_cast<float4*>(&b_s[buf][(lr + ROWS * u) * ROW + lc]) = rb[u];
-  };
-  fetch(0);
-  stage(0);
-  __syncthreads();
-  int buf = 0;
-  for (int k0 = 0; k0 < K; k0 += kGK) {
-    const bool more = k0 + kGK < K;
-    if (more) fetch(k0 + kGK);
+        for (int j = 0; j < TJ; ++j)
 #pragma unroll
-    for (int h = 0; h < KQ / 4; ++h) {
-      float4 av[BI], bv[BJ];
-#pragma unroll
-      for (int i = 0; i < BI; ++i)
-        av[i] = *reinterpret_cast<const float4*>(&a_s[buf][(wm + 16 * i + li) * ROW + KQ * lq + 4 * h]);
-#pragma unroll
-      for (int j = 0; j < BJ; ++j)
-        bv[j] = *reinterpret_cast<const float4*>(&b_s[buf][(wn + 16 * j + li) * ROW + KQ * lq + 4 * h]);
-#pragma unroll
-      for (int e = 0; e < 4; ++e)
-#pragma unroll
-        for (int i = 0; i < BI; ++i)
-#pragma unroll
-          for (int j = 0; j < BJ; ++j) {
-            const float a = e == 0 ? av[i].x : e == 1 ? av[i].y : e == 2 ? av[i].z : av[i].w;
-            const float b = e == 0 ? bv[j].x : e == 1 ? bv[j].y : e == 2 ? bv[j].z : bv[j].w;
-            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, acc[i][j], 0, 0, 0);
+          for (int e = 0; e < 16; ++e) {
+            const uint32_t m = (f2u(acc[i][j][e]) & 0x7fffffffu) - 1u;
+            most = max(most, m);
+            least = min(least, m);
           }
     }
-    if (more) {
-      stage(buf ^ 1);
-      __syncthreads();
-      buf ^= 1;
-    }
-  }
+    if (most >= 0x7f7fffffu || least < kSplitLow - 1u) unsure_s = 1;
+    lds_barrier();
+    if (unsure_s) {
+      bool odd = least < kSplitLow - 1u;
+      if (ks == 0) {
 #pragma unroll
-  for (int j = 0; j < BJ; ++j) {
-    const int n = n0 + wn + 16 * j + li;
-    if (n >= N) continue;
-    const float b = bias ? bias[n] : 0.0f;
+        for (int i = 0; i < TI; ++i)
 #pragma unroll
-    for (int i = 0; i < BI; ++i)
+          for (int j = 0; j < TJ; ++j)
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int f = f0 + wm + 16 * i + 4 * lq + r;
-        if (f < M) {
-          float v = acc[i][j][r] + b;
-          if (RELU) v = v < 0.0f ? 0.0f : v;  // (-0 and NaN pass, as the reference's `v < 0 ? 0 : v`)
-          out[(size_t)f * N + n] = v;
-        }
+            for (int e = 0; e < 16; ++e) odd = odd || (f2u(acc[i][j][e]) & 0x7fffffffu) >= 0x7f800000u;
       }
-  }
-}
-
-// The same product for grids of at most one workgroup per CU: each of the
-// four waves covers the whole 32 x 64 tile (2 x 4 blocks, eight
-// accumulators in flight) over its quarter of every K tile (lane group q of
-// wave w takes k = 16 w + 4 q .. + 3), and the four partial tiles are added
-// in wave order in LDS at the end.
-template <bool RELU>
-__global__ __launch_bounds__(256) void f32_gemm_wavek_kernel(const float* __restrict__ x, const float* __restrict__ w,
-                                                             const float* __restrict__ bias, float* __restrict__ out,
-                                                             int M, int N, int K) {
-  constexpr int GK = 64, TM = 32, TN = 64, ROW = GK + 4;
-  constexpr int PER_ROW = GK / 4, ROWS = 256 / PER_ROW, LA = TM / ROWS, LB = TN / ROWS;
-  __shared__ __attribute__((aligned(16))) float a_s[2][TM * ROW];
-  __shared__ __attribute__((aligned(16))) float b_s[2][TN * ROW];
-  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-  const int f0 = blockIdx.y * TM, n0 = blockIdx.x * TN;
-  const int li = lane & 15, lq = lane >> 4;
-  floatx4 acc[2][4];
-#pragma unroll
-  for (int i = 0; i < 2; ++i)
-#pragma unroll
-    for (int j = 0; j < 4; ++j) acc[i][j] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
-  const int lr = tid / PER_ROW, lc = 4 * (tid % PER_ROW);
-  float4 ra[LA], rb[LB];
-  auto fetch = [&](int k0) {
-    const int k = k0 + lc;
-#pragma unroll
-    for (int u = 0; u < LA; ++u) {
-      const int f = f0 + lr + ROWS * u;
-      ra[u] = (f < M && k < K) ? *reinterpret_cast<const float4*>(x + (size_t)f * K + k) : make_float4(0.f, 0.f, 0.f, 0.f);
+      // Sums of zero are right unless frames held values too small for the planes.
+      for (int row = wave; row < TM && f0 + row < M; row += WAVES)
+        for (int k = lane; k < K; k += 64)
+          odd = odd || (f2u(x[(size_t)(f0 + row) * K + k]) & 0x7fffffffu) - 1u < kSplitTiny - 1u;
+      if (__syncthreads_or(odd)) return false;
     }
+    if (ks == 0) {
 #pragma unroll
-    for (int u = 0; u < LB; ++u) {
-      const int n = n0 + lr + ROWS * u;
-      rb[u] = (n < N && k < K) ? *reinterpret_cast<const float4*>(w + (size_t)n * K + k) : make_float4(0.f, 0.f, 0.f, 0.f);
-    }
-  };
-  auto stage = [&](int buf) {
+      for (int j = 0; j < TJ; ++j) {
+        const int n = n0 + 32 * (TJ * wn + j) + l32;
+        if (n >= N) continue;
+        const float b = bias ? bias[n] : 0.0f;
+        float* o = out + (size_t)(f0 + 4 * lk) * N + n;
+        const bool whole = f0 + TM <= M;
 #pragma unroll
-    for (int u = 0; u < LA; ++u) *reinterpret_cast<float4*>(&a_s[buf][(lr + ROWS * u) * ROW + lc]) = ra[u];
+        for (int i = 0; i < TI; ++i)
 #pragma unroll
-    for (int u = 0; u < LB; ++u) *reinterpret_cast<float4*>(&b_s[buf][(lr + ROWS * u) * ROW + lc]) = rb[u];
-  };
-  fetch(0);
-  stage(0);
-  __syncthreads();
-  int buf = 0;
-  const int kl = 16 * wave + 4 * lq;
-  for (int k0 = 0; k0 < K; k0 += GK) {
-    const bool more = k0 + GK < K;
-    if (more) fetch(k0 + GK);
-    float4 av[2], bv[4];
-#pragma unroll
-    for (int i = 0; i < 2; ++i) av[i] = *reinterpret_cast<const float4*>(&a_s[buf][(16 * i + li) * ROW + kl]);
-#pragma unroll
-    for (int j = 0; j < 4; ++j) bv[j] = *reinterpret_cast<const float4*>(&b_s[buf][(16 * j + li) * ROW + kl]);
-#pragma unroll
-    for (int e = 0; e < 4; ++e)
-#pragma unroll
-      for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const float a = e == 0 ? av[i].x : e == 1 ? av[i].y : e == 2 ? av[i].z : av[i].w;
-          const float b = e == 0 ? bv[j].x : e == 1 ? bv[j].y : e == 2 ? bv[j].z : bv[j].w;
-          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, acc[i][j], 0, 0, 0);
-        }
-    if (more) {
-      stage(buf ^ 1);
-      __syncthreads();
-      buf ^= 1;
-    }
-  }
-  // Partial tiles into LDS (the staging buffers, free once every wave is
-  // past its last reads): part[w][f][n], then summed in wave order.
-  __syncthreads();
-  float* part = &a_s[0][0];
-  static_assert(4 * TM * TN <= 2 * TM * ROW + 2 * TN * ROW, "partials fit the staging buffers");
-  float* part_b = &b_s[0][0];
-  auto slot = [&](int wv, int f, int n) -> float& {
-    const int e = (wv * TM + f) * TN + n;
-    return e < 2 * TM * ROW ? part[e] : part_b[e - 2 * TM * ROW];
-  };
-#pragma unroll
-  for (int i = 0; i < 2; ++i)
-#pragma unroll
-    for (int j = 0; j < 4; ++j)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) slot(wave, 16 * i + 4 * lq + r, 16 * j + li) = acc[i][j][r];
-  __syncthreads();
-  for (int e = tid; e < TM * TN; e += 256) {
-    const int f = e / TN, n = e % TN;
-    if (f0 + f >= M || n0 + n >= N) continue;
-    float v = ((slot(0, f, n) + slot(1, f, n)) + slot(2, f, n)) + slot(3, f, n);
-    v = v + (bias ? bias[n0 + n] : 0.0f);
-    if (RELU) v = v < 0.0f ? 0.0f : v;
-    out[(size_t)(f0 + f) * N + n0 + n] = v;
-  }
-}
-
-// Any K and alignment: 64 x 64 tiles, K in steps of 32 staged in LDS one
-// float per thread and row, four waves of 2 x 2 v_mfma_f32_16x16x4f32 blocks.
-constexpr int kGT = 64, kGA = 32, kGPad = kGA + 1;
-
-template <bool RELU>
-__global__ __launch_bounds__(256) void f32_gemm_any_kernel(const float* __restrict__ x, const float* __restrict__ w,
-                                                           const float* __restrict__ bias, float* __restrict__ out,
-                                                           int M, int N, int K) {
-  __shared__ float a_s[kGT][kGPad];  // frames x k
-  __shared__ float b_s[kGT][kGPad];  // rows x k
-  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-  const int f0 = blockIdx.y * kGT, n0 = blockIdx.x * kGT;
-  const int fm = (wave >> 1) * 32, rn = (wave & 1) * 32;
-  floatx4 acc[2][2];
-#pragma unroll
-  for (int i = 0; i < 2; ++i)
-#pragma unroll
-    for (int j = 0; j < 2; ++j) acc[i][j] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
-  // Staging: thread t loads rows t / 32 + 8 s (s < 8), column t % 32.
-  const int lr = tid >> 5, lc = tid & 31;
-  for (int k0 = 0; k0 < K; k0 += kGA) {
-    const int k = k0 + lc;
-#pragma unroll
-    for (int s = 0; s < 8; ++s) {
-      const int r = lr + 8 * s;
-      const int f = f0 + r, n = n0 + r;
-      a_s[r][lc] = (f < M && k < K) ? x[(size_t)f * K + k] : 0.0f;
-      b_s[r][lc] = (n < N && k < K) ? w[(size_t)n * K + k] : 0.0f;
-    }
-    __syncthreads();
-#pragma unroll
-    for (int ks = 0; ks < kGA; ks += 4) {
-      const int kk = ks + (lane >> 4), ii = lane & 15;
-      const float a0 = a_s[fm + ii][kk], a1 = a_s[fm + 16 + ii][kk];
-      const float b0 = b_s[rn + ii][kk], b1 = b_s[rn + 16 + ii][kk];
-      acc[0][0] = __builtin_amdgcn_mfma_f32_16x16x4f32(a0, b0, acc[0][0], 0, 0, 0);
-      acc[0][1] = __builtin_amdgcn_mfma_f32_16x16x4f32(a0, b1, acc[0][1], 0, 0, 0);
-      acc[1][0] = __builtin_amdgcn_mfma_f32_16x16x4f32(a1, b0, acc[1][0], 0, 0, 0);
-      acc[1][1] = __builtin_amdgcn_mfma_f32_16x16x4f32(a1, b1, acc[1][1], 0, 0, 0);
-    }
-    __syncthreads();
-  }
-#pragma unroll
-  for (int i = 0; i < 2; ++i)
-#pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      const int n = n0 + rn + 16 * j + (lane & 15);
-      if (n >= N) continue;
-      const float b = bias ? bias[n] : 0.0f;
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int f = f0 + fm + 16 * i + 4 * (lane >> 4) + r;
-        if (f < M) {
-          float v = acc[i][j][r] + b;
-          if (RELU) v = v < 0.0f ? 0.0f : v;
-          out[(size_t)f * N + n] = v;
-        }
+          for (int r = 0; r < 16; ++r) {
+            const int row = 32 * i + 8 * (r >> 2) + (r & 3);
+            float v = acc[i][j][r] + b;
+            if (relu) v = v < 0.0f ? 0.0f : v;  // (-0 and NaN pass, as the reference's `v < 0 ? 0 : v`)
+            if (whole || f0 + 4 * lk + row < M) __builtin_nontemporal_store(v, o + (size_t)row * N);
+          }
       }
     }
+    return true;
+  };
+  if (!splittable || !split_tile()) tile_f32<TM, TN, WAVES>(smem, x, w, bias, out, M, N, K, f0, n0, relu);
 }
 
 // ---- GEMV (few frames, weight-bandwidth bound) ------------------------------
@@ -608,8 +754,31 @@ bool f32_attention_supported(int frames, int width, int heads) {
          width / heads <= kAMaxS;
 }
 
+// An FP32 weight on the device: its values, the range check's word (padded to
+// 16 bytes), its planes.
+static size_t planes_offset(int64_t rows, int cols) { return (((size_t)rows * cols * 4 + 15) & ~(size_t)15) + 16; }
+
+size_t f32_weight_bytes(int64_t rows, int cols) {
+  return planes_offset(rows, cols) + (size_t)split_pieces(rows, cols) * 16;
+}
+
+const int* f32_weight_outside(const float* w, int64_t rows, int cols) {
+  return reinterpret_cast<const int*>(reinterpret_cast<const char*>(w) + planes_offset(rows, cols) - 16);
+}
+
+hipError_t launch_f32_split(float* w, int64_t rows, int cols, hipStream_t s) {
+  int* outside = const_cast<int*>(f32_weight_outside(w, rows, cols));
+  const hipError_t e = hipMemsetAsync(outside, 0, 16, s);
+  if (e != hipSuccess) return e;
+  f32_split_range_kernel<<<(int)std::min<int64_t>((rows + 3) / 4, 2048), 256, 0, s>>>(w, rows, cols, outside);
+  const int64_t lanes = split_pieces(rows, cols) / 3;
+  f32_split_planes_kernel<<<(int)std::min<int64_t>((lanes + 255) / 256, 4096), 256, 0, s>>>(
+      w, rows, cols, reinterpret_cast<uint4*>(reinterpret_cast<char*>(w) + planes_offset(rows, cols)));
+  return hipGetLastError();
+}
+
 hipError_t launch_f32_linear(const float* x, const float* w, const float* bias, float* out, int M, int N, int K,
-                             bool relu, hipStream_t s) {
+                             bool relu, bool splittable, hipStream_t s) {
   if (M < 1 || N < 1 || K < 1) return hipErrorInvalidValue;
   if (M <= kVMaxFrames && K <= kVMaxK) {
     // Four rows per wave when that still leaves 512+ workgroups, else one.
@@ -628,32 +797,30 @@ hipError_t launch_f32_linear(const float* x, const float* w, const float* bias, 
 #undef FAH_GEMV
     return hipGetLastError();
   }
-  const bool aligned = K % 4 == 0 && reinterpret_cast<uintptr_t>(x) % 16 == 0 && reinterpret_cast<uintptr_t>(w) % 16 == 0;
-  if (!aligned) {
-    const dim3 grid((N + kGT - 1) / kGT, (M + kGT - 1) / kGT);
-    if (relu) f32_gemm_any_kernel<true><<<grid, 256, 0, s>>>(x, w, bias, out, M, N, K);
-    else f32_gemm_any_kernel<false><<<grid, 256, 0, s>>>(x, w, bias, out, M, N, K);
-    return hipGetLastError();
-  }
-  // The tile whose grid loads the CUs most evenly: rounds of 256
-  // workgroups times the tile's area, the larger tile on a tie; a grid of at
-  // most one 32 x 64 workgroup per CU splits K over its waves.
-  const int big = ((M + 63) / 64) * ((N + 63) / 64), small = ((M + 31) / 32) * ((N + 63) / 64);
-  const int64_t big_cost = (int64_t)((big + 255) / 256) * 2, small_cost = (small + 255) / 256;
-  if (big_cost <= small_cost) {
-    const dim3 grid((N + 63) / 64, (M + 63) / 64);
-    if (relu) f32_gemm_kernel<2, 2, true><<<grid, 256, 0, s>>>(x, w, bias, out, M, N, K);
-    else f32_gemm_kernel<2, 2, false><<<grid, 256, 0, s>>>(x, w, bias, out, M, N, K);
-  } else {
-    const dim3 grid((N + 63) / 64, (M + 31) / 32);
-    if (small <= 256 && K >= 256) {
-      if (relu) f32_gemm_wavek_kernel<true><<<grid, 256, 0, s>>>(x, w, bias, out, M, N, K);
-      else f32_gemm_wavek_kernel<false><<<grid, 256, 0, s>>>(x, w, bias, out, M, N, K);
-    } else {
-      if (relu) f32_gemm_kernel<1, 2, true><<<grid, 256, 0, s>>>(x, w, bias, out, M, N, K);
-      else f32_gemm_kernel<1, 2, false><<<grid, 256, 0, s>>>(x, w, bias, out, M, N, K);
-    }
-  }
+  const bool vec = K % 4 == 0 && reinterpret_cast<uintptr_t>(x) % 16 == 0;
+  const uint4* planes = reinterpret_cast<const uint4*>(reinterpret_cast<const char*>(w) + planes_offset(N, K));
+  const auto tiles = [&](int tm, int tn) { return ((M + tm - 1) / tm) * ((N + tn - 1) / tn); };
+  const auto run = [&](auto aligned, auto unaligned, int grid, int threads) {
+    if (vec) aligned<<<grid, threads, 0, s>>>(x, w, planes, bias, out, M, N, K, relu, splittable);
+    else unaligned<<<grid, threads, 0, s>>>(x, w, planes, bias, out, M, N, K, relu, splittable);
+  };
+#define FAH_SPLIT(WN, KS, TI, TJ, KB, D)                                                                     \
+  run(f32_split_gemm_kernel<WN, KS, TI, TJ, KB, D, true>, f32_split_gemm_kernel<WN, KS, TI, TJ, KB, D, false>, \
+      tiles(32 * TI, 32 * TJ * WN), 64 * WN * KS)
+  // The largest tile that still loads the chip: 64 x 128 from 224 workgroups
+  // on (with eight waves where they all run at once, four where several
+  // workgroups of a CU follow each other), 32 x 64 from 128 on, else 32 x 32
+  // with K split over four waves. Measured, us (8 waves, 4 waves, 32 x 64,
+  // 32 x 32): 1000 x 512 -> 2048 19.2 19.7 23.7 25.0; 4000 x 2048 -> 512 52.7
+  // 57.5 63.4 82.4; 4000 x 512 -> 2048 68.9 55.9 74.6 91.7; 1000 x 512 -> 1536
+  // 17.2 17.5 16.3 20.5; 333 x 560 -> 1536 18.8 18.0 12.1 12.9; 300 x 1023 ->
+  // 700 40.5 38.9 21.3 19.0; 20 x 512 -> 1024 14.4 14.2 8.2 7.1.
+  const int wide = tiles(64, 128);
+  if (wide > 256) FAH_SPLIT(4, 1, 2, 1, 1, 2);
+  else if (wide >= 224) FAH_SPLIT(4, 2, 2, 1, 2, 2);
+  else if (tiles(32, 64) >= 128) FAH_SPLIT(2, 2, 1, 1, 2, 2);
+  else FAH_SPLIT(1, 4, 1, 1, 2, 2);
+#undef FAH_SPLIT
   return hipGetLastError();
 }
 

@@ -250,10 +250,18 @@ hipError_t launch_session_embed(const int8_t* q, const void* scales, bool half_s
                                 const SessionRef* sessions, int count, float* x, hipStream_t s);
 
 
-// FP32 projections y[M][N] = x[M][K] W[N][K]^T (+ bias) (ReLU): fp32 MFMA
-// GEMM, or a GEMV for up to 4 frames of at most 4096 columns.
+// FP32 weights [N][K] as the projections take them: an allocation of
+// f32_weight_bytes that holds the values first; launch_f32_split then fills in
+// their bf16 planes and the word that f32_weight_outside points to (on the
+// device; not 0: the weight is not to be split).
+size_t f32_weight_bytes(int64_t rows, int cols);
+const int* f32_weight_outside(const float* w, int64_t rows, int cols);
+hipError_t launch_f32_split(float* w, int64_t rows, int cols, hipStream_t s);
+// FP32 projections y[M][N] = x[M][K] W[N][K]^T (+ bias) (ReLU): products of
+// bf16 planes on MFMA (fp32 MFMA for a weight that is not splittable), or a
+// GEMV for up to 4 frames of at most 4096 columns.
 hipError_t launch_f32_linear(const float* x, const float* w, const float* bias, float* out, int M, int N, int K,
-                             bool relu, hipStream_t s);
+                             bool relu, bool splittable, hipStream_t s);
 // Non-causal multi-head attention over [frames][width] rows (head size
 // width / heads <= 256, frames <= 4096).
 bool f32_attention_supported(int frames, int width, int heads);

@@ -141,7 +141,8 @@ int fah_weight_q8_upload_blocks(fah_context* context, const uint8_t* blocks, int
  * of fah_linear_many; the Q8_0 entry points decline it. */
 int fah_weight_f32_upload(fah_context* context, const float* values, int rows, int cols, fah_weight** out);
 int fah_weight_release(fah_weight* weight);
-/* Device bytes held by the weight (int8 plane plus scale plane). */
+/* Device bytes held by the weight (int8 plane plus scale plane; an FP32
+ * weight's values and their bf16 planes). */
 int64_t fah_weight_device_bytes(const fah_weight* weight);
 
 /* Projections (host buffers) ------------------------------------------------ */
@@ -173,7 +174,8 @@ int fah_quantized_linear_noalloc(fah_context* context, const float* input, int f
 /* IFloatComputeBackend.TryLinear (src/FunAsrNet/IFloatComputeBackend.cs:11-18;
  * reference device version src/FunAsrNet.Vulkan/VulkanFloatBackend.cs:127-171):
  * output[frames*rows] = input[frames*cols] W^T (+ bias) for an FP32 weight,
- * on fp32 MFMA (or a bandwidth-bound GEMV for up to 4 frames). Declines
+ * on the matrix cores with fp32 sums (each value split exactly into three bf16
+ * planes), or a bandwidth-bound GEMV for up to 4 frames. Declines
  * (output untouched) Q8_0 weights and projections below the minimum
  * operations. Float order differs from the CPU kernels, as the reference's
  * own device path does (its check: 2e-4 x max(1, |expected|)). The encoder's

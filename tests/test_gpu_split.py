@@ -1,0 +1,79 @@
+"""FP32 projections as products of bf16 planes: every tile shape and its edges
+against float64 sums, and what the planes cannot hold against fp32 rules.
+
+The bound is that of any fp32 sum of K products: (K + 2) roundings of 2^-24
+relative to sum |x w| (the planes themselves lose 2^-25 of a product)."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def backend():
+    from funasrnet_amd.hip import HipBackend
+    b = HipBackend(0, minimum_operations=0)
+    yield b
+    b.close()
+
+
+def run(backend, x, w, b=None):
+    out = np.full((x.shape[0], w.shape[0]), np.nan, np.float32)
+    assert backend.try_linear(x, x.shape[0], w, b, out.reshape(-1))
+    return out
+
+
+def check(got, x, w, b=None):
+    x, w = x.astype(np.float64), w.astype(np.float64)
+    bias = 0.0 if b is None else b.astype(np.float64)
+    bound = (x.shape[1] + 2) * 2.0**-24 * (np.abs(x) @ np.abs(w).T + np.abs(bias)) + 2.0**-149
+    assert np.all(np.abs(got - (x @ w.T + bias)) <= bound)
+
+
+# 32 x 32 tiles, 32 x 64 from 128 of them on, 64 x 128 from 224 (eight waves) and 257 (four) on.
+@pytest.mark.parametrize("frames,cols,rows", [(5, 4, 1), (31, 33, 31), (33, 128, 33), (64, 132, 65), (511, 60, 500),
+                                              (513, 96, 511), (1023, 36, 1793), (1025, 260, 2049), (2100, 31, 1100)])
+@pytest.mark.parametrize("biased", [False, True])
+def test_split_tiles(backend, frames, cols, rows, biased):
+    rng = np.random.default_rng(frames)
+    x = rng.standard_normal((frames, cols)).astype(np.float32)
+    w = rng.standard_normal((rows, cols)).astype(np.float32)
+    b = rng.standard_normal(rows).astype(np.float32) if biased else None
+    check(run(backend, x, w, b), x, w, b)
+
+
+@pytest.mark.parametrize("frames,rows", [(40, 70), (400, 700), (1100, 2100)])
+def test_split_range(backend, frames, rows):
+    """Zero frames, tiny and huge values, infinities and NaN."""
+    rng = np.random.default_rng(rows)
+    x = rng.standard_normal((frames, 64)).astype(np.float32)
+    w = rng.standard_normal((rows, 64)).astype(np.float32)
+    x[3] = 0.0
+    check(run(backend, x, w), x, w)
+    for scale in (2.0**-60, 2.0**-110, 2.0**-120, 2.0**100):
+        scaled = x.copy()
+        scaled[7] *= np.float32(scale)
+        check(run(backend, scaled, w), scaled, w)
+    x[5, 2], x[6, 1], x[9, 0] = np.inf, np.nan, np.float32(3.4e38)
+    w = w.copy()
+    w[:, 0] = np.abs(w[:, 0]) * np.float32(0.1)
+    got = run(backend, x, w)
+    sound = np.ones(frames, bool)
+    sound[[5, 6]] = False
+    check(got[sound], x[sound], w)
+    assert np.all(np.isnan(got[6])) and np.array_equal(got[5], np.where(w[:, 2] < 0, -np.inf, np.inf).astype(np.float32))
+
+
+@pytest.mark.parametrize("value", [2.0**21, 2.0**-90, np.inf])
+def test_weights_outside_the_planes(backend, value):
+    rng = np.random.default_rng(1)
+    x = rng.standard_normal((200, 100)).astype(np.float32)
+    w = rng.standard_normal((130, 100)).astype(np.float32)
+    w[4] = np.float32(value) * (np.sign(w[4]) if np.isfinite(value) else 1)
+    got = run(backend, x, w)
+    if np.isfinite(value):
+        check(got, x, w)
+    else:
+        keep = np.arange(130) != 4
+        check(got[:, keep], x, w[keep])
+        assert not np.any(np.isfinite(got[:, 4]))
