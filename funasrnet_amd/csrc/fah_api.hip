@@ -198,6 +198,10 @@ struct Ctx {
   bool disposed = false;
   int64_t minimum_operations = 250000;
   DeviceBuffer in, out, q, s;
+  // Planes and partial sums of an attention call (stream-ordered: one call's
+  // kernels run before the next one's), and the calls that used them.
+  DeviceBuffer attention;
+  unsigned attention_epoch = 0;
   std::string name;
   std::unique_ptr<SessionBatch> batch;  // last lock-step batch (its sessions alive)
   // Seam-call statistics (fah_context_statistics) and the call observer;
@@ -244,6 +248,7 @@ Ctx::~Ctx() {
   out.release();
   q.release();
   s.release();
+  attention.release();
   if (mark) (void)hipEventDestroy(mark);
   if (t0) (void)hipEventDestroy(t0);
   if (t1) (void)hipEventDestroy(t1);
@@ -308,6 +313,31 @@ struct CallMeter {
     if (observer) observer(user, kind, frames, cols, rows, device_ms, total_ms);
   }
 };
+
+// The attention workspace for these buffers, or nullptr where the kernel
+// without one runs: shapes that have none, a stream under capture (a graph
+// would keep the address of a buffer that a later, larger call replaces) and
+// no memory left.
+void* attention_workspace(Ctx* c, const float* q, const float* k, const float* out, int frames, int width, int heads) {
+  const size_t bytes = fah::f32_attention_workspace(q, k, out, frames, width, heads);
+  if (!bytes) return nullptr;
+  hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(c->stream, &capture) != hipSuccess || capture != hipStreamCaptureStatusNone) return nullptr;
+  if (bytes > c->attention.bytes) {
+    check(hipStreamSynchronize(c->stream), "hipStreamSynchronize");  // earlier calls still read the old one
+    c->attention.release();
+    if (hipMalloc(&c->attention.ptr, bytes) != hipSuccess) {
+      (void)hipGetLastError();
+      c->attention.ptr = nullptr;
+      return nullptr;
+    }
+    c->attention.bytes = bytes;
+    check(hipMemsetAsync(c->attention.ptr, 0, 4096, c->stream), "hipMemsetAsync");
+    c->attention_epoch = 0;
+  }
+  if (++c->attention_epoch == 0) ++c->attention_epoch;
+  return c->attention.ptr;
+}
 
 int declined(Ctx* c, int kind) {
   std::lock_guard<std::mutex> lock(c->stats_m);
@@ -1948,8 +1978,11 @@ int fah_attention(fah_context* h, const float* query, const float* key, const fl
     check(hipMemcpyAsync(dq, query, bytes, hipMemcpyHostToDevice, c->stream), "H2D query");
     check(hipMemcpyAsync(dk, key, bytes, hipMemcpyHostToDevice, c->stream), "H2D key");
     check(hipMemcpyAsync(dv, value, bytes, hipMemcpyHostToDevice, c->stream), "H2D value");
+    void* workspace = attention_workspace(c, dq, dk, c->out.as<float>(), frames, width, heads);
     meter.kernels_begin();
-    check(fah::launch_f32_attention(dq, dk, dv, c->out.as<float>(), frames, width, heads, c->stream), "attention");
+    check(fah::launch_f32_attention(dq, dk, dv, c->out.as<float>(), frames, width, heads, workspace, c->attention_epoch,
+                                    c->stream),
+          "attention");
     meter.kernels_end();
     check(hipMemcpyAsync(output, c->out.ptr, bytes, hipMemcpyDeviceToHost, c->stream), "D2H output");
     work.release();  // enqueued: other contexts may enqueue while this stream drains
@@ -1970,7 +2003,10 @@ int fah_attention_device(fah_context* h, const float* query, const float* key, c
     if (c->disposed) return fail(FAH_ERROR_DISPOSED, "context disposed");
     check(hipSetDevice(c->device), "hipSetDevice");
     DeviceWork work(*c);
-    check(fah::launch_f32_attention(query, key, value, output, frames, width, heads, c->stream), "attention");
+    void* workspace = attention_workspace(c, query, key, output, frames, width, heads);
+    check(fah::launch_f32_attention(query, key, value, output, frames, width, heads, workspace, c->attention_epoch,
+                                    c->stream),
+          "attention");
     return FAH_OK;
   });
 }

@@ -15,6 +15,7 @@
 #include "fah_internal.h"
 
 #include <algorithm>
+#include <cmath>
 #include <cstdint>
 
 namespace fah {
@@ -617,8 +618,8 @@ __global__ __launch_bounds__(256) void f32_attention_kernel(const float* __restr
   }
 }
 
-// ---- Non-causal multi-head attention on fp32 MFMA (head size HS, 64 or 128) ----
-// One workgroup per (head, 16 query rows); wave w takes key blocks (16 keys)
+// ---- Non-causal multi-head attention on fp32 MFMA (head size HS, a multiple of 16) ----
+// A workgroup's tile of 16 query rows of a head; wave w takes key blocks (16 keys)
 // w, w + 4, ... and keeps its own running maximum, sum and outputs; the four
 // partial results are merged in LDS at the end. Per key block the scores
 // come transposed, S^T = K Q^T (16 keys x 16 queries, HS / 4 MFMAs with key
@@ -626,16 +627,18 @@ __global__ __launch_bounds__(256) void f32_attention_kernel(const float* __restr
 // lane group g multiplies channel g HS/4 + t), so that lane (query j, group
 // g) holds the probabilities of keys 4g .. 4g + 3 for query j, which is
 // exactly the A operand of P V when substep u takes key 4g + u.
+constexpr int attention_tile_bytes(int HS) { return (64 * HS + 128) * 4; }
+
 template <int HS>
-__global__ __launch_bounds__(256) void f32_attention_mfma_kernel(const float* __restrict__ q,
-                                                                 const float* __restrict__ k,
-                                                                 const float* __restrict__ v, float* __restrict__ out,
-                                                                 int frames, int width, float divisor) {
+__device__ __forceinline__ void attention_tile_f32(char* smem, const float* __restrict__ q, const float* __restrict__ k,
+                                                   const float* __restrict__ v, float* __restrict__ out, int frames,
+                                                   int width, float divisor, int head, int t0) {
   constexpr int CB = HS / 16, KQ = HS / 4;  // channel blocks; channels per lane group
-  __shared__ __attribute__((aligned(16))) float o_s[4][16][HS];
-  __shared__ float m_s[4][16], l_s[4][16];
+  float(*o_s)[16][HS] = reinterpret_cast<float(*)[16][HS]>(smem);
+  float(*m_s)[16] = reinterpret_cast<float(*)[16]>(smem + 64 * HS * 4);
+  float(*l_s)[16] = m_s + 4;
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, j = lane & 15, g = lane >> 4;
-  const int head = blockIdx.x, t0 = blockIdx.y * 16, hoff = head * HS;
+  const int hoff = head * HS;
   // This lane's query channels g KQ .. g KQ + KQ - 1 of query t0 + j (zero past the end).
   float qv[KQ];
   {
@@ -747,6 +750,290 @@ __global__ __launch_bounds__(256) void f32_attention_mfma_kernel(const float* __
   }
 }
 
+template <int HS>
+__global__ __launch_bounds__(256) void f32_attention_mfma_kernel(const float* __restrict__ q,
+                                                                 const float* __restrict__ k,
+                                                                 const float* __restrict__ v, float* __restrict__ out,
+                                                                 int frames, int width, float divisor) {
+  __shared__ __attribute__((aligned(16))) char smem[attention_tile_bytes(HS)];
+  attention_tile_f32<HS>(smem, q, k, v, out, frames, width, divisor, blockIdx.x, blockIdx.y * 16);
+}
+
+// ---- Non-causal multi-head attention on the bf16 matrix cores (head size 64, 96, 128) ----
+// The products of f32_split_gemm_kernel: q, k, v and the probabilities as three
+// bf16 planes each, six products, fp32 sums.
+//
+// attention_planes_kernel lays the planes out once, in the order the lanes of
+// v_mfma_f32_32x32x16_bf16 hold them (fragments of [plane 3][lane 64] 16-byte
+// pieces): q and k per 32 rows and 16 channels (lane l: row l % 32, channels
+// 8 (l / 32) .. + 7), v per 16 keys and 32 channels (lane l: channel l % 32,
+// keys 8 (i / 4) + 4 (l / 32) + i % 4, i < 8). attention_split_kernel, a
+// workgroup per (head, 64 queries, share of the keys), runs two waves of 32
+// queries over the even key blocks of 32 and two over the odd ones. Scores come
+// transposed, S^T = K Q^T, so that lane l holds 16 of a block's scores of query
+// l % 32 and lane l ^ 32 the others: the softmax needs one exchange a block.
+// Exponentials of them are, as they lie, the B operand of O^T = V^T P^T in the
+// key order above, and the outputs of a lane are its query's. The running
+// maximum moves (and the sums are rescaled) only when a score exceeds it by
+// more than kSlack (in powers of two): exponentials up to 2^kSlack are as exact. The
+// waves' sums are merged in LDS, those of the key shares by
+// attention_merge_kernel.
+//
+// Bound by the MFMAs (16 key blocks a wave: 1.57 us a block of 3,072 MFMA
+// cycles) and, for short inputs, by launches and first loads. One wave a SIMD
+// (402 registers at 128: eight operand groups, 1 to 1.5 us of MFMAs, are on
+// their way; four measured 176 us where eight take 169). Measured against
+// attention_tile_f32 for all: 4096 frames of 4 x 128 569 -> 169 us, 1864 133 ->
+// 54, 1000 44 -> 32, 1100 of 8 x 96 984 -> 43 (it ran on the VALU); error against
+// 64 bits 7.2e-7 -> 4.1e-7 (4096), 5.0e-7 -> 1.8e-7 (1000).
+//
+// Values outside [2^-100, 2^60] in magnitude, but zero, set the head's word in
+// `outside` (so do infinities and NaN); its tiles run on fp32 MFMA.
+constexpr uint32_t kPlaneMost = 0x5d800000u;  // 2^60
+constexpr float kSlack = 8.0f;
+constexpr int kSplitQ = 64;  // queries a workgroup
+
+struct SplitAttnArgs {
+  const float *q, *k, *v;
+  float* out;
+  int frames, width, heads, shares;
+  float divisor, scale;         // sqrt(head size); log2(e) / divisor
+  uint4 *qp, *kp, *vp;          // planes [head][block 32][HS / 16][3][64]
+  float* part;                  // [share][head][frames padded to 64][HS] sums (shares > 1)
+  float2* part_ml;              // [share][head][frames padded to 64] maximum, denominator
+  unsigned* outside;            // [heads]: `epoch` where the head's values do not fit the planes
+  unsigned epoch;
+};
+
+template <int HS>
+__global__ __launch_bounds__(256) void attention_planes_kernel(SplitAttnArgs a) {
+  constexpr int C16 = HS / 16;
+  const int blocks = (a.frames + 63) / 64 * 2, per_head = blocks * C16 * 64, total = a.heads * per_head;
+  const int i = blockIdx.x * 256 + threadIdx.x;
+  if (i >= total) return;
+  const int which = blockIdx.y;  // 0 q, 1 k, 2 v
+  const int head = i / per_head, lane = i & 63, fragment = (i % per_head) >> 6;
+  const float* src = (which == 0 ? a.q : which == 1 ? a.k : a.v) + head * HS;
+  float v[8];
+  if (which < 2) {
+    const int row = fragment / C16 * 32 + (lane & 31), ch = fragment % C16 * 16 + 8 * (lane >> 5);
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const float4 x4 = row < a.frames ? *reinterpret_cast<const float4*>(src + (size_t)row * a.width + ch + 4 * h)
+                                       : make_float4(0.f, 0.f, 0.f, 0.f);
+      v[4 * h] = x4.x;
+      v[4 * h + 1] = x4.y;
+      v[4 * h + 2] = x4.z;
+      v[4 * h + 3] = x4.w;
+    }
+  } else {
+    // Fragments of a 32-key block: 16-key step (outer), 32-channel block.
+    const int step = fragment / (HS / 32), ch = fragment % (HS / 32) * 32 + (lane & 31);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const int key = 16 * step + 8 * (e >> 2) + 4 * (lane >> 5) + (e & 3);
+      v[e] = key < a.frames ? src[(size_t)key * a.width + ch] : 0.0f;
+    }
+  }
+  bool odd = false;
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    const uint32_t m = f2u(v[e]) & 0x7fffffffu;
+    odd = odd || m > kPlaneMost || m - 1u < kSplitTiny - 1u;
+  }
+  if (odd) a.outside[head] = a.epoch;
+  uint4 p[3];
+  split8(v, p);
+  uint4* dst = (which == 0 ? a.qp : which == 1 ? a.kp : a.vp) + ((size_t)head * (per_head >> 6) + fragment) * 192 + lane;
+#pragma unroll
+  for (int s = 0; s < 3; ++s) dst[64 * s] = p[s];
+}
+
+template <int HS>
+__global__ __launch_bounds__(256, 1) void attention_split_kernel(SplitAttnArgs a) {
+  constexpr int C16 = HS / 16, CB = HS / 32, G = 2 * C16, ROW = HS + 4;  // fragment groups a key block: C16 of k, C16 of v
+  constexpr int AHEAD = G / 2;
+  static_assert(G % AHEAD == 0, "a block's groups fill the ring a whole number of times");
+  extern __shared__ __attribute__((aligned(16))) char attn_split_s[];
+  float* o_s = reinterpret_cast<float*>(attn_split_s);  // [2][64][ROW]
+  float2* ml_s = reinterpret_cast<float2*>(o_s + 2 * kSplitQ * ROW);  // [2][64]
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, l32 = lane & 31, lk = lane >> 5;
+  const int wq = wave & 1, wk = wave >> 1;
+  // Workgroups are dealt to the XCDs in turn: each takes a run of tiles, the
+  // queries of one head and share together, whose k and v its L2 then holds.
+  const int tiles = gridDim.x, xcd = blockIdx.x & 7, q8 = tiles >> 3, r8 = tiles & 7, qtiles = (a.frames + 63) / 64;
+  const int tile = xcd * q8 + min(xcd, r8) + (blockIdx.x >> 3);
+  const int q0 = tile % qtiles * kSplitQ, share = tile / qtiles % a.shares, head = tile / qtiles / a.shares;
+  const unsigned outside = a.outside[head];
+  const int blocks64 = (a.frames + 63) / 64, blocks = (a.frames + 31) / 32;
+  const size_t head_pieces = (size_t)blocks64 * 2 * C16 * 192;
+  bf16x8 q[C16][3];
+  {
+    const uint4* src = a.qp + head * head_pieces + (size_t)(q0 / 32 + wq) * C16 * 192 + lane;
+#pragma unroll
+    for (int c = 0; c < C16; ++c)
+#pragma unroll
+      for (int s = 0; s < 3; ++s) q[c][s] = __builtin_bit_cast(bf16x8, src[c * 192 + 64 * s]);
+  }
+  const int first = blocks * share / a.shares + wk, last = blocks * (share + 1) / a.shares;
+  const uint4* kp = a.kp + head * head_pieces + lane;
+  const uint4* vp = a.vp + head * head_pieces + lane;
+  floatx16 o[CB], small[CB];  // sums of the large products and of the corrections
+#pragma unroll
+  for (int c = 0; c < CB; ++c) o[c] = small[c] = floatx16{};
+  float run_m = -__builtin_inff(), run_l = 0.0f;  // of this lane's query; the sum over this lane's keys
+  bf16x8 ring[AHEAD][3];
+  // Group g of block b: k's 16-channel steps, then v's (step, channel block) fragments.
+  auto load = [&](int b, int g) {
+    if (g >= G) {
+      g -= G;
+      b += 2;
+    }
+    b = min(b, blocks - 1);
+    const uint4* src = (g < C16 ? kp : vp) + ((size_t)b * C16 + (g < C16 ? g : g - C16)) * 192;
+#pragma unroll
+    for (int s = 0; s < 3; ++s) ring[g % AHEAD][s] = __builtin_bit_cast(bf16x8, src[64 * s]);
+  };
+  if (first < last) {
+#pragma unroll
+    for (int g = 0; g < AHEAD; ++g) load(first, g);
+  }
+  // (The operands are on their way meanwhile.)
+  if (outside == a.epoch) {
+    if (share == 0)
+      for (int t = 0; t < kSplitQ && q0 + t < a.frames; t += 16)
+      {
+        __syncthreads();
+        attention_tile_f32<HS>(attn_split_s, a.q, a.k, a.v, a.out, a.frames, a.width, a.divisor, head, q0 + t);
+      }
+    return;
+  }
+  constexpr int pa[6] = {2, 0, 1, 0, 1, 0}, pb[6] = {0, 2, 1, 0, 0, 1};
+  for (int b = first; b < last; b += 2) {
+    floatx16 sc = floatx16{}, rest = floatx16{};
+#pragma unroll
+    for (int g = 0; g < C16; ++g) {
+#pragma unroll
+      for (int p = 0; p < 6; ++p) {
+        floatx16& sum = p == 3 ? sc : rest;
+        sum = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ring[g % AHEAD][pa[p]], q[g][pb[p]], sum, 0, 0, 0);
+      }
+      load(b, g + AHEAD);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    float t[16], top = -__builtin_inff();
+#pragma unroll
+    for (int r = 0; r < 16; ++r) t[r] = sc[r] + rest[r];
+    if (b == blocks - 1) {
+#pragma unroll
+      for (int r = 0; r < 16; ++r)
+        if (b * 32 + 8 * (r >> 2) + 4 * lk + (r & 3) >= a.frames) t[r] = -__builtin_inff();
+    }
+#pragma unroll
+    for (int r = 0; r < 16; ++r) top = fmaxf(top, t[r]);
+    top = fmaxf(top, __shfl_xor(top, 32, 64)) * a.scale;
+    if (__any(top > run_m + kSlack)) {
+      const float m = fmaxf(run_m, top), down = __builtin_amdgcn_exp2f(run_m - m);
+      run_m = m;
+      run_l *= down;
+#pragma unroll
+      for (int c = 0; c < CB; ++c)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          o[c][r] *= down;
+          small[c][r] *= down;
+        }
+    }
+    bf16x8 pr[2][3];
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      float e[8];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        e[i] = __builtin_amdgcn_exp2f(__builtin_fmaf(t[8 * h + i], a.scale, -run_m));
+        run_l += e[i];
+      }
+      uint4 w[3];
+      split8(e, w);
+#pragma unroll
+      for (int s = 0; s < 3; ++s) pr[h][s] = __builtin_bit_cast(bf16x8, w[s]);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int g = C16; g < G; ++g) {
+      const int h = (g - C16) / CB, c = (g - C16) % CB;
+#pragma unroll
+      for (int p = 0; p < 6; ++p) {
+        floatx16& sum = p == 3 ? o[c] : small[c];
+        sum = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ring[g % AHEAD][pa[p]], pr[h][pb[p]], sum, 0, 0, 0);
+      }
+      load(b, g + AHEAD);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  }
+  run_l += __shfl_xor(run_l, 32, 64);
+  // Sums of both key halves to LDS: channel 32 c + 8 (r / 4) + 4 lk + r % 4 of query l32.
+  {
+    float* row = o_s + (size_t)(wk * kSplitQ + 32 * wq + l32) * ROW + 4 * lk;
+#pragma unroll
+    for (int c = 0; c < CB; ++c)
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        *reinterpret_cast<float4*>(row + 32 * c + 8 * r) =
+            make_float4(o[c][4 * r] + small[c][4 * r], o[c][4 * r + 1] + small[c][4 * r + 1],
+                        o[c][4 * r + 2] + small[c][4 * r + 2], o[c][4 * r + 3] + small[c][4 * r + 3]);
+    if (lk == 0) ml_s[wk * kSplitQ + 32 * wq + l32] = make_float2(run_m, run_l);
+  }
+  lds_barrier();
+  const int padded = blocks64 * 64;
+  for (int e = tid; e < kSplitQ * HS / 4; e += 256) {
+    const int row = e / (HS / 4), ch = e % (HS / 4) * 4, f = q0 + row;
+    const float2 x = ml_s[row], y = ml_s[kSplitQ + row];
+    const float m = fmaxf(x.x, y.x);
+    const float fx = x.x == -__builtin_inff() ? 0.0f : __builtin_amdgcn_exp2f(x.x - m);
+    const float fy = y.x == -__builtin_inff() ? 0.0f : __builtin_amdgcn_exp2f(y.x - m);
+    const float l = fx * x.y + fy * y.y;
+    const float4 u = *reinterpret_cast<const float4*>(o_s + (size_t)row * ROW + ch);
+    const float4 v = *reinterpret_cast<const float4*>(o_s + (size_t)(kSplitQ + row) * ROW + ch);
+    float4 s = make_float4(fx * u.x + fy * v.x, fx * u.y + fy * v.y, fx * u.z + fy * v.z, fx * u.w + fy * v.w);
+    if (a.shares == 1) {
+      if (f < a.frames) {
+        float* o4 = a.out + (size_t)f * a.width + head * HS + ch;
+        *reinterpret_cast<float4*>(o4) = make_float4(s.x / l, s.y / l, s.z / l, s.w / l);
+      }
+    } else {
+      const size_t at = ((size_t)share * a.heads + head) * padded + f;
+      *reinterpret_cast<float4*>(a.part + at * HS + ch) = s;
+      if (ch == 0) a.part_ml[at] = make_float2(m, l);
+    }
+  }
+}
+
+// out = sum of the shares' sums / sum of their denominators, each at the common maximum.
+template <int HS>
+__global__ __launch_bounds__(256) void attention_merge_kernel(SplitAttnArgs a) {
+  const int i = blockIdx.x * 256 + threadIdx.x, per = HS / 4;
+  const int ch = i % per * 4, head = i / per % a.heads, f = i / per / a.heads;
+  if (f >= a.frames || a.outside[head] == a.epoch) return;
+  const size_t stride = (size_t)a.heads * ((a.frames + 63) / 64 * 64), at = stride / a.heads * head + f;
+  float m = -__builtin_inff();
+  for (int s = 0; s < a.shares; ++s) m = fmaxf(m, a.part_ml[s * stride + at].x);
+  float4 sum = make_float4(0.f, 0.f, 0.f, 0.f);
+  float l = 0.0f;
+  for (int s = 0; s < a.shares; ++s) {
+    const float2 ml = a.part_ml[s * stride + at];
+    const float w = ml.x == -__builtin_inff() ? 0.0f : __builtin_amdgcn_exp2f(ml.x - m);
+    const float4 u = *reinterpret_cast<const float4*>(a.part + (s * stride + at) * HS + ch);
+    l += w * ml.y;
+    sum.x += w * u.x;
+    sum.y += w * u.y;
+    sum.z += w * u.z;
+    sum.w += w * u.w;
+  }
+  float* o = a.out + (size_t)f * a.width + head * HS + ch;
+  *reinterpret_cast<float4*>(o) = make_float4(sum.x / l, sum.y / l, sum.z / l, sum.w / l);
+}
+
 }  // namespace
 
 bool f32_attention_supported(int frames, int width, int heads) {
@@ -824,11 +1111,83 @@ hipError_t launch_f32_linear(const float* x, const float* w, const float* bias, 
   return hipGetLastError();
 }
 
+// Key shares of attention_split_kernel: as many as its workgroups (one a CU)
+// leave room for, with four key blocks of 32 or more each. Measured with 1, 2,
+// 3, 4 shares, us: 1000 frames of 4 heads of 128 (64 query tiles) 44 35 34 31;
+// 1864 of 4 (120) 71 54 63 55; 1068 of 8 of 64 (136) 31 35 31 36; 4096 of 4
+// (256) 169 177 181 185; 184 of 8 of 96 (24 tiles, 6 blocks) 12.9 14.8 14.6 15.4.
+static int attention_shares(int frames, int heads) {
+  const int tiles = (frames + 63) / 64 * heads, blocks = (frames + 31) / 32;
+  return std::max(1, std::min(std::min(4, 256 / tiles), blocks / 4));
+}
+
+struct AttnLayout {
+  size_t planes, part, part_ml, outside, bytes;
+};
+static AttnLayout attention_layout(int frames, int width, int heads) {
+  const size_t padded = (size_t)(frames + 63) / 64 * 64, shares = attention_shares(frames, heads);
+  AttnLayout l;
+  l.planes = 4096;  // the heads' words first: they outlive a call
+  l.part = l.planes + 3 * padded * width * 6;
+  l.part_ml = l.part + (shares > 1 ? shares * padded * width * 4 : 0);
+  l.bytes = l.part_ml + (shares > 1 ? shares * padded * heads * 8 : 0);
+  return l;
+}
+
+size_t f32_attention_workspace(const float* q, const float* k, const float* out, int frames, int width, int heads) {
+  const int S = width / heads;
+  const bool aligned = (reinterpret_cast<uintptr_t>(q) | reinterpret_cast<uintptr_t>(k) | reinterpret_cast<uintptr_t>(out)) % 16 == 0;
+  if (!aligned || heads > 1024 || (S != 64 && S != 96 && S != 128)) return 0;
+  // Shorter ones are quicker without the extra launches (us, fp32 MFMA and
+  // split: 250 frames of 4 x 128 14.5 16.2, 400 20.8 20.2, 576 25.6 23.1; 500
+  // of 8 x 64 15.7 17.2, 1068 55.6 31.4). 96 has no fp32 MFMA kernel (184
+  // frames of 8 x 96: 57 on the VALU, 13 here).
+  if ((S == 128 && frames < 400) || (S == 64 && frames < 640)) return 0;
+  return attention_layout(frames, width, heads).bytes;
+}
+
+template <int HS>
+static hipError_t launch_split_attention(const SplitAttnArgs& a, hipStream_t s) {
+  const int planes = a.heads * ((a.frames + 63) / 64 * 2) * (HS / 16) * 64, tiles = (a.frames + 63) / 64 * a.heads * a.shares;
+  constexpr int lds = std::max((2 * kSplitQ * (HS + 4) + 4 * kSplitQ) * 4, attention_tile_bytes(HS));
+  static const hipError_t raised = hipFuncSetAttribute(reinterpret_cast<const void*>(attention_split_kernel<HS>),
+                                                       hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+  if (raised != hipSuccess) return raised;
+  attention_planes_kernel<HS><<<dim3((planes + 255) / 256, 3), 256, 0, s>>>(a);
+  attention_split_kernel<HS><<<tiles, 256, lds, s>>>(a);
+  if (a.shares > 1) attention_merge_kernel<HS><<<(a.frames * a.heads * (HS / 4) + 255) / 256, 256, 0, s>>>(a);
+  return hipGetLastError();
+}
+
 hipError_t launch_f32_attention(const float* q, const float* k, const float* v, float* out, int frames, int width,
-                                int heads, hipStream_t s) {
+                                int heads, void* workspace, unsigned epoch, hipStream_t s) {
   if (!f32_attention_supported(frames, width, heads)) return hipErrorInvalidValue;
   const int S = width / heads;
   const float divisor = sqrtf((float)S);
+  if (workspace) {
+    const AttnLayout l = attention_layout(frames, width, heads);
+    char* base = static_cast<char*>(workspace);
+    SplitAttnArgs a{};
+    a.q = q;
+    a.k = k;
+    a.v = v;
+    a.out = out;
+    a.frames = frames;
+    a.width = width;
+    a.heads = heads;
+    a.shares = attention_shares(frames, heads);
+    a.divisor = divisor;
+    a.scale = (float)(1.4426950408889634 / std::sqrt((double)S));
+    const size_t plane = (size_t)(frames + 63) / 64 * 64 * width * 6;
+    a.qp = reinterpret_cast<uint4*>(base + l.planes);
+    a.kp = reinterpret_cast<uint4*>(base + l.planes + plane);
+    a.vp = reinterpret_cast<uint4*>(base + l.planes + 2 * plane);
+    a.part = reinterpret_cast<float*>(base + l.part);
+    a.part_ml = reinterpret_cast<float2*>(base + l.part_ml);
+    a.outside = reinterpret_cast<unsigned*>(base);
+    a.epoch = epoch;
+    return S == 128 ? launch_split_attention<128>(a, s) : S == 96 ? launch_split_attention<96>(a, s) : launch_split_attention<64>(a, s);
+  }
   const bool aligned = width % 4 == 0 && (reinterpret_cast<uintptr_t>(q) | reinterpret_cast<uintptr_t>(k)) % 16 == 0;
   if (aligned && (S == 64 || S == 128)) {
     const dim3 grid(heads, (frames + 15) / 16);

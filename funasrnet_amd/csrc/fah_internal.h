@@ -265,8 +265,12 @@ hipError_t launch_f32_linear(const float* x, const float* w, const float* bias, 
 // Non-causal multi-head attention over [frames][width] rows (head size
 // width / heads <= 256, frames <= 4096).
 bool f32_attention_supported(int frames, int width, int heads);
+// With a workspace (f32_attention_workspace bytes, 0 where there is none to
+// use; its first 4096 bytes zero when allocated and then left alone) and an
+// epoch that no earlier call on it had, the products run on bf16 MFMA.
+size_t f32_attention_workspace(const float* q, const float* k, const float* out, int frames, int width, int heads);
 hipError_t launch_f32_attention(const float* q, const float* k, const float* v, float* out, int frames, int width,
-                                int heads, hipStream_t s);
+                                int heads, void* workspace, unsigned epoch, hipStream_t s);
 
 bool persistent_shape_supported(int width, int heads, int kv_heads, int head_size, int ffn, int blocks);
 // long_cache: the step at a position from a.long_from on (the long-cache

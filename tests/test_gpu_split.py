@@ -1,7 +1,8 @@
-"""FP32 projections as products of bf16 planes: every tile shape and its edges
-against float64 sums, and what the planes cannot hold against fp32 rules.
+"""FP32 projections and attention as products of bf16 planes: every tile shape
+and its edges against float64 sums, and what the planes cannot hold against fp32
+rules.
 
-The bound is that of any fp32 sum of K products: (K + 2) roundings of 2^-24
+The bound of a projection is that of any fp32 sum of K products: (K + 2) roundings of 2^-24
 relative to sum |x w| (the planes themselves lose 2^-25 of a product)."""
 import numpy as np
 import pytest
@@ -77,3 +78,47 @@ def test_weights_outside_the_planes(backend, value):
         keep = np.arange(130) != 4
         check(got[:, keep], x, w[keep])
         assert not np.any(np.isfinite(got[:, 4]))
+
+
+def attend(backend, q, k, v, heads):
+    out = np.full(q.shape, np.nan, np.float32)
+    assert backend.try_attention(q, k, v, q.shape[0], q.shape[1], heads, out.reshape(-1))
+    return out
+
+
+# Tiles of 64 queries, blocks of 32 keys, one to four key shares; either side of
+# the lengths from which heads of 128 and 64 take the planes. The tolerance is the
+# reference's device check's (AttentionGpuChecks.cs), relative to values of 4.
+@pytest.mark.parametrize("frames,heads,size", [(1, 2, 96), (33, 1, 96), (63, 4, 96), (65, 8, 96), (399, 1, 128),
+                                               (400, 4, 128), (449, 1, 128), (513, 3, 128), (1857, 4, 128),
+                                               (640, 2, 64), (671, 8, 64), (1100, 8, 64)])
+def test_split_attention(backend, oracle_lib, frames, heads, size):
+    rng = np.random.default_rng(frames)
+    width = heads * size
+    q, k, v = (rng.uniform(-s, s, (frames, width)).astype(np.float32) for s in (3, 3, 4))
+    q[0] *= 8  # one peaked row
+    expected = oracle_lib.attention_f64(q, k, v, frames, width, heads)
+    assert np.abs(attend(backend, q, k, v, heads) - expected).max() <= 5e-5 * 4
+
+
+@pytest.mark.parametrize("value", [2.0**-101, 2.0**70, np.inf, np.nan])
+def test_split_attention_range(backend, oracle_lib, value):
+    """A value that the planes do not hold moves its head, and only it, to fp32."""
+    rng = np.random.default_rng(3)
+    frames, heads, size = 450, 3, 128
+    q, k, v = (rng.uniform(-2, 2, (frames, heads * size)).astype(np.float32) for _ in range(3))
+    plain = attend(backend, q, k, v, heads)
+    v[7, size + 5] = value
+    got = attend(backend, q, k, v, heads)
+    other = np.ones(heads * size, bool)
+    other[size:2 * size] = False
+    assert np.array_equal(got[:, other].view(np.uint32), plain[:, other].view(np.uint32))
+    if np.isfinite(value):
+        expected = oracle_lib.attention_f64(q, k, v, frames, heads * size, heads)
+        assert np.all(np.abs(got - expected) <= 5e-5 * np.maximum(4, np.abs(expected)))
+    else:
+        assert not np.any(np.isfinite(got[:, size + 5]))
+    # The workspace serves the next call as before.
+    v[7, size + 5] = 1.0
+    again = attend(backend, q, k, v, heads)
+    assert np.all(np.isfinite(again)) and np.array_equal(again, attend(backend, q, k, v, heads))
