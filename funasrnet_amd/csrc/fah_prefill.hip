@@ -906,14 +906,16 @@ __device__ __forceinline__ f32x16 outer16(float a, float b) {
   return __builtin_amdgcn_mfma_f32_16x16x1f32(a, b, zero, 0, 0, 0);
 }
 
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void attn_rows_kernel(PrefillAttnArgs a) {
+template <int kRowThreads>
+__global__ __launch_bounds__(kRowThreads) __attribute__((amdgpu_waves_per_eu(2))) void attn_rows_kernel(PrefillAttnArgs a) {
   extern __shared__ __attribute__((aligned(16))) float rows_s[];
   __shared__ __attribute__((aligned(16))) float q_s[kRowPairs * kQRow];  // q rows, then output rows
   __shared__ double lane_s[kRowPairs * 8];
   __shared__ float inv_s[kRowPairs];
   // The last row blocks see the most positions: they are dispatched first.
   const int kh = blockIdx.x, r0 = (gridDim.y - 1 - blockIdx.y) * kRowBlock, tid = threadIdx.x;
-  const int lane = tid & 63, wave = tid >> 6, hs = 128;
+  constexpr int hs = 128;
+  const int lane = tid & 63, wave = tid >> 6;
   const int rows = min(kRowBlock, a.frames - r0);
   const int n0 = a.position + r0 + 1;  // positions the block's first row sees; row rr sees n0 + rr
   const int nmax = n0 + rows - 1;
@@ -922,7 +924,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void a
   char* ring = reinterpret_cast<char*>(rows_s + (size_t)kRowPairs * PS);
   const _Float16* kc = a.kcache + (size_t)kh * a.capacity * hs;
   const _Float16* vc = a.vcache + (size_t)kh * a.capacity * hs;
-  for (int i = tid; i < kRowPairs * hs; i += 256) {
+  for (int i = tid; i < kRowPairs * hs; i += kRowThreads) {
     const int pi = i >> 7, c = i & 127, hh = pi >> 3, rr = pi & 7;
     q_s[pi * kQRow + c] = rr < rows ? a.q[((size_t)(r0 + rr) * a.heads + 2 * kh + hh) * hs + c] : 0.0f;
   }
@@ -933,7 +935,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void a
   // from LDS), its 16 products added to the channel's accumulator (c % 8) of
   // each (pair, position) the lane holds.
   const int mp = lane & 15, mg = lane >> 4;
-  for (int t0 = 64 * wave; t0 < nmax; t0 += 256) {
+  for (int t0 = 64 * wave; t0 < nmax; t0 += kRowThreads) {
     const uint4* row = reinterpret_cast<const uint4*>(kc + (size_t)min(t0 + lane, nmax - 1) * hs);
     uint4 kk[16];
 #pragma unroll
@@ -1002,15 +1004,17 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void a
   }
   __syncthreads();
 
-  // 2. Softmax: 16 lanes per pair, four pairs per wave.
-  const int pi = wave * 4 + (lane >> 4), sub = lane & 15;
+  // 2. Softmax: kLanes lanes per pair.
+  constexpr int kLanes = kRowThreads / kRowPairs;
+  const int pi = tid / kLanes, sub = tid % kLanes;
   const int n = (pi & 7) < rows ? n0 + (pi & 7) : 0;
   float* pp = p_s + (size_t)pi * PS;
   {
     float m = -__builtin_inff();
-    for (int t = sub; t < n; t += 16) m = nan_max_p(m, pp[t]);
+    for (int t = sub; t < n; t += kLanes) m = nan_max_p(m, pp[t]);
     m = max16_nan(m);
-    for (int t = sub; t < n; t += 16) pp[t] = exp_ref(fadd(pp[t], -m));
+    if (kLanes == 32) m = nan_max_p(m, __shfl_xor(m, 16, 64));
+    for (int t = sub; t < n; t += kLanes) pp[t] = exp_ref(fadd(pp[t], -m));
   }
   __syncthreads();
   const int full = n & ~7;
@@ -1038,50 +1042,51 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void a
   __syncthreads();
   {
     const float inverse = n > 0 ? inv_s[pi] : 0.0f;
-    for (int t = sub; t < n; t += 16) pp[t] = fmul(pp[t], inverse);
+    for (int t = sub; t < n; t += kLanes) pp[t] = fmul(pp[t], inverse);
   }
 
-  // 3. Time-ordered value sums, all four waves: wave w owns channels
-  // 32 w .. 32 w + 31 as two groups of 16. One outer product covers four
-  // positions t .. t + 3 (one per 16 x 16 block: the 16 pairs' probabilities
-  // at t + b times 16 channels' v at t + b), so lane l holds, for channel
-  // 32 w + 16 h + l % 16 and pairs 4 (l / 16) + r, the products of four
-  // consecutive positions and adds them in order. V rows pass through a
+  // 3. Time-ordered value sums, all waves: wave w owns kGroups groups of 16
+  // channels from 16 kGroups w on. One outer product covers four positions t .. t + 3
+  // (one per 16 x 16 block: the 16 pairs' probabilities at t + b times 16
+  // channels' v at t + b), so lane l holds, for a channel and
+  // pairs 4 (l / 16) + r, the products of four consecutive positions and
+  // adds them in order. V rows pass through a
   // two-slot LDS ring (direct global->LDS loads of 16-byte pieces, the next
   // chunk's issued before this one is added; a slot is refilled only after
   // the barrier that follows its last use).
+  constexpr int kGroups = 512 / kRowThreads;
   const int chunks = (nmax + kVRing - 1) / kVRing;
   auto fill = [&](int j) {  // rows past the last are read again, unused
 #pragma unroll
-    for (int m = 0; m < 2; ++m) {
-      const int piece = tid + 256 * m, rr = piece >> 4;
-      const int row = min(j * kVRing + rr, nmax - 1);
+    for (int m = 0; m < kGroups; ++m) {
+      const int piece = tid + kRowThreads * m, row = min(j * kVRing + (piece >> 4), nmax - 1);
       const char* src = reinterpret_cast<const char*>(vc) + (size_t)row * 256 + 16 * (piece & 15);
-      __builtin_amdgcn_global_load_lds(src, (lds_ptr)(ring + (size_t)(j & 1) * kVRing * 256 + 1024 * (4 * m + wave)), 16, 0, 0);
+      __builtin_amdgcn_global_load_lds(src, (lds_ptr)(ring + (size_t)(j & 1) * kVRing * 256 + kRowThreads * 16 * m + 1024 * wave),
+                                       16, 0, 0);
     }
   };
   fill(0);
   __builtin_amdgcn_s_waitcnt(0);
   __syncthreads();  // the normalised probabilities and the first V chunk
-  float acc[2][4] = {{0.0f, 0.0f, 0.0f, 0.0f}, {0.0f, 0.0f, 0.0f, 0.0f}};
+  float acc[kGroups][4] = {};
   const float* pa = p_s + (size_t)mp * PS + mg;  // A operand: pair mp at position t + l / 16
   for (int j = 0; j < chunks; ++j) {
     if (j + 1 < chunks) fill(j + 1);
-    const _Float16* vr = reinterpret_cast<const _Float16*>(ring + (size_t)(j & 1) * kVRing * 256) + mg * hs + 32 * wave + mp;
+    const _Float16* vr = reinterpret_cast<const _Float16*>(ring + (size_t)(j & 1) * kVRing * 256) + mg * hs + 16 * kGroups * wave + mp;
     const int t0 = j * kVRing, len = min(kVRing, nmax - t0);
     for (int s = 0; s < len; s += 4) {
       const int t = t0 + s;
       const float av = pa[t];
-      const f32x16 d0 = outer16(av, (float)vr[s * hs]);
-      const f32x16 d1 = outer16(av, (float)vr[s * hs + 16]);
+      f32x16 d[kGroups];
+#pragma unroll
+      for (int h = 0; h < kGroups; ++h) d[h] = outer16(av, (float)vr[s * hs + 16 * h]);
       if (t + 3 < n0) {  // every row of the block sees all four positions
 #pragma unroll
         for (int b = 0; b < 4; ++b)
 #pragma unroll
-          for (int r = 0; r < 4; ++r) {
-            acc[0][r] = fadd(acc[0][r], d0[4 * b + r]);
-            acc[1][r] = fadd(acc[1][r], d1[4 * b + r]);
-          }
+          for (int r = 0; r < 4; ++r)
+#pragma unroll
+            for (int h = 0; h < kGroups; ++h) acc[h][r] = fadd(acc[h][r], d[h][4 * b + r]);
       } else {
 #pragma unroll
         for (int b = 0; b < 4; ++b)
@@ -1089,8 +1094,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void a
           for (int r = 0; r < 4; ++r) {
             const int rr = (4 * mg + r) & 7;  // the pair's row: it sees positions < n0 + rr
             if (t + b < n0 + rr) {
-              acc[0][r] = fadd(acc[0][r], d0[4 * b + r]);
-              acc[1][r] = fadd(acc[1][r], d1[4 * b + r]);
+#pragma unroll
+              for (int h = 0; h < kGroups; ++h) acc[h][r] = fadd(acc[h][r], d[h][4 * b + r]);
             }
           }
       }
@@ -1100,19 +1105,19 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void a
   }
 
   // 4. Output rows (float and/or Q8_0 blocks): pair 4 mg + r, channel
-  // 32 w + 16 h + mp.
+  // 16 kGroups w + 16 h + mp.
 #pragma unroll
-  for (int h = 0; h < 2; ++h)
+  for (int h = 0; h < kGroups; ++h)
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
-      const int pq = 4 * mg + r, c = 32 * wave + 16 * h + mp, rr = pq & 7;
+      const int pq = 4 * mg + r, c = 16 * (kGroups * wave + h) + mp, rr = pq & 7;
       q_s[pq * kQRow + c] = acc[h][r];
       if (a.out && rr < rows) a.out[((size_t)(r0 + rr) * a.heads + 2 * kh + (pq >> 3)) * hs + c] = acc[h][r];
     }
   if (a.xq) {
     __syncthreads();
 #pragma unroll
-    for (int g0 = 0; g0 < kRowPairs * hs / 4; g0 += 256) {
+    for (int g0 = 0; g0 < kRowPairs * hs / 4; g0 += kRowThreads) {
       const int g = g0 + tid, pq = g >> 5, c4 = (g & 31) * 4, rr = pq & 7;
       const float4 v4 = *reinterpret_cast<const float4*>(q_s + pq * kQRow + c4);
       float d;
@@ -1276,10 +1281,19 @@ hipError_t launch_attn_prefill(const PrefillAttnArgs& args, hipStream_t s) {
   if (raised != hipSuccess) return raised;
   // Many rows of one cache (a prefill): blocks of rows share K/V reads.
   if (!a.sessions && a.heads == 2 * a.kv_heads && a.frames >= 2 * kRowBlock && rows_lds_bytes(n) <= kStageLds) {
-    static const hipError_t raised_rows = hipFuncSetAttribute(
-        reinterpret_cast<const void*>(attn_rows_kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)kStageLds);
-    if (raised_rows != hipSuccess) return raised_rows;
-    attn_rows_kernel<<<dim3(a.kv_heads, (a.frames + kRowBlock - 1) / kRowBlock), 256, rows_lds_bytes(n), s>>>(a);
+    const dim3 grid(a.kv_heads, (a.frames + kRowBlock - 1) / kRowBlock);
+    const auto rows = [&](auto kernel, int threads) {
+      static const hipError_t raised_rows =
+          hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)kStageLds);
+      if (raised_rows == hipSuccess) kernel<<<grid, threads, rows_lds_bytes(n), s>>>(a);
+      return raised_rows;
+    };
+    // Up to two workgroups a CU, the time is that of the last rows' workgroup,
+    // which eight waves shorten (375 rows: 49.5 -> 39 us a layer); with more, two
+    // workgroups of four waves a CU fill each other's waits (prefill of 750 rows
+    // 5.6 ms against 6.3; 500 rows, 504 workgroups, 4.76 and 4.68).
+    const hipError_t e = grid.x * grid.y <= 512 ? rows(attn_rows_kernel<512>, 512) : rows(attn_rows_kernel<256>, 256);
+    if (e != hipSuccess) return e;
     return hipGetLastError();
   }
   attn_prefill_kernel<<<dim3(a.heads, a.frames), 256, a.stage ? staged : (size_t)n * 4, s>>>(a);
