@@ -6,7 +6,7 @@
 // q8_gemm_kernel: out[t][r] = sum over blocks b, in order, from 0f, of
 // ((float)dot_b * w_scale[r][b]) * x_scale[t][b]. The exact int32 32-term
 // block dots come from one v_mfma_i32_16x16x32_i8 per block and 16x16 tile
-// with a zero accumulator; the fp32 steps then run on the result registers
+// with a constant accumulator; the fp32 steps then run on the result registers
 // in block order, so the result is the one of the reference's per-row loop
 // for every frame. Row and frame scales are staged in LDS as fp32.
 //
@@ -22,7 +22,6 @@
 namespace fah {
 namespace {
 
-constexpr int kGT = 256;  // threads per GEMM workgroup
 using lds_ptr = __attribute__((address_space(3))) void*;
 typedef int v4i __attribute__((ext_vector_type(4)));
 typedef int v2i __attribute__((ext_vector_type(2)));
@@ -52,262 +51,331 @@ __device__ __forceinline__ int gate_up_row(int r, int kind, int base, int extra)
   return 2 * r0 + kind * count + (r - r0);
 }
 
-// One wave owns a (16 TR) x (16 TF) tile of 16x16 MFMA tiles; a workgroup
-// (4 waves, 2 x 2) owns (32 TR) x (32 TF). SwiGLU workgroups hold 16 TR gate
-// rows (waves 0 and 2) and the matching 16 TR up rows (waves 1 and 3).
-// Operands move through LDS in stages of four blocks (128 bytes of every
-// tile row, 16 bytes a lane): the next stage's global loads are in flight in
-// registers while the current stage is computed, then written to the other
-// LDS buffer. The 16-byte chunk c of tile row t sits at slot c ^ (t & 7), so
-// that the 16 rows of an MFMA operand read spread over the banks.
-constexpr int kStages = 2;
-constexpr int kStageBlocks = 4;
+// One wave owns a (16 TI frames) x (16 TJ storage rows) tile of 16x16 MFMA
+// tiles, a workgroup WF x WR of them. SwiGLU waves hold 8 TJ gate rows (tiles
+// 0 .. TJ / 2 - 1) and the matching up rows.
+//
+// What bounds it: the ordered fp32 steps, at three VALU operations a row, frame
+// and block. The dots' MFMA starts from 0x4b400000, the bits of 1.5 2^23, so
+// that its integer result is, as a float, 1.5 2^23 + dot exactly; with c =
+// -1.5 2^23 w_scale (exact: w_scale has 11 bits), fma(result, w_scale, c) is
+// dot w_scale rounded once, what (float)dot * w_scale is, without the
+// conversion. (fp32 scales keep the conversion: c would round. An infinite
+// scale makes c infinite: sums that are not finite are formed again by
+// row_reference.) Rows and scales move through LDS in stages of SB blocks, one
+// stage in use, one being filled, two in registers or on their way; rows are
+// padded so that the 16 rows of an operand read fall on distinct banks, and
+// hold the pieces of two blocks side by side (one 16-byte read an operand and
+// pair). The pipeline is written out (operands a pair of blocks ahead, dots a
+// block ahead): the compiler had each block's reads, MFMA and terms wait for
+// each other (28 x 2048 -> 1024 at SB = 8: 9.1 us, then 7.2).
+// Lane layout of the result: frame 4 (l / 16) + j, row l % 16.
+//
+// Measured against the four-operation kernel with rows as the MFMA's rows, us:
+// 28 x 2048 -> 1024 9.2 -> 7.2, 100 x 3072 -> 1024 12.9 -> 9.6, 375 x 3072 -> 1024
+// 15.7 -> 13.8, 375 x 1024 -> 4096 13.9 -> 13.5, 500 x 2944 -> 6000 50.5 -> 44.8. At
+// the largest the VALU is busy for two thirds of the CU's time and the MFMAs
+// for a sixth; below, the serial block chain of a wave (about 110 cycles a
+// block of 16 x 16) is what is left. Weights read straight from memory in the
+// operand's order (32 bytes a row and load) took two to three times as long.
+constexpr int kMagicBits = 0x4b400000;
+constexpr float kMagic = 12582912.0f;  // 1.5 2^23
 
-template <class Scale, int OUT, int TR, int TF>
-__global__ __launch_bounds__(kGT) void q8_gemm_kernel(GemmArgs g) {
-  extern __shared__ __attribute__((aligned(16))) float gemm_s[];
-  constexpr bool kSwiGLU = OUT == kGemmSwiGLU;
-  constexpr int RW = 16 * TR, FW = 16 * TF;  // wave tile
-  constexpr int RT = 2 * RW, FT = 2 * FW;    // workgroup tile (SwiGLU: gate rows then up rows)
-  constexpr int LR = kSwiGLU ? RW : RT;      // logical rows per workgroup
-  constexpr int US = LR + 4;                 // up_s row stride (floats)
-  constexpr int kRowBytes = 32 * kStageBlocks;
-  // A stage: operand rows [RT + FT][128 B], then the stage's scales as fp32,
-  // [4][RT] for the rows and [4][FT] for the frames.
-  constexpr int kOperandBytes = (RT + FT) * kRowBytes;
-  constexpr int kStageBytes = kOperandBytes + (RT + FT) * kStageBlocks * 4;
-  const int B = g.K >> 5;
-  char* stage_s = reinterpret_cast<char*>(gemm_s);                                 // [kStages][kStageBytes]
-  float* up_s = reinterpret_cast<float*>(stage_s + kStages * kStageBytes);         // SwiGLU: [FT][US] up sums
-  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-  const int wr = wave & 1, wf = wave >> 1;
-  const int row0 = blockIdx.x * LR, f0 = blockIdx.y * FT;
-  // Tile row tr (0..RT-1) -> storage row, or -1 past the end.
-  auto storage_row = [&](int tr) -> int {
+// One output's block terms in order, from memory.
+template <class Scale>
+__device__ __forceinline__ float row_reference(const int8_t* w, const typename Scale::type* ws, const int8_t* x,
+                                            const float* xs, int B) {
+  float sum = 0.0f;
+#pragma unroll 1
+  for (int b = 0; b < B; ++b) {
+    int dot = 0;
+#pragma unroll 1
+    for (int i = 0; i < 32; ++i) dot += (int)w[32 * b + i] * (int)x[32 * b + i];
+    sum = fadd(sum, fmul(fmul((float)dot, Scale::get(ws[b])), xs[b]));
+  }
+  return sum;
+}
+
+template <class Scale, int OUT, int WF, int WR, int TI, int TJ, int SB>
+__global__ __launch_bounds__(64 * WF * WR) void q8_gemm_kernel(GemmArgs g) {
+  constexpr bool kSwiGLU = OUT == kGemmSwiGLU, kHalf = sizeof(typename Scale::type) == 2;
+  constexpr int LW = kSwiGLU ? 8 * TJ : 16 * TJ;  // logical rows a wave
+  constexpr int NT = 64 * WF * WR, FT = 16 * TI * WF, RT = 16 * TJ * WR;  // threads; frames and storage rows
+  constexpr int ROW = 32 * SB + 16, kStage = (FT + RT) * (ROW + 4 * SB);
+  constexpr int CH = 2 * SB, RP = NT / CH, SP = NT / SB;  // 16-byte pieces a row; rows and scale rows a pass
+  constexpr int WP = (RT + RP - 1) / RP, XP = (FT + RP - 1) / RP, WS = (RT + SP - 1) / SP, XS = (FT + SP - 1) / SP;
+  using ST = typename Scale::type;
+  extern __shared__ __attribute__((aligned(16))) char gemm_s[];  // two stages: rows, then scales [SB][FT], [SB / 4][RT][4]
+  const int B = g.K >> 5, stages = (B + SB - 1) / SB;
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, l16 = lane & 15, kq = lane >> 4;
+  const int wf = wave / WR, wr = wave % WR;
+  // Workgroups are dealt to the eight XCDs in turn: each XCD takes a run of
+  // consecutive tiles, frames fastest, so that its L2 holds few weight rows.
+  const int mt = (g.frames + FT - 1) / FT, tiles = gridDim.x, xcd = blockIdx.x & 7, q8 = tiles >> 3, r8 = tiles & 7;
+  const int tile = xcd * q8 + min(xcd, r8) + (blockIdx.x >> 3);
+  const int f0 = tile % mt * FT, r0 = tile / mt * WR * LW;
+  // Storage row of the workgroup's row t (tile t / 16 % TJ of wave row t / (16
+  // TJ)); rows past the end repeat the last one (never stored).
+  auto storage_row = [&](int t) -> int {
+    const int first = r0 + t / (16 * TJ) * LW, j = t / 16 % TJ;
     if (kSwiGLU) {
-      const int r = row0 + tr % RW;
-      if (r >= g.rows) return -1;
-      return g.gu_map ? g.gu_map[2 * r + tr / RW] : gate_up_row(r, tr / RW, g.split_base, g.split_extra);
+      const int r = min(first + 16 * (j % (TJ / 2)) + t % 16, g.rows - 1), kind = j / (TJ / 2);
+      return g.gu_map ? g.gu_map[2 * r + kind] : gate_up_row(r, kind, g.split_base, g.split_extra);
     }
-    const int r = row0 + tr;
-    return r < g.rows ? r : -1;
+    return min(first + 16 * j + t % 16, g.rows - 1);
   };
-
-  // Stage loads: piece j of a stage is tile rows 8j..8j+7 (rows [0, RT) are
-  // weight rows, [RT, RT + FT) frames); lane l takes row 8j + l/8, chunk
-  // (l%8) ^ (row & 7), and writes it to slot l%8. Threads [0, RT) also take
-  // their row's four block scales, threads [RT, RT + FT) their frame's. Rows
-  // past the matrix and frames past the input load row / frame 0 (scale 0):
-  // never stored.
-  constexpr int kLoads = (RT + FT) / 8;
-  static_assert(kLoads % 4 == 0, "every wave moves the same number of pieces");
-  static_assert(RT + FT <= kGT, "one scale load per thread");
-  constexpr int kPerWave = kLoads / 4;
-  const int8_t* src[kPerWave];
+  // A stage: thread t takes piece t % CH of every RPth row from t / CH on, and
+  // the scale of block t % SB of every SPth row from t / SB on.
+  const int8_t *wsrc[WP], *xsrc[XP];
+  const ST* wssrc[WS];
+  const float* xssrc[XS];
 #pragma unroll
-  for (int i = 0; i < kPerWave; ++i) {
-    const int t = 8 * (wave + 4 * i) + (lane >> 3);
-    const int chunk = (lane & 7) ^ (t & 7);
-    if (t < RT) {
-      const int sr = storage_row(t);
-      src[i] = g.w + (size_t)max(sr, 0) * g.K + 16 * chunk;
-    } else {
-      const int f = f0 + t - RT;
-      src[i] = g.xq + (size_t)(f < g.frames ? f : 0) * g.K + 16 * chunk;
+  for (int i = 0; i < WP; ++i) wsrc[i] = g.w + (size_t)storage_row(min(RP * i + tid / CH, RT - 1)) * g.K;
+#pragma unroll
+  for (int i = 0; i < WS; ++i)
+    wssrc[i] = reinterpret_cast<const ST*>(g.ws) + (size_t)storage_row(min(SP * i + tid / SB, RT - 1)) * B;
+#pragma unroll
+  for (int i = 0; i < XP; ++i) xsrc[i] = g.xq + (size_t)min(f0 + RP * i + tid / CH, g.frames - 1) * g.K;
+#pragma unroll
+  for (int i = 0; i < XS; ++i) xssrc[i] = g.xs + (size_t)min(f0 + SP * i + tid / SB, g.frames - 1) * B;
+  constexpr int P = 2;  // stages on their way or in registers
+  struct Pending {
+    v4i w[WP], x[XP];
+    ST ws[WS];
+    float xs[XS];
+  } pending[P];
+  auto fetch = [&](Pending& p, int st) {
+    st = min(st, stages - 1);
+    // (B is a multiple of four: only a stage of eight can reach past the last
+    // block, where frame scales of zero make terms of zero.)
+    const int k = min(32 * SB * st + 16 * (tid % CH), g.K - 16), blk = SB * st + tid % SB, b = min(blk, B - 1);
+#pragma unroll
+    for (int i = 0; i < WP; ++i) p.w[i] = *reinterpret_cast<const v4i*>(wsrc[i] + k);
+#pragma unroll
+    for (int i = 0; i < XP; ++i) p.x[i] = *reinterpret_cast<const v4i*>(xsrc[i] + k);
+#pragma unroll
+    for (int i = 0; i < WS; ++i) p.ws[i] = wssrc[i][b];
+#pragma unroll
+    for (int i = 0; i < XS; ++i) {
+      const float s = xssrc[i][b];
+      p.xs[i] = blk < B ? s : 0.0f;
+    }
+  };
+  // Rows in LDS: for each pair of blocks [kq 4][block 2] 8-byte pieces, so that
+  // a lane reads its operands of two blocks at once.
+  const int piece_at = (tid % CH / 4) * 64 + (tid % 2) * 32 + (tid % CH / 2 % 2) * 8;
+  auto put = [&](const Pending& p, int buf) {
+    char* rows = gemm_s + buf * kStage + (tid / CH) * ROW + piece_at;  // frames, then weights
+    float* scales = reinterpret_cast<float*>(gemm_s + buf * kStage + (FT + RT) * ROW);
+#pragma unroll
+    for (int i = 0; i < XP; ++i)
+      if (FT % RP == 0 || RP * i + tid / CH < FT) {
+        *reinterpret_cast<v2i*>(rows + RP * i * ROW) = v2i{p.x[i].x, p.x[i].y};
+        *reinterpret_cast<v2i*>(rows + RP * i * ROW + 16) = v2i{p.x[i].z, p.x[i].w};
+      }
+#pragma unroll
+    for (int i = 0; i < WP; ++i)
+      if (RT % RP == 0 || RP * i + tid / CH < RT) {
+        *reinterpret_cast<v2i*>(rows + (FT + RP * i) * ROW) = v2i{p.w[i].x, p.w[i].y};
+        *reinterpret_cast<v2i*>(rows + (FT + RP * i) * ROW + 16) = v2i{p.w[i].z, p.w[i].w};
+      }
+#pragma unroll
+    for (int i = 0; i < XS; ++i)
+      if (FT % SP == 0 || SP * i + tid / SB < FT) scales[tid % SB * FT + SP * i + tid / SB] = p.xs[i];
+#pragma unroll
+    for (int i = 0; i < WS; ++i)
+      if (RT % SP == 0 || SP * i + tid / SB < RT)
+        scales[SB * FT + (tid % SB / 4 * RT + SP * i + tid / SB) * 4 + tid % 4] = Scale::get(p.ws[i]);
+  };
+  const v4i start = kHalf ? v4i{kMagicBits, kMagicBits, kMagicBits, kMagicBits} : v4i{0, 0, 0, 0};
+  float acc[TI][TJ][4];
+#pragma unroll
+  for (int i = 0; i < TI; ++i)
+#pragma unroll
+    for (int j = 0; j < TJ; ++j)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) acc[i][j][e] = 0.0f;
+  auto compute = [&](int buf) {
+    const char* x_rows = gemm_s + buf * kStage + (16 * TI * wf + l16) * ROW + 16 * kq;
+    const char* w_rows = gemm_s + buf * kStage + (FT + 16 * TJ * wr + l16) * ROW + 16 * kq;
+    const float* xs = reinterpret_cast<const float*>(gemm_s + buf * kStage + (FT + RT) * ROW) + 16 * TI * wf + 4 * kq;
+    const float* ws = reinterpret_cast<const float*>(gemm_s + buf * kStage + (FT + RT) * ROW) + SB * FT + 4 * (16 * TJ * wr + l16);
+    // Operands of a pair of blocks are read a pair ahead of their terms, dots
+    // formed a block ahead.
+    struct Operands {
+      union Two {
+        v4i v;
+        long block[2];
+      } a[TI], w[TJ];
+      float4 x[2][TI];
+    } o[2];
+    float4 s[TJ];
+    v4i d[2][TI][TJ];
+    auto read = [&](Operands& p, int pair) {
+#pragma unroll
+      for (int j = 0; j < TJ; ++j) p.w[j].v = *reinterpret_cast<const v4i*>(w_rows + 16 * j * ROW + 64 * pair);
+#pragma unroll
+      for (int i = 0; i < TI; ++i) p.a[i].v = *reinterpret_cast<const v4i*>(x_rows + 16 * i * ROW + 64 * pair);
+#pragma unroll
+      for (int u = 0; u < 2; ++u)
+#pragma unroll
+        for (int i = 0; i < TI; ++i) p.x[u][i] = *reinterpret_cast<const float4*>(xs + (2 * pair + u) * FT + 16 * i);
+    };
+    auto dots = [&](const Operands& p, int u, v4i(&r)[TI][TJ]) {
+#pragma unroll
+      for (int i = 0; i < TI; ++i)
+#pragma unroll
+        for (int j = 0; j < TJ; ++j)
+          r[i][j] = __builtin_amdgcn_mfma_i32_16x16x32_i8(p.a[i].block[u], p.w[j].block[u], start, 0, 0, 0);
+    };
+    read(o[0], 0);
+#pragma unroll
+    for (int j = 0; j < TJ; ++j) s[j] = *reinterpret_cast<const float4*>(ws + 64 * j);
+    __builtin_amdgcn_sched_barrier(0);
+    dots(o[0], 0, d[0]);
+#pragma unroll
+    for (int blk = 0; blk < SB; ++blk) {
+      const Operands& p = o[blk / 2 & 1];
+      if (blk % 2 == 0) {
+        if (blk + 2 < SB) read(o[(blk / 2 + 1) & 1], blk / 2 + 1);
+        dots(p, 1, d[1]);
+      } else if (blk + 1 < SB) {
+        dots(o[(blk / 2 + 1) & 1], 0, d[0]);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int j = 0; j < TJ; ++j) {
+        const float sj = blk % 4 == 0 ? s[j].x : blk % 4 == 1 ? s[j].y : blk % 4 == 2 ? s[j].z : s[j].w, c = -kMagic * sj;
+#pragma unroll
+        for (int i = 0; i < TI; ++i) {
+          const float4 xv = p.x[blk & 1][i];
+          const float x4[4] = {xv.x, xv.y, xv.z, xv.w};
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            const int dot = d[blk & 1][i][j][e];
+            const float t = kHalf ? __builtin_fmaf(u2f((uint32_t)dot), sj, c) : fmul((float)dot, sj);
+            acc[i][j][e] = fadd(acc[i][j][e], fmul(t, x4[e]));
+          }
+        }
+      }
+      if (blk % 4 == 3 && blk + 1 < SB) {
+#pragma unroll
+        for (int j = 0; j < TJ; ++j) s[j] = *reinterpret_cast<const float4*>(ws + (blk + 1) / 4 * RT * 4 + 64 * j);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  };
+#pragma unroll
+  for (int p = 0; p < P; ++p) fetch(pending[p], p);
+  put(pending[0], 0);
+  fetch(pending[0], P);
+  lds_barrier();
+  for (int st = 0; st < stages; st += P) {
+#pragma unroll
+    for (int p = 0; p < P; ++p) {
+      __builtin_amdgcn_sched_barrier(0);
+      if (p == 0 || st + p < stages) compute(p & 1);
+      put(pending[(p + 1) % P], (p & 1) ^ 1);
+      fetch(pending[(p + 1) % P], st + p + 1 + P);
+      lds_barrier();
     }
   }
-  // Scales of a stage: thread t takes block t % 4 of row t / 4 and of frame
-  // t / 4 (rows and frames past the tile or the matrix read row / frame 0,
-  // and past the matrix store scale 0).
-  using ST = typename Scale::type;
-  static_assert(RT <= 64 && FT <= 64, "one row scale and one frame scale per thread");
-  const int sblk = tid & 3, srow = tid >> 2;
-  const int s_sr = srow < RT ? storage_row(srow) : -1;
-  const int s_f = f0 + srow;
-  const bool row_live = s_sr >= 0, frame_live = srow < FT && s_f < g.frames;
-  const ST* wsrc = reinterpret_cast<const ST*>(g.ws) + (size_t)max(s_sr, 0) * B + sblk;
-  const float* xsrc = g.xs + (size_t)(frame_live ? s_f : 0) * B + sblk;
-  v4i pending[kPerWave];
-  ST wraw;
-  float xraw;
-  auto fetch = [&](int st) {  // stage st: blocks [4 st, 4 st + 4)
+  const int row0 = r0 + wr * LW;
+  const int fw = f0 + 16 * TI * wf;  // this wave's first frame
+  bool odd = false;
 #pragma unroll
-    for (int i = 0; i < kPerWave; ++i) pending[i] = *reinterpret_cast<const v4i*>(src[i] + (size_t)st * kRowBytes);
-    wraw = wsrc[kStageBlocks * st];
-    xraw = xsrc[kStageBlocks * st];
-  };
-  auto put = [&](int st) {
-    char* base = stage_s + (st % kStages) * kStageBytes;
+  for (int i = 0; i < TI; ++i)
 #pragma unroll
-    for (int i = 0; i < kPerWave; ++i) *reinterpret_cast<v4i*>(base + (wave + 4 * i) * 1024 + 16 * lane) = pending[i];
-    float* sc = reinterpret_cast<float*>(base + kOperandBytes);  // [4][RT] rows, then [4][FT] frames
-    if (srow < RT) sc[sblk * RT + srow] = row_live ? Scale::get(wraw) : 0.0f;
-    if (srow < FT) sc[kStageBlocks * RT + sblk * FT + srow] = frame_live ? xraw : 0.0f;
-  };
-  const int stages = B / kStageBlocks;
-  fetch(0);
-  put(0);
-  fetch(min(1, stages - 1));
-  lds_barrier();
-
-  // MFMA operand of lane l: 8 bytes of row (frame) l % 16 at byte 8 (l / 16)
-  // of the block; result register j of lane l: row 4 (l / 16) + j, frame l % 16.
-  const int l16 = lane & 15, kq = lane >> 4;
-  int a_at[TR], b_at[TF];  // byte offsets of this lane's operand rows in a stage
+    for (int j = 0; j < TJ; ++j)
 #pragma unroll
-  for (int tr = 0; tr < TR; ++tr) a_at[tr] = (wr * RW + 16 * tr + l16) * kRowBytes;
+      for (int e = 0; e < 4; ++e) odd = odd || (f2u(acc[i][j][e]) & 0x7fffffffu) >= 0x7f800000u;
+  if (kHalf && __any(odd)) {
 #pragma unroll
-  for (int tf = 0; tf < TF; ++tf) b_at[tf] = (RT + wf * FW + 16 * tf + l16) * kRowBytes;
-  // Chunk 2 blk + kq/2 of row t sits at slot (2 blk + kq/2) ^ (t & 7); every
-  // operand row of this lane has t & 7 == l16 & 7.
-  auto at = [&](int row_at, int blk) { return row_at + 16 * ((2 * blk + (kq >> 1)) ^ (l16 & 7)) + 8 * (kq & 1); };
-  const v4i zero4 = {0, 0, 0, 0};
-  float acc[TR][TF][4];
+    for (int i = 0; i < TI; ++i)
 #pragma unroll
-  for (int tr = 0; tr < TR; ++tr)
+      for (int j = 0; j < TJ; ++j)
 #pragma unroll
-    for (int tf = 0; tf < TF; ++tf)
-#pragma unroll
-      for (int j = 0; j < 4; ++j) acc[tr][tf][j] = 0.0f;
-
-  for (int st = 0; st < stages; ++st) {
-    const char* sa = stage_s + (st % kStages) * kStageBytes;
-    const float* ws_s = reinterpret_cast<const float*>(sa + kOperandBytes);  // [4][RT]
-    const float* xs_s = ws_s + kStageBlocks * RT;                           // [4][FT]
-    // Four-tile waves keep two blocks in flight (fewer registers, more waves
-    // a SIMD); single-tile waves all four.
-    constexpr int kBlkUnroll = TR * TF >= 4 ? 2 : kStageBlocks;
-#pragma unroll kBlkUnroll
-    for (int blk = 0; blk < kStageBlocks; ++blk) {
-      long av[TR], bv[TF];
-#pragma unroll
-      for (int tr = 0; tr < TR; ++tr) av[tr] = *reinterpret_cast<const long*>(sa + at(a_at[tr], blk));
-#pragma unroll
-      for (int tf = 0; tf < TF; ++tf) bv[tf] = *reinterpret_cast<const long*>(sa + at(b_at[tf], blk));
-      v4i d[TR][TF];
-#pragma unroll
-      for (int tr = 0; tr < TR; ++tr)
-#pragma unroll
-        for (int tf = 0; tf < TF; ++tf) d[tr][tf] = __builtin_amdgcn_mfma_i32_16x16x32_i8(av[tr], bv[tf], zero4, 0, 0, 0);
-      // The reference's ((float)dot * w_scale) * x_scale, added in block order.
-      float4 w4[TR];
-      float xv[TF];
-#pragma unroll
-      for (int tr = 0; tr < TR; ++tr) w4[tr] = *reinterpret_cast<const float4*>(ws_s + blk * RT + wr * RW + 16 * tr + 4 * kq);
-#pragma unroll
-      for (int tf = 0; tf < TF; ++tf) xv[tf] = xs_s[blk * FT + wf * FW + 16 * tf + l16];
-#pragma unroll
-      for (int tr = 0; tr < TR; ++tr)
-#pragma unroll
-        for (int tf = 0; tf < TF; ++tf) {
-          acc[tr][tf][0] = fadd(acc[tr][tf][0], fmul(fmul((float)d[tr][tf][0], w4[tr].x), xv[tf]));
-          acc[tr][tf][1] = fadd(acc[tr][tf][1], fmul(fmul((float)d[tr][tf][1], w4[tr].y), xv[tf]));
-          acc[tr][tf][2] = fadd(acc[tr][tf][2], fmul(fmul((float)d[tr][tf][2], w4[tr].z), xv[tf]));
-          acc[tr][tf][3] = fadd(acc[tr][tf][3], fmul(fmul((float)d[tr][tf][3], w4[tr].w), xv[tf]));
-        }
-    }
-    // Stage st + 1 into the other buffer (last read at stage st - 1, before
-    // the previous barrier), then stage st + 2's loads into the registers
-    // (past the last stage: the last one again, unused).
-    put(st + 1);
-    fetch(min(st + 2, stages - 1));
-    lds_barrier();
+        for (int e = 0; e < 4; ++e)
+          if ((f2u(acc[i][j][e]) & 0x7fffffffu) >= 0x7f800000u) {
+            const int f = min(fw + 16 * i + 4 * kq + e, g.frames - 1);
+            const int sr = storage_row(16 * (TJ * wr + j) + l16);
+            acc[i][j][e] = row_reference<Scale>(g.w + (size_t)sr * g.K, reinterpret_cast<const ST*>(g.ws) + (size_t)sr * B,
+                                                g.xq + (size_t)f * g.K, g.xs + (size_t)f * B, B);
+          }
   }
 
   if (!kSwiGLU) {
 #pragma unroll
-    for (int tf = 0; tf < TF; ++tf) {
-      const int f = f0 + wf * FW + 16 * tf + l16;
-      if (f >= g.frames) continue;
+    for (int j = 0; j < TJ; ++j) {
+      const int r = row0 + 16 * j + l16;
+      if (r >= g.rows) continue;
+      const float bias = OUT == kGemmPlain && g.bias ? g.bias[r] : 0.0f;
 #pragma unroll
-      for (int tr = 0; tr < TR; ++tr) {
-        const int r = row0 + wr * RW + 16 * tr + 4 * kq;
-        float v[4];
+      for (int i = 0; i < TI; ++i)
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          v[j] = acc[tr][tf][j];
-          if (r + j < g.rows) {
-            if (OUT == kGemmResidual) v[j] = fadd(v[j], g.resid[(size_t)f * g.out_stride + r + j]);
-            if (OUT == kGemmPlain && g.bias) v[j] = fadd(g.bias[r + j], v[j]);
-          }
+        for (int e = 0; e < 4; ++e) {
+          const int f = fw + 16 * i + 4 * kq + e;
+          if (f >= g.frames) continue;
+          const size_t at = (size_t)f * g.out_stride + r;
+          float v = acc[i][j][e];
+          if (OUT == kGemmResidual) v = fadd(v, g.resid[at]);
+          if (OUT == kGemmPlain && g.bias) v = fadd(bias, v);
+          g.out[at] = v;
         }
-        float* o = g.out + (size_t)f * g.out_stride + r;
-        if (r + 3 < g.rows && ((g.out_stride | r) & 3) == 0) {
-          *reinterpret_cast<float4*>(o) = make_float4(v[0], v[1], v[2], v[3]);
-        } else {
-#pragma unroll
-          for (int j = 0; j < 4; ++j)
-            if (r + j < g.rows) o[j] = v[j];
-        }
-      }
     }
   } else {
-    // SwiGLU (Elementwise.cs:167-196): gate waves meet their up rows in LDS.
-    if (wr == 1) {
+    // SwiGLU (Elementwise.cs:167-196).
 #pragma unroll
-      for (int tf = 0; tf < TF; ++tf)
+    for (int i = 0; i < TI; ++i)
 #pragma unroll
-        for (int tr = 0; tr < TR; ++tr)
-          *reinterpret_cast<float4*>(up_s + (wf * FW + 16 * tf + l16) * US + 16 * tr + 4 * kq) =
-              make_float4(acc[tr][tf][0], acc[tr][tf][1], acc[tr][tf][2], acc[tr][tf][3]);
-    }
-    lds_barrier();
-    if (wr == 0) {
+      for (int j = 0; j < TJ / 2; ++j)
 #pragma unroll
-      for (int tf = 0; tf < TF; ++tf) {
-        const int f = f0 + wf * FW + 16 * tf + l16;
-        float h[TR][4];
-#pragma unroll
-        for (int tr = 0; tr < TR; ++tr) {
-          const float4 u = *reinterpret_cast<const float4*>(up_s + (wf * FW + 16 * tf + l16) * US + 16 * tr + 4 * kq);
-          const float uj[4] = {u.x, u.y, u.z, u.w};
-#pragma unroll
-          for (int j = 0; j < 4; ++j) {
-            const float gv = acc[tr][tf][j];
-            const float silu = fdiv(gv, fadd(1.0f, exp_ref(-gv)));
-            h[tr][j] = fmul(silu, uj[j]);
-          }
+        for (int e = 0; e < 4; ++e) {
+          const float gv = acc[i][j][e];
+          acc[i][j][e] = fmul(fdiv(gv, fadd(1.0f, exp_ref(-gv))), acc[i][j + TJ / 2][e]);
         }
-        if (TR == 2 && g.out_q) {
-          // The 32 rows of the workgroup are one Q8_0 block of frame f, held
-          // by lanes l16, l16 + 16, l16 + 32, l16 + 48 (eight values each):
-          // TensorMath.Quantize of the block (amax over the bit patterns).
-          uint32_t m = 0;
+    if (TJ == 2 && WR == 2 && g.out_q) {
+      // The 32 rows of the two wave rows are one Q8_0 block of each frame:
+      // TensorMath.Quantize of it (amax over the bit patterns, 16 lanes of each).
+      uint32_t* amax_s = reinterpret_cast<uint32_t*>(gemm_s);  // [2][FT]
+      uint32_t m[TI][4];
 #pragma unroll
-          for (int tr = 0; tr < TR; ++tr)
+      for (int i = 0; i < TI; ++i)
 #pragma unroll
-            for (int j = 0; j < 4; ++j) {
-              const uint32_t a = f2u(h[tr][j]) & 0x7fffffffu;
-              m = a > m ? a : m;
-            }
-          uint32_t o = (uint32_t)__shfl_xor((int)m, 16);
-          m = o > m ? o : m;
-          o = (uint32_t)__shfl_xor((int)m, 32);
-          m = o > m ? o : m;
+        for (int e = 0; e < 4; ++e) {
+          uint32_t v = f2u(acc[i][0][e]) & 0x7fffffffu;
+          v = max(v, dpp_u32<kDppQuadXor1>(v));
+          v = max(v, dpp_u32<kDppQuadXor2>(v));
+          v = max(v, dpp_u32<kDppHalfMirror>(v));
+          v = max(v, dpp_u32<kDppMirror>(v));
+          m[i][e] = v;
+          if (l16 == 0) amax_s[wr * FT + 16 * (TI * wf + i) + 4 * kq + e] = v;
+        }
+      lds_barrier();
+#pragma unroll
+      for (int i = 0; i < TI; ++i)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const int fl = 16 * (TI * wf + i) + 4 * kq + e, f = f0 + fl;
           float inverse;
-          const float d = block_scale(m, &inverse);
+          const float d = block_scale(max(m[i][e], amax_s[(wr ^ 1) * FT + fl]), &inverse);
           if (f < g.frames) {
-            int8_t* q = g.out_q + (size_t)f * g.rows + row0 + 4 * kq;
-#pragma unroll
-            for (int tr = 0; tr < TR; ++tr) {
-              const uint32_t packed = (uint32_t)(uint8_t)quantize_value(h[tr][0], inverse) |
-                                      ((uint32_t)(uint8_t)quantize_value(h[tr][1], inverse) << 8) |
-                                      ((uint32_t)(uint8_t)quantize_value(h[tr][2], inverse) << 16) |
-                                      ((uint32_t)(uint8_t)quantize_value(h[tr][3], inverse) << 24);
-              *reinterpret_cast<uint32_t*>(q + 16 * tr) = packed;
-            }
-            if (kq == 0) g.out_s[(size_t)f * (g.rows / 32) + row0 / 32] = d;
-          }
-        } else if (f < g.frames) {
-#pragma unroll
-          for (int tr = 0; tr < TR; ++tr) {
-            const int r = row0 + 16 * tr + 4 * kq;
-#pragma unroll
-            for (int j = 0; j < 4; ++j)
-              if (r + j < g.rows) g.out[(size_t)f * g.out_stride + r + j] = h[tr][j];
+            g.out_q[(size_t)f * g.rows + row0 + l16] = quantize_value(acc[i][0][e], inverse);
+            if (wr == 0 && l16 == 0) g.out_s[(size_t)f * (g.rows / 32) + row0 / 32] = d;
           }
         }
-      }
+      return;
+    }
+#pragma unroll
+    for (int j = 0; j < TJ / 2; ++j) {
+      const int r = row0 + 16 * j + l16;
+#pragma unroll
+      for (int i = 0; i < TI; ++i)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const int f = fw + 16 * i + 4 * kq + e;
+          if (f < g.frames && r < g.rows) g.out[(size_t)f * g.out_stride + r] = acc[i][j][e];
+        }
     }
   }
 }
@@ -1131,30 +1199,38 @@ __global__ __launch_bounds__(kRowThreads) __attribute__((amdgpu_waves_per_eu(2))
   }
 }
 
-template <class Scale, int OUT, int TR, int TF>
+template <class Scale, int OUT, int WF, int WR, int TI, int TJ, int SB>
 static hipError_t launch_gemm_tiles(const GemmArgs& g, hipStream_t s) {
-  constexpr int RW = 16 * TR, FW = 16 * TF;
-  constexpr int LR = OUT == kGemmSwiGLU ? RW : 2 * RW;
-  const size_t lds = (size_t)kStages * (2 * RW + 2 * FW) * (32 + 4) * kStageBlocks +
-                     (OUT == kGemmSwiGLU ? (size_t)2 * FW * (LR + 4) * 4 : 0);
-  static const hipError_t raised = hipFuncSetAttribute(reinterpret_cast<const void*>(q8_gemm_kernel<Scale, OUT, TR, TF>),
-                                                       hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+  constexpr int kRows = WR * (OUT == kGemmSwiGLU ? 8 * TJ : 16 * TJ);  // logical rows a workgroup
+  constexpr int kLds = 2 * 16 * (TI * WF + TJ * WR) * (32 * SB + 16 + 4 * SB);
+  static const hipError_t raised = hipFuncSetAttribute(reinterpret_cast<const void*>(q8_gemm_kernel<Scale, OUT, WF, WR, TI, TJ, SB>),
+                                                       hipFuncAttributeMaxDynamicSharedMemorySize, kLds);
   if (raised != hipSuccess) return raised;
-  dim3 grid((g.rows + LR - 1) / LR, (g.frames + 2 * FW - 1) / (2 * FW));
-  q8_gemm_kernel<Scale, OUT, TR, TF><<<grid, kGT, lds, s>>>(g);
+  const int tiles = ((g.rows + kRows - 1) / kRows) * ((g.frames + 16 * TI * WF - 1) / (16 * TI * WF));
+  q8_gemm_kernel<Scale, OUT, WF, WR, TI, TJ, SB><<<tiles, 64 * WF * WR, kLds, s>>>(g);
   return hipGetLastError();
 }
 
-// Largest wave tile that still gives the chip about two waves per SIMD.
+// The largest tile that still loads the chip. Measured, us (64 x 64, 32 x 64,
+// 32 x 32 with stages of eight blocks; frames x K -> rows): 750 x 1024 -> 4096
+// 20.7 25.1 27.7; 500 x 2944 -> 6000 44.8 55.3 63.0; 375 x 1024 -> 4096 14.6 13.5
+// 15.3; 200 x 1024 -> 4096 11.8 10.2 10.6; 375 x 2048 -> 1024 17.8 12.6 10.2; 750 x
+// 3072 -> 1024 27.1 22.0 20.1; 28 x 2048 -> 1024 17.3 11.8 7.2. SwiGLU tiles hold
+// the gate and up rows of 32 outputs (a prefill of all layers, ms: 750 rows 5.49
+// 5.61 5.75, 300 rows 2.94 3.04 3.03, 203 rows 2.51 2.45 2.52, 28 rows 1.96 1.88
+// 1.82; the third a 32 x 64 tile with stages of eight).
 template <class Scale, int OUT>
 static hipError_t launch_gemm_out(const GemmArgs& g, hipStream_t s) {
-  const long rows = (long)g.rows * (OUT == kGemmSwiGLU ? 2 : 1);
-  auto waves = [&](int tr, int tf) { return ((rows + 16 * tr - 1) / (16 * tr)) * ((g.frames + 16 * tf - 1) / (16 * tf)); };
-  constexpr long kWant = 2048;
-  if (waves(2, 2) >= kWant) return launch_gemm_tiles<Scale, OUT, 2, 2>(g, s);
-  // A quantised SwiGLU output needs 32-row tiles (one Q8_0 block a frame).
-  if (waves(2, 1) >= kWant || (OUT == kGemmSwiGLU && g.out_q)) return launch_gemm_tiles<Scale, OUT, 2, 1>(g, s);
-  return launch_gemm_tiles<Scale, OUT, 1, 1>(g, s);
+  const auto tiles = [&](int frames, int rows) { return ((g.frames + frames - 1) / frames) * ((g.rows + rows - 1) / rows); };
+  if constexpr (OUT == kGemmSwiGLU) {
+    if (tiles(64, 32) >= 480) return launch_gemm_tiles<Scale, OUT, 2, 2, 2, 2, 4>(g, s);
+    if (tiles(32, 32) >= 448) return launch_gemm_tiles<Scale, OUT, 2, 2, 1, 2, 4>(g, s);
+    return launch_gemm_tiles<Scale, OUT, 2, 2, 1, 2, 8>(g, s);
+  } else {
+    if (tiles(64, 64) >= 512) return launch_gemm_tiles<Scale, OUT, 2, 2, 2, 2, 4>(g, s);
+    if (tiles(32, 64) >= 448) return launch_gemm_tiles<Scale, OUT, 2, 2, 1, 2, 4>(g, s);
+    return launch_gemm_tiles<Scale, OUT, 2, 2, 1, 1, 8>(g, s);
+  }
 }
 
 template <class Scale>

@@ -1,0 +1,46 @@
+"""The Q8_0 GEMM's tiles and their edges, bit for bit against the oracle, with
+every kind of block scale: fp16 (the term's product from the MFMA's biased
+result), fp32 (converted dots), and fp16 ones that are infinite or NaN."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def backend():
+    from funasrnet_amd.hip import HipBackend
+    b = HipBackend(0, minimum_operations=0)
+    yield b
+    b.close()
+
+
+def scales(rng, kind, rows, blocks):
+    s = (rng.standard_normal((rows, blocks)) * 0.02).astype(np.float16)
+    s[rng.random(s.shape) < 0.05] = 0
+    s[0, 0], s[-1, -1] = np.float16(65504), np.float16(6e-8)
+    if kind == "odd":
+        s[rows // 2, blocks // 2], s[rows // 3, 0] = np.inf, np.nan
+    s = s.astype(np.float32)
+    return s * np.float32(1.0001) if kind == "fp32" else s
+
+
+# Tiles of 32 x 32, 32 x 64 from 448 of them on, 64 x 64 from 512 on; stages of
+# eight blocks with four left over (K = 128, 384, 640).
+@pytest.mark.parametrize("frames,cols,rows", [(4, 128, 1), (31, 384, 33), (33, 640, 31), (65, 1024, 65), (225, 256, 3969),
+                                              (449, 384, 2047), (513, 128, 4033), (1023, 640, 2049)])
+@pytest.mark.parametrize("kind", ["fp16", "fp32", "odd"])
+def test_tiles(backend, oracle_lib, frames, cols, rows, kind):
+    from funasrnet_amd.model import Q8Tensor
+    rng = np.random.default_rng(frames + cols)
+    x = rng.standard_normal((frames, cols)).astype(np.float32)
+    x[0] = 0
+    q = rng.integers(-128, 128, (rows, cols), dtype=np.int8)
+    s = scales(rng, kind, rows, cols // 32)
+    bias = rng.standard_normal(rows).astype(np.float32)
+    out = np.empty(frames * rows, np.float32)
+    assert backend.try_quantized_linear(x.ravel(), frames, Q8Tensor("w", q, s), bias, out)
+    got, expected = out.reshape(frames, rows), oracle_lib.linear(x.ravel(), q, s, bias).reshape(frames, rows)
+    nan = np.isnan(expected)
+    assert np.array_equal(np.isnan(got), nan)
+    assert np.array_equal(got[~nan].view(np.uint32), expected[~nan].view(np.uint32))
