@@ -442,76 +442,87 @@ __global__ __launch_bounds__(64 * WN * KS) void f32_split_gemm_kernel(
 }
 
 // ---- GEMV (few frames, weight-bandwidth bound) ------------------------------
-// Each wave takes RW consecutive weight rows at a time (their loads all in
-// flight together), every lane a strided share of each row (four floats per
-// lane per step when rows are 16-byte aligned), the frames' inputs in LDS,
-// then a wave reduction per row and frame.
-constexpr int kVMaxFrames = 4, kVMaxK = 4096;
-
-template <bool RELU, bool VEC, int kVRows>
+// Each wave takes RW consecutive weight rows at a time, in chunks of 1,024 k
+// whose loads (16 values a lane and row) are all in flight together, with the
+// frames' values at the same k straight from the caches: a small launch is one
+// round of loads, with no LDS and no barrier before it (the frames staged in LDS
+// first, and 256 k a round: one frame of 1024 -> 3072 6.5 us, here 3.9, of 3072
+// -> 1024 9.1 and 3.8, both at what a call costs the host; 1024 -> 151936 113 and
+// 106, 5.9 TB/s). Then a wave reduction per row and frame. VEC: 16-byte loads (K
+// % 4 == 0, aligned rows).
+template <int MF, int RW, bool VEC>
 __global__ __launch_bounds__(256) void f32_gemv_kernel(const float* __restrict__ x, const float* __restrict__ w,
                                                        const float* __restrict__ bias, float* __restrict__ out, int M,
-                                                       int N, int K) {
-  __shared__ __attribute__((aligned(16))) float x_s[kVMaxFrames * kVMaxK];
-  const int tid = threadIdx.x, lane = tid & 63;
-  for (int i = tid; i < M * K; i += 256) x_s[i] = x[i];
-  __syncthreads();
-  const int waves = gridDim.x * 4;
-  for (int n0 = (blockIdx.x * 4 + (tid >> 6)) * kVRows; n0 < N; n0 += waves * kVRows) {
-    float acc[kVRows][kVMaxFrames];
-#pragma unroll
-    for (int r = 0; r < kVRows; ++r)
-#pragma unroll
-      for (int f = 0; f < kVMaxFrames; ++f) acc[r][f] = 0.0f;
-    // Rows past N re-read row N - 1 (never stored).
-    const float* rows[kVRows];
-#pragma unroll
-    for (int r = 0; r < kVRows; ++r) rows[r] = w + (size_t)min(n0 + r, N - 1) * K;
+                                                       int N, int K, int relu) {
+  constexpr int kChunk = 1024, E = kChunk / 64;
+  const int lane = threadIdx.x & 63, waves = gridDim.x * 4;
+  // Value e of this lane: k0 + at(e); with `all`, the whole chunk lies in the row.
+  auto load = [&](const float* row, int k0, bool all, float* v) {
     if (VEC) {
-      for (int k = 4 * lane; k < K; k += 256) {
-        float4 v[kVRows];
 #pragma unroll
-        for (int r = 0; r < kVRows; ++r) v[r] = *reinterpret_cast<const float4*>(rows[r] + k);
-#pragma unroll
-        for (int f = 0; f < kVMaxFrames; ++f)
-          if (f < M) {
-            const float4 u = *reinterpret_cast<const float4*>(x_s + f * K + k);
-#pragma unroll
-            for (int r = 0; r < kVRows; ++r) {
-              acc[r][f] = __builtin_fmaf(v[r].x, u.x, acc[r][f]);
-              acc[r][f] = __builtin_fmaf(v[r].y, u.y, acc[r][f]);
-              acc[r][f] = __builtin_fmaf(v[r].z, u.z, acc[r][f]);
-              acc[r][f] = __builtin_fmaf(v[r].w, u.w, acc[r][f]);
-            }
-          }
+      for (int e = 0; e < E; e += 4) {
+        const int k = k0 + 64 * e + 4 * lane;
+        const float4 q = all || k < K ? *reinterpret_cast<const float4*>(row + k) : make_float4(0.f, 0.f, 0.f, 0.f);
+        v[e] = q.x;
+        v[e + 1] = q.y;
+        v[e + 2] = q.z;
+        v[e + 3] = q.w;
       }
     } else {
-      for (int k = lane; k < K; k += 64) {
-        float v[kVRows];
 #pragma unroll
-        for (int r = 0; r < kVRows; ++r) v[r] = rows[r][k];
-#pragma unroll
-        for (int f = 0; f < kVMaxFrames; ++f)
-          if (f < M) {
-            const float u = x_s[f * K + k];
-#pragma unroll
-            for (int r = 0; r < kVRows; ++r) acc[r][f] = __builtin_fmaf(v[r], u, acc[r][f]);
-          }
+      for (int e = 0; e < E; ++e) {
+        const int k = k0 + 64 * e + lane;
+        v[e] = all || k < K ? row[k] : 0.0f;
       }
     }
+  };
+  for (int n0 = (blockIdx.x * 4 + (threadIdx.x >> 6)) * RW; n0 < N; n0 += waves * RW) {
+    float acc[RW][MF];
 #pragma unroll
-    for (int r = 0; r < kVRows; ++r) {
+    for (int r = 0; r < RW; ++r)
+#pragma unroll
+      for (int f = 0; f < MF; ++f) acc[r][f] = 0.0f;
+    // Rows past N re-read row N - 1 (never stored).
+    const float* rows[RW];
+#pragma unroll
+    for (int r = 0; r < RW; ++r) rows[r] = w + (size_t)min(n0 + r, N - 1) * K;
+    float v[RW][E];
+    auto chunk = [&](int k0, bool all) {
+#pragma unroll
+      for (int f = 0; f < MF; ++f) {
+        if (MF > 1 && f >= M) break;
+        float u[E];
+        load(x + (size_t)f * K, k0, all, u);
+#pragma unroll
+        for (int e = 0; e < E; ++e)
+#pragma unroll
+          for (int r = 0; r < RW; ++r) acc[r][f] = __builtin_fmaf(v[r][e], u[e], acc[r][f]);
+      }
+    };
+    int k0 = 0;
+    for (; k0 + kChunk <= K; k0 += kChunk) {
+#pragma unroll
+      for (int r = 0; r < RW; ++r) load(rows[r], k0, true, v[r]);
+      chunk(k0, true);
+    }
+    if (k0 < K) {
+#pragma unroll
+      for (int r = 0; r < RW; ++r) load(rows[r], k0, false, v[r]);
+      chunk(k0, false);
+    }
+#pragma unroll
+    for (int r = 0; r < RW; ++r) {
       const int n = n0 + r;
 #pragma unroll
-      for (int f = 0; f < kVMaxFrames; ++f) {
-        if (f >= M) break;
+      for (int f = 0; f < MF; ++f) {
+        if (MF > 1 && f >= M) break;
         float s = acc[r][f];
 #pragma unroll
         for (int m = 32; m >= 1; m >>= 1) s += __shfl_xor(s, m, 64);
         if (lane == 0 && n < N) {
-          float v = s + (bias ? bias[n] : 0.0f);
-          if (RELU) v = v < 0.0f ? 0.0f : v;
-          out[(size_t)f * N + n] = v;
+          float y = s + (bias ? bias[n] : 0.0f);
+          if (relu) y = y < 0.0f ? 0.0f : y;
+          out[(size_t)f * N + n] = y;
         }
       }
     }
@@ -1067,24 +1078,32 @@ hipError_t launch_f32_split(float* w, int64_t rows, int cols, hipStream_t s) {
 hipError_t launch_f32_linear(const float* x, const float* w, const float* bias, float* out, int M, int N, int K,
                              bool relu, bool splittable, hipStream_t s) {
   if (M < 1 || N < 1 || K < 1) return hipErrorInvalidValue;
-  if (M <= kVMaxFrames && K <= kVMaxK) {
-    // Four rows per wave when that still leaves 512+ workgroups, else one.
-    const bool wide = N >= 4 * 4 * 512;
-    const int per = wide ? 16 : 4;
-    const int groups = std::min((N + per - 1) / per, 2048);
-    const bool vec = K % 4 == 0;
-#define FAH_GEMV(R, V, RW) f32_gemv_kernel<R, V, RW><<<groups, 256, 0, s>>>(x, w, bias, out, M, N, K)
-    if (wide) {
-      if (relu) vec ? FAH_GEMV(true, true, 4) : FAH_GEMV(true, false, 4);
-      else vec ? FAH_GEMV(false, true, 4) : FAH_GEMV(false, false, 4);
+  const bool vec = K % 4 == 0 && reinterpret_cast<uintptr_t>(x) % 16 == 0;
+  if (M <= 4 || (M <= 8 && N <= 8192)) {
+    // One row a wave; four (fewer reads of the frames' values) only where they
+    // still leave the chip many rounds of waves. Measured, us (one row, four rows,
+    // GEMM): 1024 -> 3072, one frame 3.9 4.1 8.3; 1024 -> 151936, one 108 106 162,
+    // four 178 145 164; eight frames of 1024 -> 2048 6.2 11.2 8.6, of 1024 ->
+    // 20000 37.6 37.8 23.1; sixteen of 1024 -> 2048 9.5 31 9.0.
+#define FAH_GEMV(MF, RW)                                                                                        \
+  do {                                                                                                          \
+    const int groups = std::min((N + 4 * RW - 1) / (4 * RW), 2048);                                             \
+    if (vec) f32_gemv_kernel<MF, RW, true><<<groups, 256, 0, s>>>(x, w, bias, out, M, N, K, relu);              \
+    else f32_gemv_kernel<MF, RW, false><<<groups, 256, 0, s>>>(x, w, bias, out, M, N, K, relu);                 \
+  } while (0)
+    const bool many = N >= 65536;
+    if (M == 1) {
+      if (many) FAH_GEMV(1, 4);
+      else FAH_GEMV(1, 1);
+    } else if (M <= 4) {
+      if (many) FAH_GEMV(4, 4);
+      else FAH_GEMV(4, 1);
     } else {
-      if (relu) vec ? FAH_GEMV(true, true, 1) : FAH_GEMV(true, false, 1);
-      else vec ? FAH_GEMV(false, true, 1) : FAH_GEMV(false, false, 1);
+      FAH_GEMV(8, 1);
     }
 #undef FAH_GEMV
     return hipGetLastError();
   }
-  const bool vec = K % 4 == 0 && reinterpret_cast<uintptr_t>(x) % 16 == 0;
   const uint4* planes = reinterpret_cast<const uint4*>(reinterpret_cast<const char*>(w) + planes_offset(N, K));
   const auto tiles = [&](int tm, int tn) { return ((M + tm - 1) / tm) * ((N + tn - 1) / tn); };
   const auto run = [&](auto aligned, auto unaligned, int grid, int threads) {

@@ -259,7 +259,7 @@ const int* f32_weight_outside(const float* w, int64_t rows, int cols);
 hipError_t launch_f32_split(float* w, int64_t rows, int cols, hipStream_t s);
 // FP32 projections y[M][N] = x[M][K] W[N][K]^T (+ bias) (ReLU): products of
 // bf16 planes on MFMA (fp32 MFMA for a weight that is not splittable), or a
-// GEMV for up to 4 frames of at most 4096 columns.
+// GEMV for up to 4 frames (8 of up to 8192 rows).
 hipError_t launch_f32_linear(const float* x, const float* w, const float* bias, float* out, int M, int N, int K,
                              bool relu, bool splittable, hipStream_t s);
 // Non-causal multi-head attention over [frames][width] rows (head size

@@ -175,7 +175,7 @@ int fah_quantized_linear_noalloc(fah_context* context, const float* input, int f
  * reference device version src/FunAsrNet.Vulkan/VulkanFloatBackend.cs:127-171):
  * output[frames*rows] = input[frames*cols] W^T (+ bias) for an FP32 weight,
  * on the matrix cores with fp32 sums (each value split exactly into three bf16
- * planes), or a bandwidth-bound GEMV for up to 4 frames. Declines
+ * planes), or a bandwidth-bound GEMV for up to 4 frames (8 of up to 8192 rows). Declines
  * (output untouched) Q8_0 weights and projections below the minimum
  * operations. Float order differs from the CPU kernels, as the reference's
  * own device path does (its check: 2e-4 x max(1, |expected|)). The encoder's

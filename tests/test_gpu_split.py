@@ -43,6 +43,19 @@ def test_split_tiles(backend, frames, cols, rows, biased):
     check(run(backend, x, w, b), x, w, b)
 
 
+# The GEMV of one, up to four and up to eight frames: parts of a chunk of 1,024 k,
+# aligned and not, and the row counts where four rows a wave and the GEMM begin.
+@pytest.mark.parametrize("frames,cols,rows", [(1, 1, 1), (1, 63, 5), (1, 1023, 9), (1, 1028, 65537), (2, 4, 3),
+                                              (3, 1025, 70), (4, 2052, 65541), (5, 1024, 6), (7, 67, 8192), (8, 5000, 33),
+                                              (8, 64, 8193), (1, 6148, 11)])
+def test_gemv(backend, frames, cols, rows):
+    rng = np.random.default_rng(cols)
+    x = rng.standard_normal((frames, cols)).astype(np.float32)
+    w = rng.standard_normal((rows, cols)).astype(np.float32)
+    b = rng.standard_normal(rows).astype(np.float32)
+    check(run(backend, x, w, b), x, w, b)
+
+
 @pytest.mark.parametrize("frames,rows", [(40, 70), (400, 700), (1100, 2100)])
 def test_split_range(backend, frames, rows):
     """Zero frames, tiny and huge values, infinities and NaN."""
