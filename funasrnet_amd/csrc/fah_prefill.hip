@@ -61,7 +61,7 @@ __device__ __forceinline__ int gate_up_row(int r, int kind, int base, int extra)
 // -1.5 2^23 w_scale (exact: w_scale has 11 bits), fma(result, w_scale, c) is
 // dot w_scale rounded once, what (float)dot * w_scale is, without the
 // conversion. (fp32 scales keep the conversion: c would round. An infinite
-// scale makes c infinite: sums that are not finite are formed again by
+// scale makes c infinite: the sums of such rows are formed again by
 // row_reference.) Rows and scales move through LDS in stages of SB blocks, one
 // stage in use, one being filled, two in registers or on their way; rows are
 // padded so that the 16 rows of an operand read fall on distinct banks, and
@@ -289,19 +289,23 @@ __global__ __launch_bounds__(64 * WF * WR) void q8_gemm_kernel(GemmArgs g) {
     for (int j = 0; j < TJ; ++j)
 #pragma unroll
       for (int e = 0; e < 4; ++e) odd = odd || (f2u(acc[i][j][e]) & 0x7fffffffu) >= 0x7f800000u;
+  // (Inputs that are infinite or NaN give what they give in any form.)
   if (kHalf && __any(odd)) {
 #pragma unroll
-    for (int i = 0; i < TI; ++i)
+    for (int j = 0; j < TJ; ++j) {
+      const int sr = storage_row(16 * (TJ * wr + j) + l16);
+      const ST* ws = reinterpret_cast<const ST*>(g.ws) + (size_t)sr * B;
+      bool infinite = false;
+      for (int b = 0; b < B; ++b) infinite = infinite || __builtin_isinf(Scale::get(ws[b]));
+      if (!infinite) continue;
 #pragma unroll
-      for (int j = 0; j < TJ; ++j)
+      for (int i = 0; i < TI; ++i)
 #pragma unroll
-        for (int e = 0; e < 4; ++e)
-          if ((f2u(acc[i][j][e]) & 0x7fffffffu) >= 0x7f800000u) {
-            const int f = min(fw + 16 * i + 4 * kq + e, g.frames - 1);
-            const int sr = storage_row(16 * (TJ * wr + j) + l16);
-            acc[i][j][e] = row_reference<Scale>(g.w + (size_t)sr * g.K, reinterpret_cast<const ST*>(g.ws) + (size_t)sr * B,
-                                                g.xq + (size_t)f * g.K, g.xs + (size_t)f * B, B);
-          }
+        for (int e = 0; e < 4; ++e) {
+          const int f = min(fw + 16 * i + 4 * kq + e, g.frames - 1);
+          acc[i][j][e] = row_reference<Scale>(g.w + (size_t)sr * g.K, ws, g.xq + (size_t)f * g.K, g.xs + (size_t)f * B, B);
+        }
+    }
   }
 
   if (!kSwiGLU) {

@@ -35,6 +35,8 @@ def test_tiles(backend, oracle_lib, frames, cols, rows, kind):
     rng = np.random.default_rng(frames + cols)
     x = rng.standard_normal((frames, cols)).astype(np.float32)
     x[0] = 0
+    if kind == "odd":
+        x[1, 3], x[2, 0] = np.nan, np.inf
     q = rng.integers(-128, 128, (rows, cols), dtype=np.int8)
     s = scales(rng, kind, rows, cols // 32)
     bias = rng.standard_normal(rows).astype(np.float32)
