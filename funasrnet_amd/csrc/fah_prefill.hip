@@ -996,22 +996,30 @@ __global__ __launch_bounds__(kRowThreads) __attribute__((amdgpu_waves_per_eu(2))
   char* ring = reinterpret_cast<char*>(rows_s + (size_t)kRowPairs * PS);
   const _Float16* kc = a.kcache + (size_t)kh * a.capacity * hs;
   const _Float16* vc = a.vcache + (size_t)kh * a.capacity * hs;
-  for (int i = tid; i < kRowPairs * hs; i += kRowThreads) {
+  // The first pass's K rows are on their way while q goes to LDS.
+  const int mp = lane & 15, mg = lane >> 4;
+  uint4 kk[16];
+  auto load_k = [&](int t0) {
+    const uint4* row = reinterpret_cast<const uint4*>(kc + (size_t)min(t0 + lane, nmax - 1) * hs);
+#pragma unroll
+    for (int i = 0; i < 16; ++i) kk[i] = row[i];
+  };
+  if (64 * wave < nmax) load_k(64 * wave);
+#pragma unroll
+  for (int i = 4 * tid; i < kRowPairs * hs; i += 4 * kRowThreads) {
     const int pi = i >> 7, c = i & 127, hh = pi >> 3, rr = pi & 7;
-    q_s[pi * kQRow + c] = rr < rows ? a.q[((size_t)(r0 + rr) * a.heads + 2 * kh + hh) * hs + c] : 0.0f;
+    *reinterpret_cast<float4*>(q_s + pi * kQRow + c) =
+        rr < rows ? *reinterpret_cast<const float4*>(a.q + ((size_t)(r0 + rr) * a.heads + 2 * kh + hh) * hs + c)
+                  : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
   }
-  __syncthreads();
+  lds_barrier();
 
   // 1. Scores, 64 positions per wave pass: lane l loads position t0 + l's K
   // row; per channel one outer product with the pairs' q (pair l % 16's q
   // from LDS), its 16 products added to the channel's accumulator (c % 8) of
   // each (pair, position) the lane holds.
-  const int mp = lane & 15, mg = lane >> 4;
   for (int t0 = 64 * wave; t0 < nmax; t0 += kRowThreads) {
-    const uint4* row = reinterpret_cast<const uint4*>(kc + (size_t)min(t0 + lane, nmax - 1) * hs);
-    uint4 kk[16];
-#pragma unroll
-    for (int i = 0; i < 16; ++i) kk[i] = row[i];
+    if (t0 >= kRowThreads) load_k(t0);
     const float* qrow = q_s + mp * kQRow;
     // Two passes over the row, each with four of the eight accumulators:
     // channels 8i + {0, 1, 4, 5}, then 8i + {2, 3, 6, 7}; the tree
@@ -1074,8 +1082,23 @@ __global__ __launch_bounds__(kRowThreads) __attribute__((amdgpu_waves_per_eu(2))
       *reinterpret_cast<float4*>(prow + 16 * b) = make_float4(sc[0], sc[1], sc[2], sc[3]);
     }
   }
-  __syncthreads();
+  lds_barrier();
 
+  // The first V chunks, in flight during the softmax.
+  constexpr int kGroups = 512 / kRowThreads, kAhead = 4;
+  const int chunks = (nmax + kVRing - 1) / kVRing;
+  struct Chunk {
+    v4i piece[kGroups];
+  } ahead[kAhead];
+  auto fetch = [&](Chunk& v, int j) {  // rows past the last are read again, unused
+#pragma unroll
+    for (int m = 0; m < kGroups; ++m) {
+      const int piece = tid + kRowThreads * m, row = min(j * kVRing + (piece >> 4), nmax - 1);
+      v.piece[m] = *reinterpret_cast<const v4i*>(reinterpret_cast<const char*>(vc) + (size_t)row * 256 + 16 * (piece & 15));
+    }
+  };
+#pragma unroll
+  for (int u = 0; u < kAhead; ++u) fetch(ahead[u], u);
   // 2. Softmax: kLanes lanes per pair.
   constexpr int kLanes = kRowThreads / kRowPairs;
   const int pi = tid / kLanes, sub = tid % kLanes;
@@ -1088,7 +1111,7 @@ __global__ __launch_bounds__(kRowThreads) __attribute__((amdgpu_waves_per_eu(2))
     if (kLanes == 32) m = nan_max_p(m, __shfl_xor(m, 16, 64));
     for (int t = sub; t < n; t += kLanes) pp[t] = exp_ref(fadd(pp[t], -m));
   }
-  __syncthreads();
+  lds_barrier();
   const int full = n & ~7;
   if (sub < 8) {
     // Lane j of the pair: p[j] + p[j+8] + ... in order, in double.
@@ -1104,48 +1127,74 @@ __global__ __launch_bounds__(kRowThreads) __attribute__((amdgpu_waves_per_eu(2))
     for (; t < full; t += 8) l = l + (double)pp[t];
     lane_s[pi * 8 + sub] = l;
   }
-  __syncthreads();
+  lds_barrier();
   if (sub == 0 && n > 0) {
     const double* L = lane_s + pi * 8;
     double sum = ((L[0] + L[4]) + (L[1] + L[5])) + ((L[2] + L[6]) + (L[3] + L[7]));
     for (int t = full; t < n; ++t) sum = sum + (double)pp[t];
     inv_s[pi] = (float)(1.0 / sum);
   }
-  __syncthreads();
+  lds_barrier();
   {
     const float inverse = n > 0 ? inv_s[pi] : 0.0f;
     for (int t = sub; t < n; t += kLanes) pp[t] = fmul(pp[t], inverse);
   }
 
   // 3. Time-ordered value sums, all waves: wave w owns kGroups groups of 16
-  // channels from 16 kGroups w on. One outer product covers four positions t .. t + 3
-  // (one per 16 x 16 block: the 16 pairs' probabilities at t + b times 16
-  // channels' v at t + b), so lane l holds, for a channel and
-  // pairs 4 (l / 16) + r, the products of four consecutive positions and
-  // adds them in order. V rows pass through a
-  // two-slot LDS ring (direct global->LDS loads of 16-byte pieces, the next
-  // chunk's issued before this one is added; a slot is refilled only after
-  // the barrier that follows its last use).
-  constexpr int kGroups = 512 / kRowThreads;
-  const int chunks = (nmax + kVRing - 1) / kVRing;
-  auto fill = [&](int j) {  // rows past the last are read again, unused
+  // channels from 16 kGroups w on. One outer product covers four positions
+  // t .. t + 3 (one per 16 x 16 block: the 16 pairs' probabilities at t + b
+  // times 16 channels' v at t + b), so lane l holds, for a channel and pairs
+  // 4 (l / 16) + r, the products of four consecutive positions and adds them
+  // in order. V rows pass through a two-slot LDS ring, chunks of 32 rows, of
+  // which the next kAhead are in registers or on their way (with one, by direct
+  // loads, a chunk's chains were shorter than the loads' latency). Bound by the
+  // adds' and products' issue; prefill of 375, 500 and 750 rows 3.35 -> 3.26,
+  // 3.91 -> 3.74, 5.51 -> 5.36 ms with the V rows ahead and the products formed a
+  // step before their adds.
+  auto put = [&](const Chunk& v, int j) {
 #pragma unroll
-    for (int m = 0; m < kGroups; ++m) {
-      const int piece = tid + kRowThreads * m, row = min(j * kVRing + (piece >> 4), nmax - 1);
-      const char* src = reinterpret_cast<const char*>(vc) + (size_t)row * 256 + 16 * (piece & 15);
-      __builtin_amdgcn_global_load_lds(src, (lds_ptr)(ring + (size_t)(j & 1) * kVRing * 256 + kRowThreads * 16 * m + 1024 * wave),
-                                       16, 0, 0);
-    }
+    for (int m = 0; m < kGroups; ++m)
+      *reinterpret_cast<v4i*>(ring + (size_t)(j & 1) * kVRing * 256 + 16 * (tid + kRowThreads * m)) = v.piece[m];
   };
-  fill(0);
-  __builtin_amdgcn_s_waitcnt(0);
-  __syncthreads();  // the normalised probabilities and the first V chunk
+  put(ahead[0], 0);
+  fetch(ahead[0], kAhead);
+  lds_barrier();  // the normalised probabilities and the first V chunk
   float acc[kGroups][4] = {};
   const float* pa = p_s + (size_t)mp * PS + mg;  // A operand: pair mp at position t + l / 16
-  for (int j = 0; j < chunks; ++j) {
-    if (j + 1 < chunks) fill(j + 1);
+  auto add = [&](int j) {
     const _Float16* vr = reinterpret_cast<const _Float16*>(ring + (size_t)(j & 1) * kVRing * 256) + mg * hs + 16 * kGroups * wave + mp;
     const int t0 = j * kVRing, len = min(kVRing, nmax - t0);
+    if (t0 + kVRing <= n0) {
+      // Every row of the block sees the whole chunk: operands read first, each
+      // product formed while the one before it is added.
+      constexpr int kSteps = kVRing / 4;
+      float av[kSteps], bv[kSteps][kGroups];
+#pragma unroll
+      for (int s = 0; s < kSteps; ++s) {
+        av[s] = pa[t0 + 4 * s];
+#pragma unroll
+        for (int h = 0; h < kGroups; ++h) bv[s][h] = (float)vr[4 * s * hs + 16 * h];
+      }
+      f32x16 d[2][kGroups];
+#pragma unroll
+      for (int h = 0; h < kGroups; ++h) d[0][h] = outer16(av[0], bv[0][h]);
+#pragma unroll
+      for (int s = 0; s < kSteps; ++s) {
+        if (s + 1 < kSteps) {
+#pragma unroll
+          for (int h = 0; h < kGroups; ++h) d[(s + 1) & 1][h] = outer16(av[s + 1], bv[s + 1][h]);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int b = 0; b < 4; ++b)
+#pragma unroll
+          for (int r = 0; r < 4; ++r)
+#pragma unroll
+            for (int h = 0; h < kGroups; ++h) acc[h][r] = fadd(acc[h][r], d[s & 1][h][4 * b + r]);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      return;
+    }
     for (int s = 0; s < len; s += 4) {
       const int t = t0 + s;
       const float av = pa[t];
@@ -1172,8 +1221,16 @@ __global__ __launch_bounds__(kRowThreads) __attribute__((amdgpu_waves_per_eu(2))
           }
       }
     }
-    __builtin_amdgcn_s_waitcnt(0);
-    __syncthreads();
+  };
+  for (int j0 = 0; j0 < chunks; j0 += kAhead) {
+#pragma unroll
+    for (int u = 0; u < kAhead; ++u) {
+      const int j = j0 + u;
+      put(ahead[(u + 1) % kAhead], j + 1);
+      fetch(ahead[(u + 1) % kAhead], j + 1 + kAhead);
+      if (j < chunks) add(j);
+      lds_barrier();
+    }
   }
 
   // 4. Output rows (float and/or Q8_0 blocks): pair 4 mg + r, channel
@@ -1187,7 +1244,7 @@ __global__ __launch_bounds__(kRowThreads) __attribute__((amdgpu_waves_per_eu(2))
       if (a.out && rr < rows) a.out[((size_t)(r0 + rr) * a.heads + 2 * kh + (pq >> 3)) * hs + c] = acc[h][r];
     }
   if (a.xq) {
-    __syncthreads();
+    lds_barrier();
 #pragma unroll
     for (int g0 = 0; g0 < kRowPairs * hs / 4; g0 += kRowThreads) {
       const int g = g0 + tid, pq = g >> 5, c4 = (g & 31) * 4, rr = pq & 7;
