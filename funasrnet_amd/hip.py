@@ -147,6 +147,23 @@ def _p(a: np.ndarray, ctype):
     return a.ctypes.data_as(ctypes.POINTER(ctype))
 
 
+class _Output:
+    """The result buffer of a seam call: the caller's array itself where the
+    library can write it (float32, C-contiguous, writeable), else one to copy
+    back. Declined calls leave the array as it is either way."""
+
+    def __init__(self, output: np.ndarray):
+        self.output = output
+        direct = output.dtype == np.float32 and output.flags.c_contiguous and output.flags.writeable
+        self.array = output if direct else np.empty(output.size, dtype=np.float32)
+        self.pointer = _p(self.array, ctypes.c_float)
+
+    def accept(self) -> bool:
+        if self.array is not self.output:
+            self.output.reshape(-1)[:] = self.array
+        return True
+
+
 def _raise(rc: int):
     msg = load().fah_last_error().decode()
     if rc == ERROR_ARGUMENT:
@@ -301,13 +318,12 @@ class HipBackend:
         x = np.ascontiguousarray(input, dtype=np.float32)
         if x.size != frames * w.columns or output.size != frames * w.rows:
             raise ValueError("GPU linear projection shape mismatch")
-        out = np.empty(frames * w.rows, dtype=np.float32)
+        out = _Output(output)
         b = None if bias is None else _p(np.ascontiguousarray(bias, dtype=np.float32), ctypes.c_float)
-        rc = _check(load().fah_linear(self.handle, _p(x, ctypes.c_float), frames, w.handle, b, _p(out, ctypes.c_float)))
+        rc = _check(load().fah_linear(self.handle, _p(x, ctypes.c_float), frames, w.handle, b, out.pointer))
         if rc == DECLINED:
             return False
-        output.reshape(-1)[:] = out
-        return True
+        return out.accept()
 
     def try_relu_projection(self, input: np.ndarray, frames: int, first: np.ndarray, first_bias, second: np.ndarray,
                             second_bias, output: np.ndarray) -> bool:
@@ -316,15 +332,14 @@ class HipBackend:
         x = np.ascontiguousarray(input, dtype=np.float32)
         if x.size != frames * w1.columns or output.size != frames * w2.rows:
             raise ValueError("ReLU projection input, weight or output shape mismatch")
-        out = np.empty(frames * w2.rows, dtype=np.float32)
+        out = _Output(output)
         b1 = None if first_bias is None else _p(np.ascontiguousarray(first_bias, dtype=np.float32), ctypes.c_float)
         b2 = None if second_bias is None else _p(np.ascontiguousarray(second_bias, dtype=np.float32), ctypes.c_float)
         rc = _check(load().fah_relu_projection(self.handle, _p(x, ctypes.c_float), frames, w1.handle, b1, w2.handle, b2,
-                                               _p(out, ctypes.c_float)))
+                                               out.pointer))
         if rc == DECLINED:
             return False
-        output.reshape(-1)[:] = out
-        return True
+        return out.accept()
 
     def try_attention(self, query: np.ndarray, key: np.ndarray, value: np.ndarray, frames: int, width: int,
                       heads: int, output: np.ndarray) -> bool:
@@ -337,27 +352,25 @@ class HipBackend:
             return False
         if q.size != count or k.size != count or v.size != count or output.size != count:
             raise ValueError("GPU attention input/output shapes differ")
-        out = np.empty(count, dtype=np.float32)
+        out = _Output(output)
         rc = _check(load().fah_attention(self.handle, _p(q, ctypes.c_float), _p(k, ctypes.c_float),
-                                         _p(v, ctypes.c_float), frames, width, heads, _p(out, ctypes.c_float)))
+                                         _p(v, ctypes.c_float), frames, width, heads, out.pointer))
         if rc == DECLINED:
             return False
-        output.reshape(-1)[:] = out
-        return True
+        return out.accept()
 
     def try_quantized_linear(self, input: np.ndarray, frames: int, weight: Q8Tensor, bias, output: np.ndarray) -> bool:
         w = self.weight(weight)
         x = np.ascontiguousarray(input, dtype=np.float32)
         if x.size != frames * w.columns or output.size != frames * w.rows:
             raise ValueError("Q8 GPU projection shape mismatch")
-        out = np.empty(frames * w.rows, dtype=np.float32)
+        out = _Output(output)
         b = None if bias is None else _p(np.ascontiguousarray(bias, dtype=np.float32), ctypes.c_float)
         rc = _check(load().fah_quantized_linear(self.handle, _p(x, ctypes.c_float), frames, w.handle, b,
-                                                _p(out, ctypes.c_float)))
+                                                out.pointer))
         if rc == DECLINED:
             return False
-        output.reshape(-1)[:] = out
-        return True
+        return out.accept()
 
     def try_linear_many(self, input: np.ndarray, frames: int, weights: list):
         """IGroupedComputeBackend.TryLinearMany over Q8_0 tensors or FP32 arrays."""

@@ -135,3 +135,17 @@ def test_split_attention_range(backend, oracle_lib, value):
     v[7, size + 5] = 1.0
     again = attend(backend, q, k, v, heads)
     assert np.all(np.isfinite(again)) and np.array_equal(again, attend(backend, q, k, v, heads))
+
+
+def test_output_arrays(backend):
+    """Results land in the caller's array, also one that the library cannot write."""
+    rng = np.random.default_rng(2)
+    x, w = rng.standard_normal((9, 40)).astype(np.float32), rng.standard_normal((6, 40)).astype(np.float32)
+    plain = run(backend, x, w)
+    wide = np.zeros((9, 6))
+    assert backend.try_linear(x, 9, w, None, wide) and np.array_equal(wide, plain)
+    every_other = np.zeros(2 * 9 * 6, np.float32)[::2]
+    assert backend.try_linear(x, 9, w, None, every_other) and np.array_equal(every_other, plain.ravel())
+    same = rng.standard_normal((6, 6)).astype(np.float32)
+    expected = run(backend, same.copy(), w[:, :6].copy())
+    assert backend.try_linear(same, 6, w[:, :6].copy(), None, same) and np.array_equal(same, expected)
