@@ -263,7 +263,7 @@ __device__ __forceinline__ float score_regs(const uint4* k, const float* q, floa
 typedef int v4i __attribute__((ext_vector_type(4)));
 
 // One wave's 16-row tile of a projection for up to 16 sessions on the matrix
-// cores, in q8_head_mfma16_kernel's operand layout: lane (r, q) = (lane % 16,
+// cores, in v_mfma_i32_16x16x32_i8's operand layout: lane (r, q) = (lane % 16,
 // lane / 16) keeps weight bytes 8q .. 8q + 7 of every block of tile row r and
 // the row's block scales; per block one v_mfma_i32_16x16x32_i8 forms the
 // exact int32 block dots of the 16 rows with 16 sessions' codes (session r

@@ -46,3 +46,25 @@ def test_tiles(backend, oracle_lib, frames, cols, rows, kind):
     nan = np.isnan(expected)
     assert np.array_equal(np.isnan(got), nan)
     assert np.array_equal(got[~nan].view(np.uint32), expected[~nan].view(np.uint32))
+
+
+# The lm_head of lock-step sessions: the few-frame kernel up to seven, the GEMM
+# from eight on; vocabularies that end inside a workgroup's 128 rows.
+@pytest.mark.parametrize("count", [7, 8, 13, 16])
+@pytest.mark.parametrize("vocab", [33, 4001])
+def test_session_heads(backend, count, vocab):
+    from funasrnet_amd import model
+    from funasrnet_amd.hip import HipDecoder
+    weights = model.synthetic(model.small_config(layers=1, vocab=vocab), seed=vocab)
+    parent = HipDecoder(backend, weights, capacity=32)
+    sessions, alone = ([parent.session(32) for _ in range(count)] for _ in range(2))
+    try:
+        for i, (a, b) in enumerate(zip(sessions, alone)):
+            x = np.random.default_rng(i).standard_normal((5, weights.config.width)).astype(np.float32)
+            a.decode(x, 5)
+            b.decode(x, 5)
+        tokens = HipDecoder.generate_sessions(sessions, 6)
+        assert np.array_equal(tokens, np.stack([d.generate(6) for d in alone]))
+    finally:
+        for d in [*sessions, *alone, parent]:
+            d.close()
