@@ -157,8 +157,8 @@ def float_gemv_sweep(backend, rotate_bytes: int = 512 << 20):
 
 def encoder_float(backend, frames: int = 1000, repeats: int = 20):
     """The encoder's FP32 operations at one 60 s segment's shape (1000
-    frames, width 512, 4 heads; FunEncoder.cs:100-300): the projections on
-    fp32 MFMA (TFLOP/s against the 157.3 TFLOP/s dense fp32 peak) and the
+    frames, width 512, 4 heads; FunEncoder.cs:100-300): the projections
+    (TFLOP/s beside the 157.3 TFLOP/s dense fp32 MFMA peak) and the
     non-causal attention, device-resident, HIP events over `repeats` runs."""
     from funasrnet_amd import device
 
