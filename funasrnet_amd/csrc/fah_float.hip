@@ -82,8 +82,9 @@ __device__ __forceinline__ uint32_t pack_bf16(float a, float b) {
   return r;
 }
 
-// Eight floats as three planes of eight bf16.
-__device__ __forceinline__ void split8(const float* v, uint4* p) {
+// Eight floats as three planes of eight bf16. `low`: what lies below each, added
+// to what the first two planes leave.
+__device__ __forceinline__ void split8(const float* v, uint4* p, const float* low = nullptr) {
   uint32_t w[3][4];
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
@@ -95,6 +96,10 @@ __device__ __forceinline__ void split8(const float* v, uint4* p) {
       if (s < 2) {
         a -= u2f(h << 16);
         b -= u2f(h & 0xffff0000u);
+      }
+      if (s == 1 && low) {
+        a += low[2 * i];
+        b += low[2 * i + 1];
       }
     }
   }
@@ -784,10 +789,13 @@ __global__ __launch_bounds__(256) void f32_attention_mfma_kernel(const float* __
 // transposed, S^T = K Q^T, so that lane l holds 16 of a block's scores of query
 // l % 32 and lane l ^ 32 the others: the softmax needs one exchange a block.
 // Exponentials of them are, as they lie, the B operand of O^T = V^T P^T in the
-// key order above, and the outputs of a lane are its query's. The running
-// maximum moves (and the sums are rescaled) only when a score exceeds it by
-// more than kSlack (in powers of two): exponentials up to 2^kSlack are as exact. The
-// waves' sums are merged in LDS, those of the key shares by
+// key order above, and the outputs of a lane are its query's. The planes of q
+// hold q log2(e) / sqrt(HS), so that scores are exponents as they are summed and
+// the running maximum is one of them: the exponent of the largest is 0 (of a
+// maximum that was scaled and rounded it would be the rounding error, past 128
+// from 2^32 on). The running maximum moves (and the sums are rescaled) only when
+// a score exceeds it by more than kSlack: exponentials up to 2^kSlack are as
+// exact. The waves' sums are merged in LDS, those of the key shares by
 // attention_merge_kernel.
 //
 // Bound by the MFMAs (16 key blocks a wave: 1.57 us a block of 3,072 MFMA
@@ -796,7 +804,7 @@ __global__ __launch_bounds__(256) void f32_attention_mfma_kernel(const float* __
 // their way; four measured 176 us where eight take 169). Measured against
 // attention_tile_f32 for all: 4096 frames of 4 x 128 569 -> 169 us, 1864 133 ->
 // 54, 1000 44 -> 32, 1100 of 8 x 96 984 -> 43 (it ran on the VALU); error against
-// 64 bits 7.2e-7 -> 4.1e-7 (4096), 5.0e-7 -> 1.8e-7 (1000).
+// 64 bits 7.2e-7 -> 4.1e-7 (4096), 5.0e-7 -> 1.7e-7 (1000).
 //
 // Values outside [2^-100, 2^60] in magnitude, but zero, set the head's word in
 // `outside` (so do infinities and NaN); its tiles run on fp32 MFMA.
@@ -854,7 +862,18 @@ __global__ __launch_bounds__(256) void attention_planes_kernel(SplitAttnArgs a) 
   }
   if (odd) a.outside[head] = a.epoch;
   uint4 p[3];
-  split8(v, p);
+  if (which == 0) {
+    float low[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const float scaled = v[e] * a.scale;
+      low[e] = __builtin_fmaf(v[e], a.scale, -scaled);
+      v[e] = scaled;
+    }
+    split8(v, p, low);
+  } else {
+    split8(v, p);
+  }
   uint4* dst = (which == 0 ? a.qp : which == 1 ? a.kp : a.vp) + ((size_t)head * (per_head >> 6) + fragment) * 192 + lane;
 #pragma unroll
   for (int s = 0; s < 3; ++s) dst[64 * s] = p[s];
@@ -942,7 +961,7 @@ __global__ __launch_bounds__(256, 1) void attention_split_kernel(SplitAttnArgs a
     }
 #pragma unroll
     for (int r = 0; r < 16; ++r) top = fmaxf(top, t[r]);
-    top = fmaxf(top, __shfl_xor(top, 32, 64)) * a.scale;
+    top = fmaxf(top, __shfl_xor(top, 32, 64));
     if (__any(top > run_m + kSlack)) {
       const float m = fmaxf(run_m, top), down = __builtin_amdgcn_exp2f(run_m - m);
       run_m = m;
@@ -961,7 +980,7 @@ __global__ __launch_bounds__(256, 1) void attention_split_kernel(SplitAttnArgs a
       float e[8];
 #pragma unroll
       for (int i = 0; i < 8; ++i) {
-        e[i] = __builtin_amdgcn_exp2f(__builtin_fmaf(t[8 * h + i], a.scale, -run_m));
+        e[i] = __builtin_amdgcn_exp2f(t[8 * h + i] - run_m);
         run_l += e[i];
       }
       uint4 w[3];

@@ -137,6 +137,30 @@ def test_split_attention_range(backend, oracle_lib, value):
     assert np.all(np.isfinite(again)) and np.array_equal(again, attend(backend, q, k, v, heads))
 
 
+@pytest.mark.parametrize("frames,heads,size", [(400, 2, 128), (1000, 4, 128), (640, 3, 64), (130, 4, 96)])
+@pytest.mark.parametrize("scale", [1e4, 1e5, 1e8, 1e16])
+def test_split_attention_large_scores(backend, frames, heads, size, scale):
+    """Queries and keys far above 1: a row whose largest score stands out by more than
+    two fp32 scores can be off ((size + 2) 2^-24 of sum |q k| each), and by 40 beyond (e^-40 of the
+    rest), is that key's value; every other row is still a mean of values."""
+    rng = np.random.default_rng(frames)
+    q, k = (rng.uniform(-scale, scale, (frames, heads * size)).astype(np.float32) for _ in range(2))
+    v = rng.uniform(-4, 4, (frames, heads * size)).astype(np.float32)
+    got = attend(backend, q, k, v, heads)
+    assert np.all(np.isfinite(got)) and np.abs(got).max() <= 4 * (1 + 2.0**-16)
+    clear = 0
+    for h in range(0, heads * size, size):
+        qh, kh = (a[:, h:h + size].astype(np.float64) for a in (q, k))
+        scores = qh @ kh.T
+        top = scores.argmax(axis=1)
+        gap = -np.diff(np.sort(scores, axis=1)[:, -2:][:, ::-1], axis=1)[:, 0]
+        error = 2 * (size + 2) * 2.0**-24 * (np.abs(qh) @ np.abs(kh).T).max(axis=1)
+        sure = gap > error + 40 * size**0.5
+        assert np.array_equal(got[sure, h:h + size], v[top[sure], h:h + size])
+        clear += sure.sum()
+    assert clear > 0.9 * frames * heads
+
+
 def test_output_arrays(backend):
     """Results land in the caller's array, also one that the library cannot write."""
     rng = np.random.default_rng(2)
