@@ -146,18 +146,22 @@ __global__ __launch_bounds__(64 * WF * WR) void q8_gemm_kernel(GemmArgs g) {
   auto fetch = [&](Pending& p, int st) {
     st = min(st, stages - 1);
     // (B is a multiple of four: only a stage of eight can reach past the last
-    // block, where frame scales of zero make terms of zero.)
+    // block, where both scales are zero and make terms of zero; the weight's own
+    // last scale could be infinite, or overflow with the dot.)
     const int k = min(32 * SB * st + 16 * (tid % CH), g.K - 16), blk = SB * st + tid % SB, b = min(blk, B - 1);
 #pragma unroll
     for (int i = 0; i < WP; ++i) p.w[i] = *reinterpret_cast<const v4i*>(wsrc[i] + k);
 #pragma unroll
     for (int i = 0; i < XP; ++i) p.x[i] = *reinterpret_cast<const v4i*>(xsrc[i] + k);
 #pragma unroll
-    for (int i = 0; i < WS; ++i) p.ws[i] = wssrc[i][b];
+    for (int i = 0; i < WS; ++i) {
+      const ST s = wssrc[i][b];
+      p.ws[i] = SB <= 4 || blk < B ? s : (ST)0;
+    }
 #pragma unroll
     for (int i = 0; i < XS; ++i) {
       const float s = xssrc[i][b];
-      p.xs[i] = blk < B ? s : 0.0f;
+      p.xs[i] = SB <= 4 || blk < B ? s : 0.0f;
     }
   };
   // Rows in LDS: for each pair of blocks [kq 4][block 2] 8-byte pieces, so that

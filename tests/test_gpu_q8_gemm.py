@@ -48,6 +48,27 @@ def test_tiles(backend, oracle_lib, frames, cols, rows, kind):
     assert np.array_equal(got[~nan].view(np.uint32), expected[~nan].view(np.uint32))
 
 
+# Last scales that are infinite or overflow with the dot, where the last stage
+# of eight blocks has four left over, and where it has none.
+@pytest.mark.parametrize("cols", [128, 256, 384, 896])
+def test_last_scales(backend, oracle_lib, cols):
+    from funasrnet_amd.model import Q8Tensor
+    rng = np.random.default_rng(cols)
+    frames, rows, blocks = 40, 70, cols // 32
+    x = rng.standard_normal((frames, cols)).astype(np.float32)
+    x[3] = 0
+    q = rng.integers(-128, 128, (rows, cols), dtype=np.int8)
+    s = (rng.random((rows, blocks)) * 0.02 + 0.001).astype(np.float32)
+    s[5, -1], s[6, -1], s[7, -1], s[8, -1], s[9, 0] = np.inf, -np.inf, 3e38, np.nan, 3e38
+    out = np.empty((frames, rows), np.float32)
+    assert backend.try_quantized_linear(x.ravel(), frames, Q8Tensor("w", q, s), None, out)
+    expected = oracle_lib.linear(x.ravel(), q, s).reshape(frames, rows)
+    nan = np.isnan(expected)
+    assert np.isinf(expected[:, 5]).sum() > frames // 2 and np.isinf(expected[:, 7]).sum() > frames // 2
+    assert np.array_equal(np.isnan(out), nan)
+    assert np.array_equal(out[~nan].view(np.uint32), expected[~nan].view(np.uint32))
+
+
 # The lm_head of lock-step sessions: the few-frame kernel up to seven, the GEMM
 # from eight on; vocabularies that end inside a workgroup's 128 rows.
 @pytest.mark.parametrize("count", [7, 8, 13, 16])
