@@ -58,13 +58,13 @@ typedef float floatx4 __attribute__((ext_vector_type(4)));
 // 1.0e-7. Of the 19.5, the MFMAs take 6.2 (at the 2.0 GHz seen), the 8 MB of
 // stores 3, the launch, first loads and epilogue the rest.
 //
-// Range: a weight is split only if its values are at most kSplitMost in
-// magnitude and no row but a zero one lies below kSplitRowLeast (checked once,
-// at upload). What bf16 planes cannot hold of a frame is then below 2^-126
-// 2^20 K in a sum. Frames with infinities, NaN or values that round past the
-// largest bf16 make sums infinite or NaN; a workgroup that finds such a sum,
-// one below kSplitLow, or zeros and frames with values below kSplitTiny, forms
-// its tile again on fp32 MFMA (tile_f32).
+// Range: a weight is split only if its values, but zeros, lie in [kSplitTiny,
+// kSplitMost] in magnitude, so that its planes hold each exactly, and no row but
+// a zero one lies below kSplitRowLeast (checked once, at upload). What bf16 planes
+// cannot hold of a frame is then below 2^-126 2^20 K in a sum. Frames with
+// infinities, NaN or values that round past the largest bf16 make sums infinite
+// or NaN; a workgroup that finds such a sum, one below kSplitLow, or zeros and
+// frames with values below kSplitTiny, forms its tile again on fp32 MFMA (tile_f32).
 constexpr uint32_t kSplitLow = 0x1c800000u;      // 2^-70
 constexpr uint32_t kSplitTiny = 0x0d800000u;     // 2^-100
 constexpr uint32_t kSplitMost = 0x49800000u;     // 2^20
@@ -136,8 +136,13 @@ __global__ __launch_bounds__(256) void f32_split_range_kernel(const float* __res
                                                               int* outside) {
   const int lane = threadIdx.x & 63;
   for (int64_t r = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6); r < rows; r += (int64_t)gridDim.x * 4) {
-    uint32_t most = 0u;
-    for (int k = lane; k < K; k += 64) most = max(most, f2u(w[r * K + k]) & 0x7fffffffu);
+    uint32_t most = 0u, least = 0xffffffffu;  // magnitudes; magnitudes less one (zero wraps)
+    for (int k = lane; k < K; k += 64) {
+      const uint32_t m = f2u(w[r * K + k]) & 0x7fffffffu;
+      most = max(most, m);
+      least = min(least, m - 1u);
+    }
+    if (least < kSplitTiny - 1u) *outside = 1;
 #pragma unroll
     for (int m = 32; m >= 1; m >>= 1) most = max(most, (uint32_t)__shfl_xor((int)most, m, 64));
     if (lane == 0 && (most > kSplitMost || (most != 0u && most < kSplitRowLeast))) *outside = 1;

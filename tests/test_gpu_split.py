@@ -93,6 +93,19 @@ def test_weights_outside_the_planes(backend, value):
         assert not np.any(np.isfinite(got[:, 4]))
 
 
+@pytest.mark.parametrize("value,partner", [(2.0**-135, 2.0**80), (2.0**-125, 2.0**100), (2.0**-118, 2.0**60)])
+def test_tiny_weight_beside_ordinary_ones(backend, value, partner):
+    """An element that the planes do not hold, in a row of ordinary ones, against
+    frames that are large there and zero elsewhere."""
+    rng = np.random.default_rng(4)
+    x = rng.standard_normal((70, 100)).astype(np.float32)
+    w = rng.standard_normal((130, 100)).astype(np.float32)
+    w[9, 6] = np.float32(value * 1.2345678)
+    x[[3, 40]] = 0
+    x[[3, 40], 6] = np.float32(partner)
+    check(run(backend, x, w), x, w)
+
+
 def attend(backend, q, k, v, heads):
     out = np.full(q.shape, np.nan, np.float32)
     assert backend.try_attention(q, k, v, q.shape[0], q.shape[1], heads, out.reshape(-1))
