@@ -1306,6 +1306,19 @@ hipError_t launch_norm_quantize_rows(const float* x, int frames, int K, const fl
   return hipGetLastError();
 }
 
+constexpr size_t kStageLds = 150 * 1024;  // most dynamic LDS of the attention kernels
+
+// (A template, so that each kernel has its own LDS limit raised.)
+template <int kRowThreads>
+static hipError_t launch_attn_rows(const PrefillAttnArgs& a, int positions, hipStream_t s) {
+  static const hipError_t raised = hipFuncSetAttribute(reinterpret_cast<const void*>(attn_rows_kernel<kRowThreads>),
+                                                       hipFuncAttributeMaxDynamicSharedMemorySize, (int)kStageLds);
+  if (raised != hipSuccess) return raised;
+  attn_rows_kernel<kRowThreads><<<dim3(a.kv_heads, (a.frames + kRowBlock - 1) / kRowBlock), kRowThreads,
+                                  rows_lds_bytes(positions), s>>>(a);
+  return hipGetLastError();
+}
+
 hipError_t launch_attn_prefill(const PrefillAttnArgs& args, hipStream_t s) {
   PrefillAttnArgs a = args;
   if (a.head_size != 128 || a.frames < 1 || a.heads % a.kv_heads != 0) return hipErrorInvalidValue;
@@ -1316,7 +1329,6 @@ hipError_t launch_attn_prefill(const PrefillAttnArgs& args, hipStream_t s) {
   if ((!a.sessions && n > a.capacity) || n < 1 || (size_t)n * 4 > 60 * 1024) return hipErrorInvalidValue;
   // V rows are staged in LDS when that keeps three workgroups per CU, or,
   // for grids of at most two workgroups per CU, up to kStageLds.
-  constexpr size_t kStageLds = 150 * 1024;
   const size_t staged = (((size_t)4 * n + 15) & ~(size_t)15) + (size_t)n * 256;
   const bool small_grid = (size_t)a.heads * a.frames <= 512;
   a.stage = staged <= 48 * 1024 || (small_grid && staged <= kStageLds) ? n : 0;
@@ -1325,20 +1337,12 @@ hipError_t launch_attn_prefill(const PrefillAttnArgs& args, hipStream_t s) {
   if (raised != hipSuccess) return raised;
   // Many rows of one cache (a prefill): blocks of rows share K/V reads.
   if (!a.sessions && a.heads == 2 * a.kv_heads && a.frames >= 2 * kRowBlock && rows_lds_bytes(n) <= kStageLds) {
-    const dim3 grid(a.kv_heads, (a.frames + kRowBlock - 1) / kRowBlock);
-    const auto rows = [&](auto kernel, int threads) {
-      static const hipError_t raised_rows =
-          hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)kStageLds);
-      if (raised_rows == hipSuccess) kernel<<<grid, threads, rows_lds_bytes(n), s>>>(a);
-      return raised_rows;
-    };
     // Up to two workgroups a CU, the time is that of the last rows' workgroup,
     // which eight waves shorten (375 rows: 49.5 -> 39 us a layer); with more, two
     // workgroups of four waves a CU fill each other's waits (prefill of 750 rows
     // 5.6 ms against 6.3; 500 rows, 504 workgroups, 4.76 and 4.68).
-    const hipError_t e = grid.x * grid.y <= 512 ? rows(attn_rows_kernel<512>, 512) : rows(attn_rows_kernel<256>, 256);
-    if (e != hipSuccess) return e;
-    return hipGetLastError();
+    return a.kv_heads * ((a.frames + kRowBlock - 1) / kRowBlock) <= 512 ? launch_attn_rows<512>(a, n, s)
+                                                                        : launch_attn_rows<256>(a, n, s);
   }
   attn_prefill_kernel<<<dim3(a.heads, a.frames), 256, a.stage ? staged : (size_t)n * 4, s>>>(a);
   return hipGetLastError();
