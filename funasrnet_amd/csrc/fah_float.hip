@@ -459,7 +459,9 @@ __global__ __launch_bounds__(64 * WN * KS) void f32_split_gemm_kernel(
 // first, and 256 k a round: one frame of 1024 -> 3072 6.5 us, here 3.9, of 3072
 // -> 1024 9.1 and 3.8, both at what a call costs the host; 1024 -> 151936 113 and
 // 106, 5.9 TB/s). Then a wave reduction per row and frame. VEC: 16-byte loads (K
-// % 4 == 0, aligned rows).
+// % 4 == 0); frames may start at any float, with the same order of the sum.
+typedef float floatx4_any __attribute__((ext_vector_type(4), aligned(4)));
+
 template <int MF, int RW, bool VEC>
 __global__ __launch_bounds__(256) void f32_gemv_kernel(const float* __restrict__ x, const float* __restrict__ w,
                                                        const float* __restrict__ bias, float* __restrict__ out, int M,
@@ -472,7 +474,7 @@ __global__ __launch_bounds__(256) void f32_gemv_kernel(const float* __restrict__
 #pragma unroll
       for (int e = 0; e < E; e += 4) {
         const int k = k0 + 64 * e + 4 * lane;
-        const float4 q = all || k < K ? *reinterpret_cast<const float4*>(row + k) : make_float4(0.f, 0.f, 0.f, 0.f);
+        const floatx4 q = all || k < K ? floatx4(*reinterpret_cast<const floatx4_any*>(row + k)) : floatx4{0.f, 0.f, 0.f, 0.f};
         v[e] = q.x;
         v[e + 1] = q.y;
         v[e + 2] = q.z;
@@ -1102,7 +1104,6 @@ hipError_t launch_f32_split(float* w, int64_t rows, int cols, hipStream_t s) {
 hipError_t launch_f32_linear(const float* x, const float* w, const float* bias, float* out, int M, int N, int K,
                              bool relu, bool splittable, hipStream_t s) {
   if (M < 1 || N < 1 || K < 1) return hipErrorInvalidValue;
-  const bool vec = K % 4 == 0 && reinterpret_cast<uintptr_t>(x) % 16 == 0;
   if (M <= 4 || (M <= 8 && N <= 8192)) {
     // One row a wave; four (fewer reads of the frames' values) only where they
     // still leave the chip many rounds of waves. Measured, us (one row, four rows,
@@ -1112,7 +1113,7 @@ hipError_t launch_f32_linear(const float* x, const float* w, const float* bias, 
 #define FAH_GEMV(MF, RW)                                                                                        \
   do {                                                                                                          \
     const int groups = std::min((N + 4 * RW - 1) / (4 * RW), 2048);                                             \
-    if (vec) f32_gemv_kernel<MF, RW, true><<<groups, 256, 0, s>>>(x, w, bias, out, M, N, K, relu);              \
+    if (K % 4 == 0) f32_gemv_kernel<MF, RW, true><<<groups, 256, 0, s>>>(x, w, bias, out, M, N, K, relu);              \
     else f32_gemv_kernel<MF, RW, false><<<groups, 256, 0, s>>>(x, w, bias, out, M, N, K, relu);                 \
   } while (0)
     const bool many = N >= 65536;
@@ -1128,6 +1129,7 @@ hipError_t launch_f32_linear(const float* x, const float* w, const float* bias, 
 #undef FAH_GEMV
     return hipGetLastError();
   }
+  const bool vec = K % 4 == 0 && reinterpret_cast<uintptr_t>(x) % 16 == 0;
   const uint4* planes = reinterpret_cast<const uint4*>(reinterpret_cast<const char*>(w) + planes_offset(N, K));
   const auto tiles = [&](int tm, int tn) { return ((M + tm - 1) / tm) * ((N + tn - 1) / tn); };
   const auto run = [&](auto aligned, auto unaligned, int grid, int threads) {

@@ -56,6 +56,27 @@ def test_gemv(backend, frames, cols, rows):
     check(run(backend, x, w, b), x, w, b)
 
 
+@pytest.mark.parametrize("frames,cols,rows", [(1, 1024, 70), (1, 516, 65541), (3, 1028, 33), (8, 2052, 65), (40, 560, 100),
+                                              (600, 132, 1100)])
+def test_frames_at_any_float(backend, frames, cols, rows):
+    """Device frames that start at a multiple of 4 bytes give the bits that aligned ones do."""
+    from funasrnet_amd import device
+    from funasrnet_amd.hip import HipFloatWeight
+    rng = np.random.default_rng(rows)
+    x = rng.standard_normal((frames, cols)).astype(np.float32)
+    weight = HipFloatWeight(backend, rng.standard_normal((rows, cols)).astype(np.float32))
+    results = []
+    for offset in range(4):
+        held = np.zeros(x.size + 4, np.float32)
+        held[offset:offset + x.size] = x.ravel()
+        dx, out = device.DeviceArray.from_numpy(held), device.DeviceArray((frames, rows), np.float32)
+        backend.linear_device(dx.ptr + 4 * offset, frames, weight, None, out.ptr)
+        backend.synchronize()
+        results.append(out.numpy())
+    for r in results[1:]:
+        assert np.array_equal(r.view(np.uint32), results[0].view(np.uint32))
+
+
 @pytest.mark.parametrize("frames,rows", [(40, 70), (400, 700), (1100, 2100)])
 def test_split_range(backend, frames, rows):
     """Zero frames, tiny and huge values, infinities and NaN."""
