@@ -160,7 +160,7 @@ class _Output:
 
     def accept(self) -> bool:
         if self.array is not self.output:
-            self.output.reshape(-1)[:] = self.array
+            self.output[...] = self.array.reshape(self.output.shape)
         return True
 
 

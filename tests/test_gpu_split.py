@@ -204,6 +204,8 @@ def test_output_arrays(backend):
     assert backend.try_linear(x, 9, w, None, wide) and np.array_equal(wide, plain)
     every_other = np.zeros(2 * 9 * 6, np.float32)[::2]
     assert backend.try_linear(x, 9, w, None, every_other) and np.array_equal(every_other, plain.ravel())
+    for strided in (np.zeros((9, 12), np.float32)[:, ::2], np.zeros((6, 9), np.float32).T, np.zeros((9, 8), np.float32)[:, 1:7]):
+        assert backend.try_linear(x, 9, w, None, strided) and np.array_equal(strided, plain)
     same = rng.standard_normal((6, 6)).astype(np.float32)
     expected = run(backend, same.copy(), w[:, :6].copy())
     assert backend.try_linear(same, 6, w[:, :6].copy(), None, same) and np.array_equal(same, expected)
