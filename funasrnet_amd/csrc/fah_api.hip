@@ -199,8 +199,12 @@ struct Ctx {
   int64_t minimum_operations = 250000;
   DeviceBuffer in, out, q, s;
   // Planes and partial sums of an attention call (stream-ordered: one call's
-  // kernels run before the next one's), and the calls that used them.
+  // kernels run before the next one's), and the calls that used them. Buffers
+  // that a longer call has outgrown stay until the context ends: kernels may
+  // still read them, and freeing would wait. Each growth at least doubles, so
+  // together they are no larger than the one in use.
   DeviceBuffer attention;
+  std::vector<DeviceBuffer> attention_outgrown;
   unsigned attention_epoch = 0;
   std::string name;
   std::unique_ptr<SessionBatch> batch;  // last lock-step batch (its sessions alive)
@@ -249,6 +253,7 @@ Ctx::~Ctx() {
   q.release();
   s.release();
   attention.release();
+  attention_outgrown.clear();
   if (mark) (void)hipEventDestroy(mark);
   if (t0) (void)hipEventDestroy(t0);
   if (t1) (void)hipEventDestroy(t1);
@@ -317,22 +322,31 @@ struct CallMeter {
 // The attention workspace for these buffers, or nullptr where the kernel
 // without one runs: shapes that have none, a stream under capture (a graph
 // would keep the address of a buffer that a later, larger call replaces) and
-// no memory left.
+// no memory left. Never waits for the stream.
 void* attention_workspace(Ctx* c, const float* q, const float* k, const float* out, int frames, int width, int heads) {
   const size_t bytes = fah::f32_attention_workspace(q, k, out, frames, width, heads);
   if (!bytes) return nullptr;
   hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
   if (hipStreamIsCapturing(c->stream, &capture) != hipSuccess || capture != hipStreamCaptureStatusNone) return nullptr;
   if (bytes > c->attention.bytes) {
-    check(hipStreamSynchronize(c->stream), "hipStreamSynchronize");  // earlier calls still read the old one
-    c->attention.release();
-    if (hipMalloc(&c->attention.ptr, bytes) != hipSuccess) {
+    // (This thread may be capturing another stream, which an allocation would
+    // break in any but the relaxed mode.)
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    check(hipThreadExchangeStreamCaptureMode(&mode), "hipThreadExchangeStreamCaptureMode");
+    DeviceBuffer larger;
+    for (const size_t size : {std::max(bytes, 2 * c->attention.bytes), bytes}) {
+      if (hipMalloc(&larger.ptr, size) == hipSuccess) {
+        larger.bytes = size;
+        break;
+      }
       (void)hipGetLastError();
-      c->attention.ptr = nullptr;
-      return nullptr;
+      larger.ptr = nullptr;
     }
-    c->attention.bytes = bytes;
-    check(hipMemsetAsync(c->attention.ptr, 0, 4096, c->stream), "hipMemsetAsync");
+    check(hipThreadExchangeStreamCaptureMode(&mode), "hipThreadExchangeStreamCaptureMode");
+    if (!larger.ptr) return nullptr;
+    check(hipMemsetAsync(larger.ptr, 0, 4096, c->stream), "hipMemsetAsync");
+    if (c->attention.ptr) c->attention_outgrown.push_back(std::move(c->attention));
+    c->attention = std::move(larger);
     c->attention_epoch = 0;
   }
   if (++c->attention_epoch == 0) ++c->attention_epoch;

@@ -195,6 +195,40 @@ def test_split_attention_large_scores(backend, frames, heads, size, scale):
     assert clear > 0.9 * frames * heads
 
 
+def test_attention_workspace_grows(oracle_lib):
+    """Ever longer device calls on a busy stream return before it has drained, and
+    also while the thread captures another stream."""
+    import ctypes
+    from funasrnet_amd import device
+    from funasrnet_amd.hip import HipBackend, HipFloatWeight
+    backend, rt = HipBackend(0, minimum_operations=0), device.runtime()
+    other, graph = ctypes.c_void_p(), ctypes.c_void_p()
+    assert rt.hipStreamCreate(ctypes.byref(other)) == 0
+    rng = np.random.default_rng(8)
+    weight = HipFloatWeight(backend, rng.standard_normal((512, 2048)).astype(np.float32))
+    x, y = device.DeviceArray((4000, 2048), np.float32), device.DeviceArray((4000, 512), np.float32)
+    x.fill_zero()
+    calls = []
+    for frames in (400, 640, 1000, 1001):
+        q, k, v = (rng.uniform(-2, 2, (frames, 256)).astype(np.float32) for _ in range(3))
+        calls.append((frames, (q, k, v), [device.DeviceArray.from_numpy(a) for a in (q, k, v)],
+                      device.DeviceArray((frames, 256), np.float32)))
+    device.synchronize()
+    for frames, _, d, out in calls:
+        for _ in range(400):  # some 20 ms of work
+            backend.linear_device(x.ptr, 4000, weight, None, y.ptr)
+        assert rt.hipStreamBeginCapture(other, 0) == 0  # global: this thread may not allocate by itself
+        backend.attention_device(d[0].ptr, d[1].ptr, d[2].ptr, frames, 256, 2, out.ptr)
+        assert rt.hipStreamEndCapture(other, ctypes.byref(graph)) == 0
+        assert rt.hipStreamQuery(ctypes.c_void_p(backend.stream)) == 600  # hipErrorNotReady
+        rt.hipGraphDestroy(graph)
+    backend.synchronize()
+    for frames, host, _, out in calls:
+        assert np.abs(out.numpy() - oracle_lib.attention_f64(*host, frames, 256, 2)).max() <= 5e-5 * 2
+    rt.hipStreamDestroy(other)
+    backend.close()
+
+
 def test_output_arrays(backend):
     """Results land in the caller's array, also one that the library cannot write."""
     rng = np.random.default_rng(2)
