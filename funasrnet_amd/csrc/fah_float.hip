@@ -65,6 +65,7 @@ typedef float floatx4 __attribute__((ext_vector_type(4)));
 // infinities, NaN or values that round past the largest bf16 make sums infinite
 // or NaN; a workgroup that finds such a sum, one below kSplitLow, or zeros and
 // frames with values below kSplitTiny, forms its tile again on fp32 MFMA (tile_f32).
+// Other weights run on the fp32 MFMA kernels below.
 constexpr uint32_t kSplitLow = 0x1c800000u;      // 2^-70
 constexpr uint32_t kSplitTiny = 0x0d800000u;     // 2^-100
 constexpr uint32_t kSplitMost = 0x49800000u;     // 2^20
@@ -233,7 +234,7 @@ __device__ __forceinline__ int split_slot(int row, int chunk) {
 template <int WN, int KS, int TI, int TJ, int KB, int D, bool VEC>
 __global__ __launch_bounds__(64 * WN * KS) void f32_split_gemm_kernel(
     const float* __restrict__ x, const float* __restrict__ w, const uint4* __restrict__ planes,
-    const float* __restrict__ bias, float* __restrict__ out, int M, int N, int K, int relu, int splittable) {
+    const float* __restrict__ bias, float* __restrict__ out, int M, int N, int K, int relu) {
   constexpr int TM = 32 * TI, TN = 32 * TJ * WN, WAVES = WN * KS, NT = 64 * WAVES, KT = 32 * KB;
   constexpr int CH = KT / 8, PLANE = TM * KT * 2, BUF = 3 * PLANE, UA = TM * CH / NT, HS = 2 * KB / KS;
   static_assert(D % 2 == 0 && 128 % (D * KT) == 0, "two LDS buffers; planes padded to whole groups of D tiles");
@@ -448,7 +449,274 @@ __global__ __launch_bounds__(64 * WN * KS) void f32_split_gemm_kernel(
     }
     return true;
   };
-  if (!splittable || !split_tile()) tile_f32<TM, TN, WAVES>(smem, x, w, bias, out, M, N, K, f0, n0, relu);
+  if (!split_tile()) tile_f32<TM, TN, WAVES>(smem, x, w, bias, out, M, N, K, f0, n0, relu);
+}
+
+// ---- GEMM on fp32 MFMA: weights that the planes do not hold -----------------------
+// out[f][n] = sum_k x[f][k] * w[n][k] (+ bias[n]) (ReLU), any M (frames), N,
+// K with K % 4 == 0 and 16-byte aligned rows. Four waves in a 2 x 2 grid,
+// each a (16 BI) x (16 BJ) tile of v_mfma_f32_16x16x4f32 blocks; workgroup
+// tile (32 BI) x (32 BJ); K in tiles of GK staged in two LDS buffers as
+// row-major [row][GK + 4] (16-byte loads and stores; the next tile's global
+// loads sit in registers while the current one is multiplied, then go to
+// the other buffer, one barrier per tile). Lane layout of 16x16x4: A[i][k]
+// from lane i + 16k, B[k][j] from lane j + 16k, D[4q + r][j] in lane j + 16q
+// (r < 4). In substep s of a K tile, lane group q multiplies k =
+// (GK / 4) q + s, so each lane reads its GK / 4 values of a row as 16-byte
+// LDS reads. One order per shape: the same bits whichever entry point runs it.
+constexpr int kGK = 64;
+
+template <int BI, int BJ>
+__global__ __launch_bounds__(256) void f32_gemm_kernel(const float* __restrict__ x, const float* __restrict__ w,
+                                                       const float* __restrict__ bias, float* __restrict__ out, int M,
+                                                       int N, int K, int relu) {
+  constexpr int TM = 32 * BI, TN = 32 * BJ;              // workgroup tile
+  constexpr int ROW = kGK + 4, KQ = kGK / 4;              // LDS row (floats); k values per lane group
+  constexpr int PER_ROW = kGK / 4, ROWS = 256 / PER_ROW;  // 16-byte loads per row; rows per pass
+  constexpr int LA = TM / ROWS, LB = TN / ROWS;           // 16-byte loads per thread and operand
+  static_assert(LA >= 1 && LB >= 1 && TM % ROWS == 0 && TN % ROWS == 0, "whole load passes");
+  __shared__ __attribute__((aligned(16))) float a_s[2][TM * ROW];
+  __shared__ __attribute__((aligned(16))) float b_s[2][TN * ROW];
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+  const int f0 = blockIdx.y * TM, n0 = blockIdx.x * TN;
+  const int wm = (wave >> 1) * 16 * BI, wn = (wave & 1) * 16 * BJ;
+  const int li = lane & 15, lq = lane >> 4;
+  floatx4 acc[BI][BJ];
+#pragma unroll
+  for (int i = 0; i < BI; ++i)
+#pragma unroll
+    for (int j = 0; j < BJ; ++j) acc[i][j] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+  // Global loads: thread t takes row t / PER_ROW (+ ROWS per further load),
+  // the 16 bytes at k = 4 (t % PER_ROW) of the tile; rows past the edge and
+  // k past K read as zero.
+  const int lr = tid / PER_ROW, lc = 4 * (tid % PER_ROW);
+  float4 ra[LA], rb[LB];
+  auto fetch = [&](int k0) {
+    const int k = k0 + lc;
+#pragma unroll
+    for (int u = 0; u < LA; ++u) {
+      const int f = f0 + lr + ROWS * u;
+      ra[u] = (f < M && k < K) ? *reinterpret_cast<const float4*>(x + (size_t)f * K + k) : make_float4(0.f, 0.f, 0.f, 0.f);
+    }
+#pragma unroll
+    for (int u = 0; u < LB; ++u) {
+      const int n = n0 + lr + ROWS * u;
+      rb[u] = (n < N && k < K) ? *reinterpret_cast<const float4*>(w + (size_t)n * K + k) : make_float4(0.f, 0.f, 0.f, 0.f);
+    }
+  };
+  auto stage = [&](int buf) {
+#pragma unroll
+    for (int u = 0; u < LA; ++u) *reinterpret_cast<float4*>(&a_s[buf][(lr + ROWS * u) * ROW + lc]) = ra[u];
+#pragma unroll
+    for (int u = 0; u < LB; ++u) *reinterpret_cast<float4*>(&b_s[buf][(lr + ROWS * u) * ROW + lc]) = rb[u];
+  };
+  fetch(0);
+  stage(0);
+  __syncthreads();
+  int buf = 0;
+  for (int k0 = 0; k0 < K; k0 += kGK) {
+    const bool more = k0 + kGK < K;
+    if (more) fetch(k0 + kGK);
+#pragma unroll
+    for (int h = 0; h < KQ / 4; ++h) {
+      float4 av[BI], bv[BJ];
+#pragma unroll
+      for (int i = 0; i < BI; ++i)
+        av[i] = *reinterpret_cast<const float4*>(&a_s[buf][(wm + 16 * i + li) * ROW + KQ * lq + 4 * h]);
+#pragma unroll
+      for (int j = 0; j < BJ; ++j)
+        bv[j] = *reinterpret_cast<const float4*>(&b_s[buf][(wn + 16 * j + li) * ROW + KQ * lq + 4 * h]);
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+#pragma unroll
+        for (int i = 0; i < BI; ++i)
+#pragma unroll
+          for (int j = 0; j < BJ; ++j) {
+            const float a = e == 0 ? av[i].x : e == 1 ? av[i].y : e == 2 ? av[i].z : av[i].w;
+            const float b = e == 0 ? bv[j].x : e == 1 ? bv[j].y : e == 2 ? bv[j].z : bv[j].w;
+            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, acc[i][j], 0, 0, 0);
+          }
+    }
+    if (more) {
+      stage(buf ^ 1);
+      __syncthreads();
+      buf ^= 1;
+    }
+  }
+#pragma unroll
+  for (int j = 0; j < BJ; ++j) {
+    const int n = n0 + wn + 16 * j + li;
+    if (n >= N) continue;
+    const float b = bias ? bias[n] : 0.0f;
+#pragma unroll
+    for (int i = 0; i < BI; ++i)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int f = f0 + wm + 16 * i + 4 * lq + r;
+        if (f < M) {
+          float v = acc[i][j][r] + b;
+          if (relu) v = v < 0.0f ? 0.0f : v;  // (-0 and NaN pass, as the reference's `v < 0 ? 0 : v`)
+          out[(size_t)f * N + n] = v;
+        }
+      }
+  }
+}
+
+// The same product for grids of at most one workgroup per CU: each of the
+// four waves covers the whole 32 x 64 tile (2 x 4 blocks, eight
+// accumulators in flight) over its quarter of every K tile (lane group q of
+// wave w takes k = 16 w + 4 q .. + 3), and the four partial tiles are added
+// in wave order in LDS at the end.
+__global__ __launch_bounds__(256) void f32_gemm_wavek_kernel(const float* __restrict__ x, const float* __restrict__ w,
+                                                             const float* __restrict__ bias, float* __restrict__ out,
+                                                             int M, int N, int K, int relu) {
+  constexpr int GK = 64, TM = 32, TN = 64, ROW = GK + 4;
+  constexpr int PER_ROW = GK / 4, ROWS = 256 / PER_ROW, LA = TM / ROWS, LB = TN / ROWS;
+  __shared__ __attribute__((aligned(16))) float a_s[2][TM * ROW];
+  __shared__ __attribute__((aligned(16))) float b_s[2][TN * ROW];
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+  const int f0 = blockIdx.y * TM, n0 = blockIdx.x * TN;
+  const int li = lane & 15, lq = lane >> 4;
+  floatx4 acc[2][4];
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) acc[i][j] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+  const int lr = tid / PER_ROW, lc = 4 * (tid % PER_ROW);
+  float4 ra[LA], rb[LB];
+  auto fetch = [&](int k0) {
+    const int k = k0 + lc;
+#pragma unroll
+    for (int u = 0; u < LA; ++u) {
+      const int f = f0 + lr + ROWS * u;
+      ra[u] = (f < M && k < K) ? *reinterpret_cast<const float4*>(x + (size_t)f * K + k) : make_float4(0.f, 0.f, 0.f, 0.f);
+    }
+#pragma unroll
+    for (int u = 0; u < LB; ++u) {
+      const int n = n0 + lr + ROWS * u;
+      rb[u] = (n < N && k < K) ? *reinterpret_cast<const float4*>(w + (size_t)n * K + k) : make_float4(0.f, 0.f, 0.f, 0.f);
+    }
+  };
+  auto stage = [&](int buf) {
+#pragma unroll
+    for (int u = 0; u < LA; ++u) *reinterpret_cast<float4*>(&a_s[buf][(lr + ROWS * u) * ROW + lc]) = ra[u];
+#pragma unroll
+    for (int u = 0; u < LB; ++u) *reinterpret_cast<float4*>(&b_s[buf][(lr + ROWS * u) * ROW + lc]) = rb[u];
+  };
+  fetch(0);
+  stage(0);
+  __syncthreads();
+  int buf = 0;
+  const int kl = 16 * wave + 4 * lq;
+  for (int k0 = 0; k0 < K; k0 += GK) {
+    const bool more = k0 + GK < K;
+    if (more) fetch(k0 + GK);
+    float4 av[2], bv[4];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) av[i] = *reinterpret_cast<const float4*>(&a_s[buf][(16 * i + li) * ROW + kl]);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) bv[j] = *reinterpret_cast<const float4*>(&b_s[buf][(16 * j + li) * ROW + kl]);
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const float a = e == 0 ? av[i].x : e == 1 ? av[i].y : e == 2 ? av[i].z : av[i].w;
+          const float b = e == 0 ? bv[j].x : e == 1 ? bv[j].y : e == 2 ? bv[j].z : bv[j].w;
+          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, acc[i][j], 0, 0, 0);
+        }
+    if (more) {
+      stage(buf ^ 1);
+      __syncthreads();
+      buf ^= 1;
+    }
+  }
+  // Partial tiles into LDS (the staging buffers, free once every wave is
+  // past its last reads): part[w][f][n], then summed in wave order.
+  __syncthreads();
+  float* part = &a_s[0][0];
+  static_assert(4 * TM * TN <= 2 * TM * ROW + 2 * TN * ROW, "partials fit the staging buffers");
+  float* part_b = &b_s[0][0];
+  auto slot = [&](int wv, int f, int n) -> float& {
+    const int e = (wv * TM + f) * TN + n;
+    return e < 2 * TM * ROW ? part[e] : part_b[e - 2 * TM * ROW];
+  };
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) slot(wave, 16 * i + 4 * lq + r, 16 * j + li) = acc[i][j][r];
+  __syncthreads();
+  for (int e = tid; e < TM * TN; e += 256) {
+    const int f = e / TN, n = e % TN;
+    if (f0 + f >= M || n0 + n >= N) continue;
+    float v = ((slot(0, f, n) + slot(1, f, n)) + slot(2, f, n)) + slot(3, f, n);
+    v = v + (bias ? bias[n0 + n] : 0.0f);
+    if (relu) v = v < 0.0f ? 0.0f : v;
+    out[(size_t)(f0 + f) * N + n0 + n] = v;
+  }
+}
+
+// Any K and alignment: 64 x 64 tiles, K in steps of 32 staged in LDS one
+// float per thread and row, four waves of 2 x 2 v_mfma_f32_16x16x4f32 blocks.
+constexpr int kGT = 64, kGA = 32, kGPad = kGA + 1;
+
+__global__ __launch_bounds__(256) void f32_gemm_any_kernel(const float* __restrict__ x, const float* __restrict__ w,
+                                                           const float* __restrict__ bias, float* __restrict__ out,
+                                                           int M, int N, int K, int relu) {
+  __shared__ float a_s[kGT][kGPad];  // frames x k
+  __shared__ float b_s[kGT][kGPad];  // rows x k
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+  const int f0 = blockIdx.y * kGT, n0 = blockIdx.x * kGT;
+  const int fm = (wave >> 1) * 32, rn = (wave & 1) * 32;
+  floatx4 acc[2][2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j) acc[i][j] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+  // Staging: thread t loads rows t / 32 + 8 s (s < 8), column t % 32.
+  const int lr = tid >> 5, lc = tid & 31;
+  for (int k0 = 0; k0 < K; k0 += kGA) {
+    const int k = k0 + lc;
+#pragma unroll
+    for (int s = 0; s < 8; ++s) {
+      const int r = lr + 8 * s;
+      const int f = f0 + r, n = n0 + r;
+      a_s[r][lc] = (f < M && k < K) ? x[(size_t)f * K + k] : 0.0f;
+      b_s[r][lc] = (n < N && k < K) ? w[(size_t)n * K + k] : 0.0f;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int ks = 0; ks < kGA; ks += 4) {
+      const int kk = ks + (lane >> 4), ii = lane & 15;
+      const float a0 = a_s[fm + ii][kk], a1 = a_s[fm + 16 + ii][kk];
+      const float b0 = b_s[rn + ii][kk], b1 = b_s[rn + 16 + ii][kk];
+      acc[0][0] = __builtin_amdgcn_mfma_f32_16x16x4f32(a0, b0, acc[0][0], 0, 0, 0);
+      acc[0][1] = __builtin_amdgcn_mfma_f32_16x16x4f32(a0, b1, acc[0][1], 0, 0, 0);
+      acc[1][0] = __builtin_amdgcn_mfma_f32_16x16x4f32(a1, b0, acc[1][0], 0, 0, 0);
+      acc[1][1] = __builtin_amdgcn_mfma_f32_16x16x4f32(a1, b1, acc[1][1], 0, 0, 0);
+    }
+    __syncthreads();
+  }
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      const int n = n0 + rn + 16 * j + (lane & 15);
+      if (n >= N) continue;
+      const float b = bias ? bias[n] : 0.0f;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int f = f0 + fm + 16 * i + 4 * (lane >> 4) + r;
+        if (f < M) {
+          float v = acc[i][j][r] + b;
+          if (relu) v = v < 0.0f ? 0.0f : v;
+          out[(size_t)f * N + n] = v;
+        }
+      }
+    }
 }
 
 // ---- GEMV (few frames, weight-bandwidth bound) ------------------------------
@@ -1101,6 +1369,30 @@ hipError_t launch_f32_split(float* w, int64_t rows, int cols, hipStream_t s) {
   return hipGetLastError();
 }
 
+// The GEMM on fp32 MFMA.
+static hipError_t launch_f32_gemm(const float* x, const float* w, const float* bias, float* out, int M, int N, int K,
+                                  bool relu, hipStream_t s) {
+  const bool aligned = K % 4 == 0 && reinterpret_cast<uintptr_t>(x) % 16 == 0;
+  if (!aligned) {
+    const dim3 grid((N + kGT - 1) / kGT, (M + kGT - 1) / kGT);
+    f32_gemm_any_kernel<<<grid, 256, 0, s>>>(x, w, bias, out, M, N, K, relu);
+    return hipGetLastError();
+  }
+  // The tile whose grid loads the CUs most evenly: rounds of 256
+  // workgroups times the tile's area, the larger tile on a tie; a grid of at
+  // most one 32 x 64 workgroup per CU splits K over its waves.
+  const int big = ((M + 63) / 64) * ((N + 63) / 64), small = ((M + 31) / 32) * ((N + 63) / 64);
+  const int64_t big_cost = (int64_t)((big + 255) / 256) * 2, small_cost = (small + 255) / 256;
+  const dim3 grid((N + 63) / 64, (M + 31) / 32);
+  if (big_cost <= small_cost)
+    f32_gemm_kernel<2, 2><<<dim3((N + 63) / 64, (M + 63) / 64), 256, 0, s>>>(x, w, bias, out, M, N, K, relu);
+  else if (small <= 256 && K >= 256)
+    f32_gemm_wavek_kernel<<<grid, 256, 0, s>>>(x, w, bias, out, M, N, K, relu);
+  else
+    f32_gemm_kernel<1, 2><<<grid, 256, 0, s>>>(x, w, bias, out, M, N, K, relu);
+  return hipGetLastError();
+}
+
 hipError_t launch_f32_linear(const float* x, const float* w, const float* bias, float* out, int M, int N, int K,
                              bool relu, bool splittable, hipStream_t s) {
   if (M < 1 || N < 1 || K < 1) return hipErrorInvalidValue;
@@ -1129,12 +1421,13 @@ hipError_t launch_f32_linear(const float* x, const float* w, const float* bias, 
 #undef FAH_GEMV
     return hipGetLastError();
   }
+  if (!splittable) return launch_f32_gemm(x, w, bias, out, M, N, K, relu, s);
   const bool vec = K % 4 == 0 && reinterpret_cast<uintptr_t>(x) % 16 == 0;
   const uint4* planes = reinterpret_cast<const uint4*>(reinterpret_cast<const char*>(w) + planes_offset(N, K));
   const auto tiles = [&](int tm, int tn) { return ((M + tm - 1) / tm) * ((N + tn - 1) / tn); };
   const auto run = [&](auto aligned, auto unaligned, int grid, int threads) {
-    if (vec) aligned<<<grid, threads, 0, s>>>(x, w, planes, bias, out, M, N, K, relu, splittable);
-    else unaligned<<<grid, threads, 0, s>>>(x, w, planes, bias, out, M, N, K, relu, splittable);
+    if (vec) aligned<<<grid, threads, 0, s>>>(x, w, planes, bias, out, M, N, K, relu);
+    else unaligned<<<grid, threads, 0, s>>>(x, w, planes, bias, out, M, N, K, relu);
   };
 #define FAH_SPLIT(WN, KS, TI, TJ, KB, D)                                                                     \
   run(f32_split_gemm_kernel<WN, KS, TI, TJ, KB, D, true>, f32_split_gemm_kernel<WN, KS, TI, TJ, KB, D, false>, \

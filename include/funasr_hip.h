@@ -175,7 +175,9 @@ int fah_quantized_linear_noalloc(fah_context* context, const float* input, int f
  * reference device version src/FunAsrNet.Vulkan/VulkanFloatBackend.cs:127-171):
  * output[frames*rows] = input[frames*cols] W^T (+ bias) for an FP32 weight,
  * on the matrix cores with fp32 sums (each value split exactly into three bf16
- * planes), or a bandwidth-bound GEMV for up to 4 frames (8 of up to 8192 rows). Declines
+ * planes, or fp32 MFMA where a weight has values that the planes do not hold:
+ * above 2^20, or below 2^-100 but not 0, or rows below 2^-80), or a
+ * bandwidth-bound GEMV for up to 4 frames (8 of up to 8192 rows). Declines
  * (output untouched) Q8_0 weights and projections below the minimum
  * operations. Float order differs from the CPU kernels, as the reference's
  * own device path does (its check: 2e-4 x max(1, |expected|)). The encoder's

@@ -114,6 +114,18 @@ def test_weights_outside_the_planes(backend, value):
         assert not np.any(np.isfinite(got[:, 4]))
 
 
+# Their kernels: 64 x 64 and 32 x 64 tiles, 32 x 64 with K over the waves, any K.
+@pytest.mark.parametrize("frames,cols,rows", [(257, 68, 1000), (33, 132, 70), (65, 260, 65), (1025, 1024, 513), (130, 75, 67)])
+@pytest.mark.parametrize("biased", [False, True])
+def test_fp32_tiles(backend, frames, cols, rows, biased):
+    rng = np.random.default_rng(cols)
+    x = rng.standard_normal((frames, cols)).astype(np.float32)
+    w = rng.standard_normal((rows, cols)).astype(np.float32)
+    w[rows - 1, cols - 1] = 2.0**21
+    b = rng.standard_normal(rows).astype(np.float32) if biased else None
+    check(run(backend, x, w, b), x, w, b)
+
+
 @pytest.mark.parametrize("value,partner", [(2.0**-135, 2.0**80), (2.0**-125, 2.0**100), (2.0**-118, 2.0**60)])
 def test_tiny_weight_beside_ordinary_ones(backend, value, partner):
     """An element that the planes do not hold, in a row of ordinary ones, against
