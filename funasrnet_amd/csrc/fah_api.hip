@@ -98,6 +98,18 @@ struct DeviceBuffer {
     check(hipMalloc(&ptr, n), "hipMalloc");
     bytes = n;
   }
+  // False, and empty, for n == 0 and where there is no memory left.
+  bool try_allocate(size_t n) {
+    release();
+    if (n == 0) return false;
+    if (hipMalloc(&ptr, n) != hipSuccess) {
+      (void)hipGetLastError();
+      ptr = nullptr;
+      return false;
+    }
+    bytes = n;
+    return true;
+  }
   void ensure(size_t n) {
     if (n > bytes) allocate(n);
   }
@@ -334,14 +346,7 @@ void* attention_workspace(Ctx* c, const float* q, const float* k, const float* o
     hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
     check(hipThreadExchangeStreamCaptureMode(&mode), "hipThreadExchangeStreamCaptureMode");
     DeviceBuffer larger;
-    for (const size_t size : {std::max(bytes, 2 * c->attention.bytes), bytes}) {
-      if (hipMalloc(&larger.ptr, size) == hipSuccess) {
-        larger.bytes = size;
-        break;
-      }
-      (void)hipGetLastError();
-      larger.ptr = nullptr;
-    }
+    if (!larger.try_allocate(std::max(bytes, 2 * c->attention.bytes))) larger.try_allocate(bytes);
     check(hipThreadExchangeStreamCaptureMode(&mode), "hipThreadExchangeStreamCaptureMode");
     if (!larger.ptr) return nullptr;
     check(hipMemsetAsync(larger.ptr, 0, 4096, c->stream), "hipMemsetAsync");
@@ -397,11 +402,11 @@ struct fah_weight {
   bool half_scales = true;
   DeviceBuffer q, s;
   int group_rows = 1;
-  // FP32 weight (Weight.Values): `f` holds [rows][cols] floats and their bf16
-  // planes (fah::f32_weight_bytes), q/s unused.
+  // FP32 weight (Weight.Values): `f` holds [rows][cols] floats
+  // (fah::f32_weight_bytes), `planes` their bf16 planes (empty where there are
+  // none), q/s unused.
   bool f32 = false;
-  bool splittable = false;
-  DeviceBuffer f;
+  DeviceBuffer f, planes;
 };
 
 struct DeviceMatrix {
@@ -1608,7 +1613,7 @@ int fah_weight_release(fah_weight* w) {
 }
 
 int64_t fah_weight_device_bytes(const fah_weight* w) {
-  return w ? (int64_t)(w->q.bytes + w->s.bytes + w->f.bytes) : 0;
+  return w ? (int64_t)(w->q.bytes + w->s.bytes + w->f.bytes + w->planes.bytes) : 0;
 }
 
 int fah_weight_f32_upload(fah_context* h, const float* values, int rows, int cols, fah_weight** out) {
@@ -1628,12 +1633,15 @@ int fah_weight_f32_upload(fah_context* h, const float* values, int rows, int col
     w->f32 = true;
     w->f.allocate(fah::f32_weight_bytes(rows, cols));
     check(hipMemcpyAsync(w->f.ptr, values, (size_t)rows * cols * 4, hipMemcpyHostToDevice, c->stream), "H2D weight");
-    check(fah::launch_f32_split(w->f.as<float>(), rows, cols, c->stream), "split weight");
+    // Without planes (no memory left for them, among others) the weight runs on fp32 MFMA.
     int outside = 0;
-    check(hipMemcpyAsync(&outside, fah::f32_weight_outside(w->f.as<float>(), rows, cols), 4, hipMemcpyDeviceToHost, c->stream),
-          "D2H range");
+    if (w->planes.try_allocate(fah::f32_planes_bytes(rows, cols))) {
+      check(fah::launch_f32_split(w->f.as<float>(), rows, cols, w->planes.ptr, c->stream), "split weight");
+      check(hipMemcpyAsync(&outside, fah::f32_weight_outside(w->f.as<float>(), rows, cols), 4, hipMemcpyDeviceToHost, c->stream),
+            "D2H range");
+    }
     check(hipStreamSynchronize(c->stream), "hipStreamSynchronize");
-    w->splittable = outside == 0;
+    if (outside) w->planes.release();
     *out = w.release();
     return FAH_OK;
   });
@@ -1828,8 +1836,8 @@ int fah_linear_many(fah_context* h, const float* input, int frames, const fah_we
       // through the same kernel as fah_linear, so the bits equal separate calls.
       size_t at = 0;
       for (int i = 0; i < count; ++i) {
-        check(fah::launch_f32_linear(c->in.as<float>(), weights[i]->f.as<float>(), nullptr, c->out.as<float>() + at,
-                                     frames, weights[i]->rows, cols, false, weights[i]->splittable, c->stream),
+        check(fah::launch_f32_linear(c->in.as<float>(), weights[i]->f.as<float>(), weights[i]->planes.ptr, nullptr,
+                                     c->out.as<float>() + at, frames, weights[i]->rows, cols, false, c->stream),
               "f32 linear");
         at += (size_t)frames * weights[i]->rows;
       }
@@ -1892,8 +1900,8 @@ int fah_linear(fah_context* h, const float* input, int frames, const fah_weight*
       check(hipMemcpyAsync(dbias, bias, (size_t)w->rows * 4, hipMemcpyHostToDevice, c->stream), "H2D bias");
     }
     meter.kernels_begin();
-    check(fah::launch_f32_linear(c->in.as<float>(), w->f.as<float>(), dbias, c->out.as<float>(), frames, w->rows,
-                                 w->cols, false, w->splittable, c->stream),
+    check(fah::launch_f32_linear(c->in.as<float>(), w->f.as<float>(), w->planes.ptr, dbias, c->out.as<float>(), frames,
+                                 w->rows, w->cols, false, c->stream),
           "f32 linear");
     meter.kernels_end();
     check(hipMemcpyAsync(output, c->out.ptr, out_bytes, hipMemcpyDeviceToHost, c->stream), "D2H output");
@@ -1915,7 +1923,7 @@ int fah_linear_device(fah_context* h, const float* x, int frames, const fah_weig
     if (c->disposed) return fail(FAH_ERROR_DISPOSED, "context disposed");
     check(hipSetDevice(c->device), "hipSetDevice");
     DeviceWork work(*c);
-    check(fah::launch_f32_linear(x, w->f.as<float>(), bias, out, frames, w->rows, w->cols, false, w->splittable, c->stream),
+    check(fah::launch_f32_linear(x, w->f.as<float>(), w->planes.ptr, bias, out, frames, w->rows, w->cols, false, c->stream),
           "f32 linear");
     return FAH_OK;
   });
@@ -1955,9 +1963,9 @@ int fah_relu_projection(fah_context* h, const float* input, int frames, const fa
     float* dout = reinterpret_cast<float*>(c->out.as<char>() + mid_bytes);
     // The intermediate stays on the device (IReluProjectionBackend.cs:4-16).
     meter.kernels_begin();
-    check(fah::launch_f32_linear(c->in.as<float>(), first->f.as<float>(), d1, mid, frames, H, K, true, first->splittable, c->stream),
+    check(fah::launch_f32_linear(c->in.as<float>(), first->f.as<float>(), first->planes.ptr, d1, mid, frames, H, K, true, c->stream),
           "f32 linear + ReLU");
-    check(fah::launch_f32_linear(mid, second->f.as<float>(), d2, dout, frames, N, H, false, second->splittable, c->stream), "f32 linear");
+    check(fah::launch_f32_linear(mid, second->f.as<float>(), second->planes.ptr, d2, dout, frames, N, H, false, c->stream), "f32 linear");
     meter.kernels_end();
     check(hipMemcpyAsync(output, dout, out_bytes, hipMemcpyDeviceToHost, c->stream), "D2H output");
     work.release();  // enqueued: other contexts may enqueue while this stream drains

@@ -1346,26 +1346,31 @@ bool f32_attention_supported(int frames, int width, int heads) {
          width / heads <= kAMaxS;
 }
 
-// An FP32 weight on the device: its values, the range check's word (padded to
-// 16 bytes), its planes.
-static size_t planes_offset(int64_t rows, int cols) { return (((size_t)rows * cols * 4 + 15) & ~(size_t)15) + 16; }
+// Weights of fewer columns have no planes: padded to 128 k they would take more
+// than 3 times the values' memory.
+constexpr int kSplitLeastK = 64;
 
-size_t f32_weight_bytes(int64_t rows, int cols) {
-  return planes_offset(rows, cols) + (size_t)split_pieces(rows, cols) * 16;
+// An FP32 weight's values, then the range check's word.
+static size_t outside_offset(int64_t rows, int cols) { return ((size_t)rows * cols * 4 + 15) & ~(size_t)15; }
+
+size_t f32_weight_bytes(int64_t rows, int cols) { return outside_offset(rows, cols) + 16; }
+
+size_t f32_planes_bytes(int64_t rows, int cols) {
+  return cols < kSplitLeastK ? 0 : (size_t)split_pieces(rows, cols) * 16;
 }
 
 const int* f32_weight_outside(const float* w, int64_t rows, int cols) {
-  return reinterpret_cast<const int*>(reinterpret_cast<const char*>(w) + planes_offset(rows, cols) - 16);
+  return reinterpret_cast<const int*>(reinterpret_cast<const char*>(w) + outside_offset(rows, cols));
 }
 
-hipError_t launch_f32_split(float* w, int64_t rows, int cols, hipStream_t s) {
+hipError_t launch_f32_split(float* w, int64_t rows, int cols, void* planes, hipStream_t s) {
   int* outside = const_cast<int*>(f32_weight_outside(w, rows, cols));
   const hipError_t e = hipMemsetAsync(outside, 0, 16, s);
   if (e != hipSuccess) return e;
   f32_split_range_kernel<<<(int)std::min<int64_t>((rows + 3) / 4, 2048), 256, 0, s>>>(w, rows, cols, outside);
   const int64_t lanes = split_pieces(rows, cols) / 3;
-  f32_split_planes_kernel<<<(int)std::min<int64_t>((lanes + 255) / 256, 4096), 256, 0, s>>>(
-      w, rows, cols, reinterpret_cast<uint4*>(reinterpret_cast<char*>(w) + planes_offset(rows, cols)));
+  f32_split_planes_kernel<<<(int)std::min<int64_t>((lanes + 255) / 256, 4096), 256, 0, s>>>(w, rows, cols,
+                                                                                          static_cast<uint4*>(planes));
   return hipGetLastError();
 }
 
@@ -1393,8 +1398,8 @@ static hipError_t launch_f32_gemm(const float* x, const float* w, const float* b
   return hipGetLastError();
 }
 
-hipError_t launch_f32_linear(const float* x, const float* w, const float* bias, float* out, int M, int N, int K,
-                             bool relu, bool splittable, hipStream_t s) {
+hipError_t launch_f32_linear(const float* x, const float* w, const void* weight_planes, const float* bias, float* out,
+                             int M, int N, int K, bool relu, hipStream_t s) {
   if (M < 1 || N < 1 || K < 1) return hipErrorInvalidValue;
   if (M <= 4 || (M <= 8 && N <= 8192)) {
     // One row a wave; four (fewer reads of the frames' values) only where they
@@ -1421,9 +1426,9 @@ hipError_t launch_f32_linear(const float* x, const float* w, const float* bias, 
 #undef FAH_GEMV
     return hipGetLastError();
   }
-  if (!splittable) return launch_f32_gemm(x, w, bias, out, M, N, K, relu, s);
+  if (!weight_planes) return launch_f32_gemm(x, w, bias, out, M, N, K, relu, s);
   const bool vec = K % 4 == 0 && reinterpret_cast<uintptr_t>(x) % 16 == 0;
-  const uint4* planes = reinterpret_cast<const uint4*>(reinterpret_cast<const char*>(w) + planes_offset(N, K));
+  const uint4* planes = static_cast<const uint4*>(weight_planes);
   const auto tiles = [&](int tm, int tn) { return ((M + tm - 1) / tm) * ((N + tn - 1) / tn); };
   const auto run = [&](auto aligned, auto unaligned, int grid, int threads) {
     if (vec) aligned<<<grid, threads, 0, s>>>(x, w, planes, bias, out, M, N, K, relu);

@@ -250,18 +250,20 @@ hipError_t launch_session_embed(const int8_t* q, const void* scales, bool half_s
                                 const SessionRef* sessions, int count, float* x, hipStream_t s);
 
 
-// FP32 weights [N][K] as the projections take them: an allocation of
-// f32_weight_bytes that holds the values first; launch_f32_split then fills in
-// their bf16 planes and the word that f32_weight_outside points to (on the
-// device; not 0: the weight is not to be split).
+// FP32 weights [N][K]: an allocation of f32_weight_bytes that holds the values
+// first, and one of f32_planes_bytes (0: none for such widths) for their bf16
+// planes. launch_f32_split fills in the planes and the word that
+// f32_weight_outside points to (on the device; not 0: the planes do not hold
+// the values and are not to be used).
 size_t f32_weight_bytes(int64_t rows, int cols);
+size_t f32_planes_bytes(int64_t rows, int cols);
 const int* f32_weight_outside(const float* w, int64_t rows, int cols);
-hipError_t launch_f32_split(float* w, int64_t rows, int cols, hipStream_t s);
+hipError_t launch_f32_split(float* w, int64_t rows, int cols, void* planes, hipStream_t s);
 // FP32 projections y[M][N] = x[M][K] W[N][K]^T (+ bias) (ReLU): products of
-// bf16 planes on MFMA (fp32 MFMA for a weight that is not splittable), or a
+// bf16 planes on MFMA, fp32 MFMA for a weight without planes (nullptr), or a
 // GEMV for up to 4 frames (8 of up to 8192 rows).
-hipError_t launch_f32_linear(const float* x, const float* w, const float* bias, float* out, int M, int N, int K,
-                             bool relu, bool splittable, hipStream_t s);
+hipError_t launch_f32_linear(const float* x, const float* w, const void* planes, const float* bias, float* out, int M,
+                             int N, int K, bool relu, hipStream_t s);
 // Non-causal multi-head attention over [frames][width] rows (head size
 // width / heads <= 256, frames <= 4096).
 bool f32_attention_supported(int frames, int width, int heads);

@@ -126,6 +126,20 @@ def test_fp32_tiles(backend, frames, cols, rows, biased):
     check(run(backend, x, w, b), x, w, b)
 
 
+@pytest.mark.parametrize("rows,cols,value,planes", [(300, 63, 1.0, False), (300, 64, 1.0, True), (70, 500, 1.0, True),
+                                                    (70, 500, 2.0**21, False), (1, 1, 1.0, False)])
+def test_planes_memory(backend, rows, cols, value, planes):
+    """Planes are kept only where products use them: three bf16 a value, rows to 32, columns to 128."""
+    from funasrnet_amd.hip import HipFloatWeight
+    w = np.ones((rows, cols), np.float32)
+    w[-1, -1] = value
+    held = HipFloatWeight(backend, w).device_bytes
+    padded = -(-rows // 32) * 32 * -(-cols // 128) * 128
+    assert 0 <= held - w.nbytes - (6 * padded if planes else 0) < 32
+    x = np.random.default_rng(rows).standard_normal((40, cols)).astype(np.float32)
+    check(run(backend, x, w), x, w)
+
+
 @pytest.mark.parametrize("value,partner", [(2.0**-135, 2.0**80), (2.0**-125, 2.0**100), (2.0**-118, 2.0**60)])
 def test_tiny_weight_beside_ordinary_ones(backend, value, partner):
     """An element that the planes do not hold, in a row of ordinary ones, against
