@@ -22,6 +22,8 @@ namespace fah {
 namespace {
 
 typedef float floatx4 __attribute__((ext_vector_type(4)));
+// Four floats in one load from any float: frames may start anywhere.
+typedef float floatx4_any __attribute__((ext_vector_type(4), aligned(4)));
 
 // ---- GEMM: FP32 products on the bf16 matrix cores --------------------------------
 // out[f][n] = sum_k x[f][k] * w[n][k] (+ bias[n]) (ReLU), any M (frames), N, K.
@@ -151,13 +153,13 @@ __global__ __launch_bounds__(256) void f32_split_range_kernel(const float* __res
 }
 
 // Eight k of a row from k on, clamped into the row: what lies past K meets the
-// weight planes' zeros. VEC: K % 4 == 0 and 16-byte aligned rows.
+// weight planes' zeros. VEC: K % 4 == 0.
 template <bool VEC>
 __device__ __forceinline__ void load8(const float* row, int k, int K, float* v) {
   if (VEC) {
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
-      const float4 q = *reinterpret_cast<const float4*>(row + min(k + 4 * h, K - 4));
+      const floatx4 q = *reinterpret_cast<const floatx4_any*>(row + min(k + 4 * h, K - 4));
       v[4 * h] = q.x;
       v[4 * h + 1] = q.y;
       v[4 * h + 2] = q.z;
@@ -454,7 +456,7 @@ __global__ __launch_bounds__(64 * WN * KS) void f32_split_gemm_kernel(
 
 // ---- GEMM on fp32 MFMA: weights that the planes do not hold -----------------------
 // out[f][n] = sum_k x[f][k] * w[n][k] (+ bias[n]) (ReLU), any M (frames), N,
-// K with K % 4 == 0 and 16-byte aligned rows. Four waves in a 2 x 2 grid,
+// K with K % 4 == 0. Four waves in a 2 x 2 grid,
 // each a (16 BI) x (16 BJ) tile of v_mfma_f32_16x16x4f32 blocks; workgroup
 // tile (32 BI) x (32 BJ); K in tiles of GK staged in two LDS buffers as
 // row-major [row][GK + 4] (16-byte loads and stores; the next tile's global
@@ -490,13 +492,14 @@ __global__ __launch_bounds__(256) void f32_gemm_kernel(const float* __restrict__
   // the 16 bytes at k = 4 (t % PER_ROW) of the tile; rows past the edge and
   // k past K read as zero.
   const int lr = tid / PER_ROW, lc = 4 * (tid % PER_ROW);
-  float4 ra[LA], rb[LB];
+  floatx4 ra[LA];
+  float4 rb[LB];
   auto fetch = [&](int k0) {
     const int k = k0 + lc;
 #pragma unroll
     for (int u = 0; u < LA; ++u) {
       const int f = f0 + lr + ROWS * u;
-      ra[u] = (f < M && k < K) ? *reinterpret_cast<const float4*>(x + (size_t)f * K + k) : make_float4(0.f, 0.f, 0.f, 0.f);
+      ra[u] = (f < M && k < K) ? floatx4(*reinterpret_cast<const floatx4_any*>(x + (size_t)f * K + k)) : floatx4{0.f, 0.f, 0.f, 0.f};
     }
 #pragma unroll
     for (int u = 0; u < LB; ++u) {
@@ -506,7 +509,7 @@ __global__ __launch_bounds__(256) void f32_gemm_kernel(const float* __restrict__
   };
   auto stage = [&](int buf) {
 #pragma unroll
-    for (int u = 0; u < LA; ++u) *reinterpret_cast<float4*>(&a_s[buf][(lr + ROWS * u) * ROW + lc]) = ra[u];
+    for (int u = 0; u < LA; ++u) *reinterpret_cast<floatx4*>(&a_s[buf][(lr + ROWS * u) * ROW + lc]) = ra[u];
 #pragma unroll
     for (int u = 0; u < LB; ++u) *reinterpret_cast<float4*>(&b_s[buf][(lr + ROWS * u) * ROW + lc]) = rb[u];
   };
@@ -583,13 +586,14 @@ __global__ __launch_bounds__(256) void f32_gemm_wavek_kernel(const float* __rest
 #pragma unroll
     for (int j = 0; j < 4; ++j) acc[i][j] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
   const int lr = tid / PER_ROW, lc = 4 * (tid % PER_ROW);
-  float4 ra[LA], rb[LB];
+  floatx4 ra[LA];
+  float4 rb[LB];
   auto fetch = [&](int k0) {
     const int k = k0 + lc;
 #pragma unroll
     for (int u = 0; u < LA; ++u) {
       const int f = f0 + lr + ROWS * u;
-      ra[u] = (f < M && k < K) ? *reinterpret_cast<const float4*>(x + (size_t)f * K + k) : make_float4(0.f, 0.f, 0.f, 0.f);
+      ra[u] = (f < M && k < K) ? floatx4(*reinterpret_cast<const floatx4_any*>(x + (size_t)f * K + k)) : floatx4{0.f, 0.f, 0.f, 0.f};
     }
 #pragma unroll
     for (int u = 0; u < LB; ++u) {
@@ -599,7 +603,7 @@ __global__ __launch_bounds__(256) void f32_gemm_wavek_kernel(const float* __rest
   };
   auto stage = [&](int buf) {
 #pragma unroll
-    for (int u = 0; u < LA; ++u) *reinterpret_cast<float4*>(&a_s[buf][(lr + ROWS * u) * ROW + lc]) = ra[u];
+    for (int u = 0; u < LA; ++u) *reinterpret_cast<floatx4*>(&a_s[buf][(lr + ROWS * u) * ROW + lc]) = ra[u];
 #pragma unroll
     for (int u = 0; u < LB; ++u) *reinterpret_cast<float4*>(&b_s[buf][(lr + ROWS * u) * ROW + lc]) = rb[u];
   };
@@ -659,7 +663,7 @@ __global__ __launch_bounds__(256) void f32_gemm_wavek_kernel(const float* __rest
   }
 }
 
-// Any K and alignment: 64 x 64 tiles, K in steps of 32 staged in LDS one
+// Any K: 64 x 64 tiles, K in steps of 32 staged in LDS one
 // float per thread and row, four waves of 2 x 2 v_mfma_f32_16x16x4f32 blocks.
 constexpr int kGT = 64, kGA = 32, kGPad = kGA + 1;
 
@@ -720,21 +724,20 @@ __global__ __launch_bounds__(256) void f32_gemm_any_kernel(const float* __restri
 }
 
 // ---- GEMV (few frames, weight-bandwidth bound) ------------------------------
-// Each wave takes RW consecutive weight rows at a time, in chunks of 1,024 k
-// whose loads (16 values a lane and row) are all in flight together, with the
+// Each wave takes RW consecutive weight rows at a time, in chunks of 1,024 k (256
+// for rows of at most that: four frames of 3 -> 70000 46.5 -> 23.6 us)
+// whose loads (E values a lane and row) are all in flight together, with the
 // frames' values at the same k straight from the caches: a small launch is one
 // round of loads, with no LDS and no barrier before it (the frames staged in LDS
 // first, and 256 k a round: one frame of 1024 -> 3072 6.5 us, here 3.9, of 3072
 // -> 1024 9.1 and 3.8, both at what a call costs the host; 1024 -> 151936 113 and
 // 106, 5.9 TB/s). Then a wave reduction per row and frame. VEC: 16-byte loads (K
 // % 4 == 0); frames may start at any float, with the same order of the sum.
-typedef float floatx4_any __attribute__((ext_vector_type(4), aligned(4)));
-
-template <int MF, int RW, bool VEC>
+template <int MF, int RW, bool VEC, int E>
 __global__ __launch_bounds__(256) void f32_gemv_kernel(const float* __restrict__ x, const float* __restrict__ w,
                                                        const float* __restrict__ bias, float* __restrict__ out, int M,
                                                        int N, int K, int relu) {
-  constexpr int kChunk = 1024, E = kChunk / 64;
+  constexpr int kChunk = 64 * E;
   const int lane = threadIdx.x & 63, waves = gridDim.x * 4;
   // Value e of this lane: k0 + at(e); with `all`, the whole chunk lies in the row.
   auto load = [&](const float* row, int k0, bool all, float* v) {
@@ -1347,8 +1350,8 @@ bool f32_attention_supported(int frames, int width, int heads) {
 }
 
 // Weights of fewer columns have no planes: padded to 128 k they would take more
-// than 3 times the values' memory.
-constexpr int kSplitLeastK = 64;
+// than six times the values' memory.
+constexpr int kSplitLeastK = 32;
 
 // An FP32 weight's values, then the range check's word.
 static size_t outside_offset(int64_t rows, int cols) { return ((size_t)rows * cols * 4 + 15) & ~(size_t)15; }
@@ -1377,8 +1380,7 @@ hipError_t launch_f32_split(float* w, int64_t rows, int cols, void* planes, hipS
 // The GEMM on fp32 MFMA.
 static hipError_t launch_f32_gemm(const float* x, const float* w, const float* bias, float* out, int M, int N, int K,
                                   bool relu, hipStream_t s) {
-  const bool aligned = K % 4 == 0 && reinterpret_cast<uintptr_t>(x) % 16 == 0;
-  if (!aligned) {
+  if (K % 4 != 0) {
     const dim3 grid((N + kGT - 1) / kGT, (M + kGT - 1) / kGT);
     f32_gemm_any_kernel<<<grid, 256, 0, s>>>(x, w, bias, out, M, N, K, relu);
     return hipGetLastError();
@@ -1401,17 +1403,24 @@ static hipError_t launch_f32_gemm(const float* x, const float* w, const float* b
 hipError_t launch_f32_linear(const float* x, const float* w, const void* weight_planes, const float* bias, float* out,
                              int M, int N, int K, bool relu, hipStream_t s) {
   if (M < 1 || N < 1 || K < 1) return hipErrorInvalidValue;
-  if (M <= 4 || (M <= 8 && N <= 8192)) {
+  // Up to four frames the GEMV is quicker at every size, from five on while its
+  // waves (a row each) all run at once and a GEMM's K chain is longer. Measured
+  // with five and eight frames, us (GEMV, GEMM): 1024 -> 3072 5.3 7.0, 8.4; 1024
+  // -> 4096 6.6 8.9, 8.5; 2048 -> 5000 13.4 16.9, 13.6; 512 -> 3072 4.3 5.8, 6.1; 512 ->
+  // 3500 6.1 8.1, 6.4; 192 -> 2048 3.8 4.8, 5.1; 128 -> 2048 3.9 4.9, 4.4; 64 -> 512
+  // 3.7 4.7, 3.6.
+  if (M <= 4 || (M <= 8 && (N <= 3072 ? K >= 192 || M == 5 : (int64_t)M * N <= (K >= 1024 ? 30720 : K >= 512 ? 20480 : 0)))) {
     // One row a wave; four (fewer reads of the frames' values) only where they
-    // still leave the chip many rounds of waves. Measured, us (one row, four rows,
-    // GEMM): 1024 -> 3072, one frame 3.9 4.1 8.3; 1024 -> 151936, one 108 106 162,
-    // four 178 145 164; eight frames of 1024 -> 2048 6.2 11.2 8.6, of 1024 ->
-    // 20000 37.6 37.8 23.1; sixteen of 1024 -> 2048 9.5 31 9.0.
+    // still leave the chip many rounds of waves. Measured, us (one row, four
+    // rows): 1024 -> 3072, one frame 3.9 4.1; 1024 -> 151936, one 108 106, four
+    // 178 145; 1024 -> 20000, eight 37.6 37.8 (GEMM 23.1); 1024 -> 2048, sixteen 9.5
+    // 31 (GEMM 9.0).
 #define FAH_GEMV(MF, RW)                                                                                        \
   do {                                                                                                          \
     const int groups = std::min((N + 4 * RW - 1) / (4 * RW), 2048);                                             \
-    if (K % 4 == 0) f32_gemv_kernel<MF, RW, true><<<groups, 256, 0, s>>>(x, w, bias, out, M, N, K, relu);              \
-    else f32_gemv_kernel<MF, RW, false><<<groups, 256, 0, s>>>(x, w, bias, out, M, N, K, relu);                 \
+    const auto kernel = K <= 256 ? (K % 4 ? f32_gemv_kernel<MF, RW, false, 4> : f32_gemv_kernel<MF, RW, true, 4>) \
+                                 : (K % 4 ? f32_gemv_kernel<MF, RW, false, 16> : f32_gemv_kernel<MF, RW, true, 16>); \
+    kernel<<<groups, 256, 0, s>>>(x, w, bias, out, M, N, K, relu);                                               \
   } while (0)
     const bool many = N >= 65536;
     if (M == 1) {
@@ -1426,13 +1435,21 @@ hipError_t launch_f32_linear(const float* x, const float* w, const void* weight_
 #undef FAH_GEMV
     return hipGetLastError();
   }
-  if (!weight_planes) return launch_f32_gemm(x, w, bias, out, M, N, K, relu, s);
-  const bool vec = K % 4 == 0 && reinterpret_cast<uintptr_t>(x) % 16 == 0;
+  // With planes, fp32 MFMA all the same where the call is bound by a large
+  // weight's bytes (planes are 1.5 times as many), or by the launch and the first
+  // loads of a few K steps. Measured, us (planes, fp32): 16 frames of 1024 -> 50000
+  // 60.6 49.1, of 1024 -> 20000 23.5 25.1, 20 of 256 -> 30000 13.3 9.2, 64 of 1024
+  // -> 50000 64 87; 333 x 192 -> 1100 7.4 5.8, 1000 x 128 -> 512 6.0 4.9, 64 x 64 ->
+  // 2048 5.6 3.8, 64 x 224 -> 1100 6.5 6.4, 9 x 192 -> 2048 4.8 5.4, 2000 x 192 -> 2048
+  // 16.7 24.3. (Odd K has no such tile: 333 x 65 -> 512 6.3 10.2.)
+  const bool tall = M <= 32 && N >= 28672, narrow = K <= 64 ? (int64_t)M * N <= 4000000 : K <= 192 && M > 16 && (int64_t)M * N <= 2100000;
+  if (!weight_planes || (K % 4 == 0 && (tall || narrow)))
+    return launch_f32_gemm(x, w, bias, out, M, N, K, relu, s);
   const uint4* planes = static_cast<const uint4*>(weight_planes);
   const auto tiles = [&](int tm, int tn) { return ((M + tm - 1) / tm) * ((N + tn - 1) / tn); };
-  const auto run = [&](auto aligned, auto unaligned, int grid, int threads) {
-    if (vec) aligned<<<grid, threads, 0, s>>>(x, w, planes, bias, out, M, N, K, relu);
-    else unaligned<<<grid, threads, 0, s>>>(x, w, planes, bias, out, M, N, K, relu);
+  const auto run = [&](auto whole, auto any, int grid, int threads) {
+    if (K % 4 == 0) whole<<<grid, threads, 0, s>>>(x, w, planes, bias, out, M, N, K, relu);
+    else any<<<grid, threads, 0, s>>>(x, w, planes, bias, out, M, N, K, relu);
   };
 #define FAH_SPLIT(WN, KS, TI, TJ, KB, D)                                                                     \
   run(f32_split_gemm_kernel<WN, KS, TI, TJ, KB, D, true>, f32_split_gemm_kernel<WN, KS, TI, TJ, KB, D, false>, \

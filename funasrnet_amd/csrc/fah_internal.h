@@ -260,8 +260,8 @@ size_t f32_planes_bytes(int64_t rows, int cols);
 const int* f32_weight_outside(const float* w, int64_t rows, int cols);
 hipError_t launch_f32_split(float* w, int64_t rows, int cols, void* planes, hipStream_t s);
 // FP32 projections y[M][N] = x[M][K] W[N][K]^T (+ bias) (ReLU): products of
-// bf16 planes on MFMA, fp32 MFMA for a weight without planes (nullptr), or a
-// GEMV for up to 4 frames (8 of up to 8192 rows).
+// bf16 planes on MFMA, fp32 MFMA for a weight without planes (nullptr) and for
+// sizes that are quicker so, or a GEMV for up to 4 frames (8 where that is quicker).
 hipError_t launch_f32_linear(const float* x, const float* w, const void* planes, const float* bias, float* out, int M,
                              int N, int K, bool relu, hipStream_t s);
 // Non-causal multi-head attention over [frames][width] rows (head size

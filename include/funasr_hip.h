@@ -142,7 +142,7 @@ int fah_weight_q8_upload_blocks(fah_context* context, const uint8_t* blocks, int
 int fah_weight_f32_upload(fah_context* context, const float* values, int rows, int cols, fah_weight** out);
 int fah_weight_release(fah_weight* weight);
 /* Device bytes held by the weight (int8 plane plus scale plane; an FP32
- * weight's values, and for 64 columns or more their bf16 planes, one and a half
+ * weight's values, and for 32 columns or more their bf16 planes, one and a half
  * times as large, if there is memory for them and they hold the values exactly). */
 int64_t fah_weight_device_bytes(const fah_weight* weight);
 
@@ -176,9 +176,10 @@ int fah_quantized_linear_noalloc(fah_context* context, const float* input, int f
  * reference device version src/FunAsrNet.Vulkan/VulkanFloatBackend.cs:127-171):
  * output[frames*rows] = input[frames*cols] W^T (+ bias) for an FP32 weight,
  * on the matrix cores with fp32 sums (each value split exactly into three bf16
- * planes, or fp32 MFMA where a weight has none: below 64 columns, or with values
- * above 2^20, or below 2^-100 but not 0, or rows below 2^-80), or a
- * bandwidth-bound GEMV for up to 4 frames (8 of up to 8192 rows). Declines
+ * planes, or fp32 MFMA where a weight has none: below 32 columns, or with values
+ * above 2^20, or below 2^-100 but not 0, or rows below 2^-80; and for sizes
+ * that are quicker so), or a bandwidth-bound GEMV for up to 4 frames (8 where
+ * that is quicker). Declines
  * (output untouched) Q8_0 weights and projections below the minimum
  * operations. Float order differs from the CPU kernels, as the reference's
  * own device path does (its check: 2e-4 x max(1, |expected|)). The encoder's

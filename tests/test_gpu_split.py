@@ -43,11 +43,26 @@ def test_split_tiles(backend, frames, cols, rows, biased):
     check(run(backend, x, w, b), x, w, b)
 
 
+# The same tiles above 192 columns and at odd widths, and either side of the sizes
+# that fp32 MFMA takes: up to 64 columns and 4,000,000 results, up to 192 and
+# 2,100,000 from 17 frames on, and up to 32 frames of 28,672 rows or more.
+@pytest.mark.parametrize("frames,cols,rows", [(9, 193, 33), (31, 200, 31), (33, 257, 33), (64, 260, 65), (511, 196, 500),
+                                              (513, 225, 511), (1023, 196, 1793), (2100, 199, 1100), (17, 65, 40),
+                                              (16, 192, 31), (17, 192, 31), (1000, 192, 2100), (1001, 192, 2100),
+                                              (2000, 64, 2000), (2001, 64, 2000), (32, 196, 28672), (33, 196, 28672)])
+def test_gemm_choice(backend, frames, cols, rows):
+    rng = np.random.default_rng(cols)
+    x = rng.standard_normal((frames, cols)).astype(np.float32)
+    w = rng.standard_normal((rows, cols)).astype(np.float32)
+    check(run(backend, x, w), x, w)
+
+
 # The GEMV of one, up to four and up to eight frames: parts of a chunk of 1,024 k,
 # aligned and not, and the row counts where four rows a wave and the GEMM begin.
 @pytest.mark.parametrize("frames,cols,rows", [(1, 1, 1), (1, 63, 5), (1, 1023, 9), (1, 1028, 65537), (2, 4, 3),
                                               (3, 1025, 70), (4, 2052, 65541), (5, 1024, 6), (7, 67, 8192), (8, 5000, 33),
-                                              (8, 64, 8193), (1, 6148, 11)])
+                                              (8, 64, 8193), (1, 6148, 11), (1, 255, 9), (2, 256, 66000), (4, 260, 33),
+                                              (8, 192, 3072), (6, 191, 20), (5, 512, 4096), (8, 1024, 3841), (6, 516, 3073)])
 def test_gemv(backend, frames, cols, rows):
     rng = np.random.default_rng(cols)
     x = rng.standard_normal((frames, cols)).astype(np.float32)
@@ -126,7 +141,7 @@ def test_fp32_tiles(backend, frames, cols, rows, biased):
     check(run(backend, x, w, b), x, w, b)
 
 
-@pytest.mark.parametrize("rows,cols,value,planes", [(300, 63, 1.0, False), (300, 64, 1.0, True), (70, 500, 1.0, True),
+@pytest.mark.parametrize("rows,cols,value,planes", [(300, 31, 1.0, False), (300, 32, 1.0, True), (70, 500, 1.0, True),
                                                     (70, 500, 2.0**21, False), (1, 1, 1.0, False)])
 def test_planes_memory(backend, rows, cols, value, planes):
     """Planes are kept only where products use them: three bf16 a value, rows to 32, columns to 128."""
