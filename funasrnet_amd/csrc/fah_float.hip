@@ -17,6 +17,7 @@
 #include <algorithm>
 #include <cmath>
 #include <cstdint>
+#include <type_traits>
 
 namespace fah {
 namespace {
@@ -921,9 +922,16 @@ __global__ __launch_bounds__(256) void f32_attention_kernel(const float* __restr
 // lane group g multiplies channel g HS/4 + t), so that lane (query j, group
 // g) holds the probabilities of keys 4g .. 4g + 3 for query j, which is
 // exactly the A operand of P V when substep u takes key 4g + u.
+//
+// attention_tile_f32 does T such tiles, from query t0 on, with one read of the keys
+// and values. AHEAD: the next block's are on their way while a block is multiplied,
+// for a workgroup that has a CU to itself. A block's loads are without a branch
+// (keys past the end repeat the last one): with one for each row the compiler
+// waited for them all before the first product (333 frames of 4 x 128 18.8 ->
+// 15.8 us, 500 of 8 x 64 15.9 -> 13.1; the same bits).
 constexpr int attention_tile_bytes(int HS) { return (64 * HS + 128) * 4; }
 
-template <int HS>
+template <int HS, int T, bool AHEAD>
 __device__ __forceinline__ void attention_tile_f32(char* smem, const float* __restrict__ q, const float* __restrict__ k,
                                                    const float* __restrict__ v, float* __restrict__ out, int frames,
                                                    int width, float divisor, int head, int t0) {
@@ -933,114 +941,167 @@ __device__ __forceinline__ void attention_tile_f32(char* smem, const float* __re
   float(*l_s)[16] = m_s + 4;
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, j = lane & 15, g = lane >> 4;
   const int hoff = head * HS;
-  // This lane's query channels g KQ .. g KQ + KQ - 1 of query t0 + j (zero past the end).
-  float qv[KQ];
-  {
-    const bool in = t0 + j < frames;
-    const float* src = q + (size_t)(t0 + j) * width + hoff + g * KQ;
+  // This lane's query channels g KQ .. g KQ + KQ - 1 of query t0 + 16 i + j (zero past the end).
+  float qv[T][KQ];
+#pragma unroll
+  for (int i = 0; i < T; ++i) {
+    const bool in = t0 + 16 * i + j < frames;
+    const float* src = q + (size_t)(t0 + 16 * i + j) * width + hoff + g * KQ;
 #pragma unroll
     for (int c = 0; c < KQ; c += 4) {
       const float4 x4 = in ? *reinterpret_cast<const float4*>(src + c) : make_float4(0.f, 0.f, 0.f, 0.f);
-      qv[c] = x4.x;
-      qv[c + 1] = x4.y;
-      qv[c + 2] = x4.z;
-      qv[c + 3] = x4.w;
+      qv[i][c] = x4.x;
+      qv[i][c + 1] = x4.y;
+      qv[i][c + 2] = x4.z;
+      qv[i][c + 3] = x4.w;
     }
   }
-  floatx4 o[CB];
+  floatx4 o[T][CB];
+  float run_m[T], run_l[T];  // of query j
 #pragma unroll
-  for (int c = 0; c < CB; ++c) o[c] = floatx4{0.f, 0.f, 0.f, 0.f};
-  float run_m = -__builtin_inff(), run_l = 0.0f;  // of query j
+  for (int i = 0; i < T; ++i) {
+#pragma unroll
+    for (int c = 0; c < CB; ++c) o[i][c] = floatx4{0.f, 0.f, 0.f, 0.f};
+    run_m[i] = -__builtin_inff();
+    run_l[i] = 0.0f;
+  }
   const int blocks = (frames + 15) / 16;
-  float kv[KQ];
-  auto load_k = [&](int kb) {
-    const int key = kb * 16 + j;
-    const bool in = key < frames;
-    const float* src = k + (size_t)key * width + hoff + g * KQ;
+  // Keys past the end repeat the last one: their scores are not used, and their
+  // values become zero in `outputs`.
+  auto load_k = [&](float* b, int kb) {
+    const float* src = k + (size_t)min(kb * 16 + j, frames - 1) * width + hoff + g * KQ;
 #pragma unroll
     for (int c = 0; c < KQ; c += 4) {
-      const float4 x4 = in ? *reinterpret_cast<const float4*>(src + c) : make_float4(0.f, 0.f, 0.f, 0.f);
-      kv[c] = x4.x;
-      kv[c + 1] = x4.y;
-      kv[c + 2] = x4.z;
-      kv[c + 3] = x4.w;
+      const float4 x4 = *reinterpret_cast<const float4*>(src + c);
+      b[c] = x4.x;
+      b[c + 1] = x4.y;
+      b[c + 2] = x4.z;
+      b[c + 3] = x4.w;
     }
   };
-  if (wave < blocks) load_k(wave);
-  for (int kb = wave; kb < blocks; kb += 4) {
-    // Scores S^T[key 4g + r][query j].
-    floatx4 st = floatx4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int t = 0; t < KQ; ++t) st = __builtin_amdgcn_mfma_f32_16x16x4f32(kv[t], qv[t], st, 0, 0, 0);
-    // V values of keys 4g + u, channel 16c + j (zero past the end), and the
-    // next block's keys, in flight during the softmax.
-    float vv[CB][4];
+  // Values of keys 4g + u, channel 16c + j.
+  auto load_v = [&](float (*b)[4], int kb) {
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
-      const int key = kb * 16 + 4 * g + u;
-      const bool in = key < frames;
-      const float* src = v + (size_t)key * width + hoff + j;
+      const float* src = v + (size_t)min(kb * 16 + 4 * g + u, frames - 1) * width + hoff + j;
 #pragma unroll
-      for (int c = 0; c < CB; ++c) vv[c][u] = in ? src[16 * c] : 0.0f;
+      for (int c = 0; c < CB; ++c) b[c][u] = src[16 * c];
     }
-    if (kb + 4 < blocks) load_k(kb + 4);
-    float sc[4], bm = -__builtin_inff();
+  };
+  // Scores S^T[key 4g + r][query j].
+  auto products = [&](const float* b, floatx4* st) {
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int key = kb * 16 + 4 * g + r;
-      sc[r] = key < frames ? st[r] / divisor : -__builtin_inff();
-      bm = fmaxf(bm, sc[r]);
+    for (int i = 0; i < T; ++i) st[i] = floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int t = 0; t < KQ; ++t)
+#pragma unroll
+      for (int i = 0; i < T; ++i) st[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(b[t], qv[i][t], st[i], 0, 0, 0);
+  };
+  float p[T][4], alpha[T];
+  auto softmax = [&](const floatx4* st, int kb) {
+#pragma unroll
+    for (int i = 0; i < T; ++i) {
+      float sc[4], bm = -__builtin_inff();
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        sc[r] = (kb * 16 + 4 * g + r < frames ? st[i][r] : -__builtin_inff()) / divisor;
+        bm = fmaxf(bm, sc[r]);
+      }
+      bm = fmaxf(bm, __shfl_xor(bm, 16, 64));
+      bm = fmaxf(bm, __shfl_xor(bm, 32, 64));
+      const float nm = fmaxf(run_m[i], bm);
+      float bl = 0.0f;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        p[i][r] = sc[r] == -__builtin_inff() ? 0.0f : expf(sc[r] - nm);
+        bl += p[i][r];
+      }
+      bl += __shfl_xor(bl, 16, 64);
+      bl += __shfl_xor(bl, 32, 64);
+      alpha[i] = run_m[i] == -__builtin_inff() ? 0.0f : expf(run_m[i] - nm);
+      run_l[i] = run_l[i] * alpha[i] + bl;
+      run_m[i] = nm;
     }
-    bm = fmaxf(bm, __shfl_xor(bm, 16, 64));
-    bm = fmaxf(bm, __shfl_xor(bm, 32, 64));
-    const float nm = fmaxf(run_m, bm);
-    float p[4], bl = 0.0f;
+  };
+  auto outputs = [&](float (*b)[4], int kb) {
+    if (kb == blocks - 1) {
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      p[r] = sc[r] == -__builtin_inff() ? 0.0f : expf(sc[r] - nm);
-      bl += p[r];
+      for (int u = 0; u < 4; ++u)
+#pragma unroll
+        for (int c = 0; c < CB; ++c) b[c][u] = kb * 16 + 4 * g + u < frames ? b[c][u] : 0.0f;
     }
-    bl += __shfl_xor(bl, 16, 64);
-    bl += __shfl_xor(bl, 32, 64);
-    const float alpha = run_m == -__builtin_inff() ? 0.0f : expf(run_m - nm);
-    run_l = run_l * alpha + bl;
-    run_m = nm;
-    // Output rows are queries 4g + r: their rescale factors from lanes 4g + r.
-    float ar[4];
 #pragma unroll
-    for (int r = 0; r < 4; ++r) ar[r] = __shfl(alpha, 4 * g + r, 64);
+    for (int i = 0; i < T; ++i) {
+      // Output rows are queries 4g + r: their rescale factors from lanes 4g + r.
+      float ar[4];
 #pragma unroll
-    for (int c = 0; c < CB; ++c) {
+      for (int r = 0; r < 4; ++r) ar[r] = __shfl(alpha[i], 4 * g + r, 64);
 #pragma unroll
-      for (int r = 0; r < 4; ++r) o[c][r] *= ar[r];
+      for (int c = 0; c < CB; ++c)
 #pragma unroll
-      for (int u = 0; u < 4; ++u) o[c] = __builtin_amdgcn_mfma_f32_16x16x4f32(p[u], vv[c][u], o[c], 0, 0, 0);
+        for (int r = 0; r < 4; ++r) o[i][c][r] *= ar[r];
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+#pragma unroll
+        for (int c = 0; c < CB; ++c) o[i][c] = __builtin_amdgcn_mfma_f32_16x16x4f32(p[i][u], b[c][u], o[i][c], 0, 0, 0);
+    }
+  };
+  const int last = blocks - 1;
+  floatx4 st[T];
+  float k0[KQ], v0[CB][4];
+  load_k(k0, min(wave, last));
+  if (AHEAD) {
+    float k1[KQ], v1[CB][4];
+    load_v(v0, min(wave, last));
+    auto step = [&](float* kb0, float (*vb0)[4], float* kb1, float (*vb1)[4], int kb) {
+      load_k(kb1, min(kb + 4, last));
+      load_v(vb1, min(kb + 4, last));
+      __builtin_amdgcn_sched_barrier(0);
+      products(kb0, st);
+      softmax(st, kb);
+      outputs(vb0, kb);
+    };
+    for (int kb = wave; kb < blocks; kb += 8) {
+      step(k0, v0, k1, v1, kb);
+      if (kb + 4 < blocks) step(k1, v1, k0, v0, kb + 4);
+    }
+  } else {
+    for (int kb = wave; kb < blocks; kb += 4) {
+      products(k0, st);
+      load_v(v0, kb);  // (in flight during the softmax)
+      load_k(k0, min(kb + 4, last));
+      softmax(st, kb);
+      outputs(v0, kb);
     }
   }
   // Merge the four waves' partials: out = sum_w e^(m_w - M) O_w / sum_w e^(m_w - M) l_w.
-  if (g == 0) {
-    m_s[wave][j] = run_m;
-    l_s[wave][j] = run_l;
-  }
 #pragma unroll
-  for (int c = 0; c < CB; ++c)
-#pragma unroll
-    for (int r = 0; r < 4; ++r) o_s[wave][4 * g + r][16 * c + j] = o[c][r];
-  __syncthreads();
-  for (int e = tid; e < 16 * HS; e += 256) {
-    const int row = e / HS, ch = e % HS;
-    if (t0 + row >= frames) continue;
-    float mx = -__builtin_inff();
-#pragma unroll
-    for (int w2 = 0; w2 < 4; ++w2) mx = fmaxf(mx, m_s[w2][row]);
-    float num = 0.0f, den = 0.0f;
-#pragma unroll
-    for (int w2 = 0; w2 < 4; ++w2) {
-      const float f = m_s[w2][row] == -__builtin_inff() ? 0.0f : expf(m_s[w2][row] - mx);
-      num += f * o_s[w2][row][ch];
-      den += f * l_s[w2][row];
+  for (int i = 0; i < T; ++i) {
+    if (T > 1) __syncthreads();
+    if (g == 0) {
+      m_s[wave][j] = run_m[i];
+      l_s[wave][j] = run_l[i];
     }
-    out[(size_t)(t0 + row) * width + hoff + ch] = num / den;
+#pragma unroll
+    for (int c = 0; c < CB; ++c)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) o_s[wave][4 * g + r][16 * c + j] = o[i][c][r];
+    __syncthreads();
+    for (int e = tid; e < 16 * HS; e += 256) {
+      const int row = e / HS, ch = e % HS, f = t0 + 16 * i + row;
+      if (f >= frames) continue;
+      float mx = -__builtin_inff();
+#pragma unroll
+      for (int w2 = 0; w2 < 4; ++w2) mx = fmaxf(mx, m_s[w2][row]);
+      float num = 0.0f, den = 0.0f;
+#pragma unroll
+      for (int w2 = 0; w2 < 4; ++w2) {
+        const float x = m_s[w2][row] == -__builtin_inff() ? 0.0f : expf(m_s[w2][row] - mx);
+        num += x * o_s[w2][row][ch];
+        den += x * l_s[w2][row];
+      }
+      out[(size_t)f * width + hoff + ch] = num / den;
+    }
   }
 }
 
@@ -1050,7 +1111,7 @@ __global__ __launch_bounds__(256) void f32_attention_mfma_kernel(const float* __
                                                                  const float* __restrict__ v, float* __restrict__ out,
                                                                  int frames, int width, float divisor) {
   __shared__ __attribute__((aligned(16))) char smem[attention_tile_bytes(HS)];
-  attention_tile_f32<HS>(smem, q, k, v, out, frames, width, divisor, blockIdx.x, blockIdx.y * 16);
+  attention_tile_f32<HS, 1, false>(smem, q, k, v, out, frames, width, divisor, blockIdx.x, blockIdx.y * 16);
 }
 
 // ---- Non-causal multi-head attention on the bf16 matrix cores (head size 64, 96, 128) ----
@@ -1085,7 +1146,14 @@ __global__ __launch_bounds__(256) void f32_attention_mfma_kernel(const float* __
 // 64 bits 7.2e-7 -> 4.1e-7 (4096), 5.0e-7 -> 1.7e-7 (1000).
 //
 // Values outside [2^-100, 2^60] in magnitude, but zero, set the head's word in
-// `outside` (so do infinities and NaN); its tiles run on fp32 MFMA.
+// `outside` (so do infinities and NaN); its queries run on fp32 MFMA, dealt over
+// the shares. A workgroup then has the CU to itself, and an attention call takes, us,
+// with all heads outside (as attention_tile_f32 in a launch of its own, and with
+// four tiles in turn by share 0): 400 frames of 4 x 128 39.5 (20.8, 85), 576 32.5
+// (25, 103), 1000 46.7 (40, 164), 1864 114 (133, 293), 4096 408 (569, 611); 640 of 8
+// x 64 32 (25, 75), 1068 79 (54, 116), 2500 273 (198, 366). What is left is the planes'
+// launch and one wave a SIMD. Scores of the next block beside the softmax of this
+// one, or keys read 64 bytes a row and load, took the same times.
 constexpr uint32_t kPlaneMost = 0x5d800000u;  // 2^60
 constexpr float kSlack = 8.0f;
 constexpr int kSplitQ = 64;  // queries a workgroup
@@ -1208,12 +1276,14 @@ __global__ __launch_bounds__(256, 1) void attention_split_kernel(SplitAttnArgs a
   }
   // (The operands are on their way meanwhile.)
   if (outside == a.epoch) {
-    if (share == 0)
-      for (int t = 0; t < kSplitQ && q0 + t < a.frames; t += 16)
-      {
-        __syncthreads();
-        attention_tile_f32<HS>(attn_split_s, a.q, a.k, a.v, a.out, a.frames, a.width, a.divisor, head, q0 + t);
-      }
+    // One share: all 64 queries with one read of the keys; else 32 or 16 a share.
+    const auto queries = [&](auto tiles, int first) {
+      if (first < kSplitQ && q0 + first < a.frames)
+        attention_tile_f32<HS, tiles, true>(attn_split_s, a.q, a.k, a.v, a.out, a.frames, a.width, a.divisor, head, q0 + first);
+    };
+    if (a.shares == 1) queries(std::integral_constant<int, 4>{}, 0);
+    else if (a.shares < 4) queries(std::integral_constant<int, 2>{}, 32 * share);
+    else queries(std::integral_constant<int, 1>{}, 16 * share);
     return;
   }
   constexpr int pa[6] = {2, 0, 1, 0, 1, 0}, pb[6] = {0, 2, 1, 0, 0, 1};

@@ -189,6 +189,22 @@ def test_split_attention(backend, oracle_lib, frames, heads, size):
     assert np.abs(attend(backend, q, k, v, heads) - expected).max() <= 5e-5 * 4
 
 
+# One, two, three and four key shares, of which each takes queries of its own here.
+@pytest.mark.parametrize("frames,heads,size", [(65, 8, 96), (1068, 8, 64), (1400, 4, 128), (449, 3, 128), (400, 3, 128), (1001, 3, 128)])
+def test_split_attention_range_shares(backend, oracle_lib, frames, heads, size):
+    """Heads that the planes do not hold, for a large value, a tiny query and an infinite value of the last key."""
+    rng = np.random.default_rng(frames)
+    width = heads * size
+    q, k, v = (rng.uniform(-2, 2, (frames, width)).astype(np.float32) for _ in range(3))
+    v[5, 3] = 2.0**70
+    q[frames // 2, size + 2] = 2.0**-101
+    expected = oracle_lib.attention_f64(q, k, v, frames, width, heads)
+    v[frames - 1, width - 1] = np.inf
+    got = attend(backend, q, k, v, heads)
+    assert np.all(got[:, -1] == np.inf)
+    assert np.all(np.abs(got - expected)[:, :-1] <= (5e-5 * np.maximum(4, np.abs(expected)))[:, :-1])
+
+
 @pytest.mark.parametrize("value", [2.0**-101, 2.0**70, np.inf, np.nan])
 def test_split_attention_range(backend, oracle_lib, value):
     """A value that the planes do not hold moves its head, and only it, to fp32."""
