@@ -176,7 +176,11 @@ def attend(backend, q, k, v, heads):
 
 # Tiles of 64 queries, blocks of 32 keys, one to four key shares; either side of
 # the lengths from which heads of 128 and 64 take the planes. The tolerance is the
-# reference's device check's (AttentionGpuChecks.cs), relative to values of 4.
+# reference's device check's (AttentionGpuChecks.cs), relative to values of 4. On the planes,
+# all rows but the peaked one together: 7e-7 (2-norm). The same products in numpy, added
+# exactly, are within 1.6e-7 (the kernel's fp32 sums 2.2e-7 to 4.5e-7), and off by
+# 9.8e-7 or more (33 frames on) without any one of the six, in the scores or in the
+# outputs.
 @pytest.mark.parametrize("frames,heads,size", [(1, 2, 96), (33, 1, 96), (63, 4, 96), (65, 8, 96), (399, 1, 128),
                                                (400, 4, 128), (449, 1, 128), (513, 3, 128), (1857, 4, 128),
                                                (640, 2, 64), (671, 8, 64), (1100, 8, 64)])
@@ -186,7 +190,11 @@ def test_split_attention(backend, oracle_lib, frames, heads, size):
     q, k, v = (rng.uniform(-s, s, (frames, width)).astype(np.float32) for s in (3, 3, 4))
     q[0] *= 8  # one peaked row
     expected = oracle_lib.attention_f64(q, k, v, frames, width, heads)
-    assert np.abs(attend(backend, q, k, v, heads) - expected).max() <= 5e-5 * 4
+    off = attend(backend, q, k, v, heads) - expected
+    assert np.abs(off).max() <= 5e-5 * 4
+    rest = slice(min(1, frames - 1), None)
+    if (frames, size) != (399, 128):  # (that one runs on fp32 MFMA, in longer fp32 sums)
+        assert np.linalg.norm(off[rest]) <= 7e-7 * np.linalg.norm(expected[rest])
 
 
 # One, two, three and four key shares, of which each takes queries of its own here.
