@@ -181,33 +181,50 @@ __device__ __forceinline__ void store_linear(float v, const float* bias, float* 
   }
 }
 
-// A TM x TN tile on fp32 MFMA, any K and alignment: K in steps of 32 staged in
-// LDS, one float per thread and row; wave w takes the 16 x 16 blocks w, w + WAVES,
-// ... Lane layout of 16x16x4: A[i][k] from lane i + 16k, B[k][j] from lane
-// j + 16k, D[4q + r][j] in lane j + 16q.
-template <int TM, int TN, int WAVES>
+// A TM x TN tile on fp32 MFMA: K in steps of 32 staged in LDS, the next step's
+// loads in registers meanwhile (one NaN in 1000 x 512 -> 2048 39 us, 89 with 4-byte
+// loads where they are used; in 4000 x 2048 -> 512 140 and 455; the fp32 GEMM for
+// all tiles 25 and 85); wave w takes the 16 x 16 blocks w, w + WAVES, ...
+// Lane layout of 16x16x4: A[i][k] from lane i + 16k, B[k][j] from lane j + 16k,
+// D[4q + r][j] in lane j + 16q. VEC: K % 4 == 0.
+template <int TM, int TN, int WAVES, bool VEC>
 __device__ __forceinline__ void tile_f32(char* smem, const float* x, const float* w, const float* bias, float* out, int M,
                                       int N, int K, int f0, int n0, bool relu) {
-  constexpr int PAD = 33, BLOCKS = (TM / 16) * (TN / 16), PER = BLOCKS / WAVES, NT = 64 * WAVES;
-  static_assert(BLOCKS % WAVES == 0, "whole blocks a wave");
+  constexpr int PAD = 33, BLOCKS = (TM / 16) * (TN / 16), PER = BLOCKS / WAVES, NT = 64 * WAVES, PIECES = (TM + TN) * 8 / NT;
+  static_assert(BLOCKS % WAVES == 0 && PIECES * NT == (TM + TN) * 8, "whole blocks a wave, whole pieces a thread");
   float* s = reinterpret_cast<float*>(smem);  // [TM + TN][PAD]
-  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, kc = 4 * (tid & 7);
+  // Thread t takes 4 k of every NT / 8th row from t / 8 on; rows past the end
+  // repeat the last one (never stored), k past the end become zeros in LDS.
+  float v[PIECES][4];
+  auto fetch = [&](int k) {
+#pragma unroll
+    for (int p = 0; p < PIECES; ++p) {
+      const int r = (tid + NT * p) >> 3;
+      const float* row = r < TM ? x + (size_t)min(f0 + r, M - 1) * K : w + (size_t)min(n0 + r - TM, N - 1) * K;
+      if (VEC) {
+        const floatx4 q = *reinterpret_cast<const floatx4_any*>(row + min(k, K - 4));
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[p][e] = q[e];
+      } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[p][e] = row[min(k + e, K - 1)];
+      }
+    }
+  };
   floatx4 acc[PER];
 #pragma unroll
   for (int b = 0; b < PER; ++b) acc[b] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+  fetch(kc);
   for (int k0 = 0; k0 < K; k0 += 32) {
     __syncthreads();
-    const int k = k0 + (tid & 31);
-    for (int r = tid >> 5; r < TM + TN; r += NT / 32) {
-      const int f = f0 + r, n = n0 + r - TM;
-      float v = 0.0f;
-      if (k < K) {
-        if (r < TM) v = f < M ? x[(size_t)f * K + k] : 0.0f;
-        else v = n < N ? w[(size_t)n * K + k] : 0.0f;
-      }
-      s[r * PAD + (tid & 31)] = v;
-    }
+#pragma unroll
+    for (int p = 0; p < PIECES; ++p)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) s[((tid + NT * p) >> 3) * PAD + kc + e] = k0 + kc + e < K ? v[p][e] : 0.0f;
     __syncthreads();
+    fetch(k0 + 32 + kc);
+#pragma unroll
     for (int ks = 0; ks < 32; ks += 4) {
       const int kk = ks + (lane >> 4);
 #pragma unroll
@@ -425,10 +442,33 @@ __global__ __launch_bounds__(64 * WN * KS) void f32_split_gemm_kernel(
 #pragma unroll
             for (int e = 0; e < 16; ++e) odd = odd || (f2u(acc[i][j][e]) & 0x7fffffffu) >= 0x7f800000u;
       }
-      // Sums of zero are right unless frames held values too small for the planes.
-      for (int row = wave; row < TM && f0 + row < M; row += WAVES)
-        for (int k = lane; k < K; k += 64)
-          odd = odd || (f2u(x[(size_t)(f0 + row) * K + k]) & 0x7fffffffu) - 1u < kSplitTiny - 1u;
+      if (__syncthreads_or(odd)) return false;
+      // Sums of zero (those of zero frames, as a padded batch has) are right unless
+      // frames held values too small for the planes: magnitudes less one again, a
+      // wave's TM / WAVES frames together. Half of 4000 x 2048 -> 512 zeros 63 us
+      // (137 with one load at a time), of 1000 x 512 -> 512 10.6 (20).
+      constexpr int FW = TM / WAVES, W = VEC ? 4 : 1;
+      uint32_t tiny = 0xffffffffu;
+#pragma unroll 1
+      for (int k = W * lane; k < K; k += 64 * W) {
+        float v[FW][W];
+#pragma unroll
+        for (int r = 0; r < FW; ++r) {
+          const float* row = x + (size_t)min(f0 + FW * wave + r, M - 1) * K + k;
+          if (VEC) {
+            const floatx4 q = *reinterpret_cast<const floatx4_any*>(row);
+#pragma unroll
+            for (int e = 0; e < W; ++e) v[r][e] = q[e];
+          } else {
+            v[r][0] = *row;
+          }
+        }
+#pragma unroll
+        for (int r = 0; r < FW; ++r)
+#pragma unroll
+          for (int e = 0; e < W; ++e) tiny = min(tiny, (f2u(v[r][e]) & 0x7fffffffu) - 1u);
+      }
+      odd = tiny < kSplitTiny - 1u;
       if (__syncthreads_or(odd)) return false;
     }
     if (ks == 0) {
@@ -452,7 +492,7 @@ __global__ __launch_bounds__(64 * WN * KS) void f32_split_gemm_kernel(
     }
     return true;
   };
-  if (!split_tile()) tile_f32<TM, TN, WAVES>(smem, x, w, bias, out, M, N, K, f0, n0, relu);
+  if (!split_tile()) tile_f32<TM, TN, WAVES, VEC>(smem, x, w, bias, out, M, N, K, f0, n0, relu);
 }
 
 // ---- GEMM on fp32 MFMA: weights that the planes do not hold -----------------------

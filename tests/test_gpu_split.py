@@ -92,17 +92,25 @@ def test_frames_at_any_float(backend, frames, cols, rows):
         assert np.array_equal(r.view(np.uint32), results[0].view(np.uint32))
 
 
+# (Up to 192 columns these run on fp32 MFMA, odd widths on the planes again.)
+@pytest.mark.parametrize("cols", [64, 65, 260, 517])
 @pytest.mark.parametrize("frames,rows", [(40, 70), (400, 700), (1100, 2100)])
-def test_split_range(backend, frames, rows):
+def test_split_range(backend, frames, cols, rows):
     """Zero frames, tiny and huge values, infinities and NaN."""
     rng = np.random.default_rng(rows)
-    x = rng.standard_normal((frames, 64)).astype(np.float32)
-    w = rng.standard_normal((rows, 64)).astype(np.float32)
+    x = rng.standard_normal((frames, cols)).astype(np.float32)
+    w = rng.standard_normal((rows, cols)).astype(np.float32)
     x[3] = 0.0
     check(run(backend, x, w), x, w)
     for scale in (2.0**-60, 2.0**-110, 2.0**-120, 2.0**100):
         scaled = x.copy()
         scaled[7] *= np.float32(scale)
+        check(run(backend, scaled, w), scaled, w)
+    # Values below the smallest bf16 give sums of zero on the planes.
+    for frame, col in ((7, 5), (frames - 1, cols - 1), (32, 0)):
+        scaled = x.copy()
+        scaled[frame] = 0.0
+        scaled[frame, col] = 2.0**-140
         check(run(backend, scaled, w), scaled, w)
     x[5, 2], x[6, 1], x[9, 0] = np.inf, np.nan, np.float32(3.4e38)
     w = w.copy()
