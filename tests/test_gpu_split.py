@@ -122,11 +122,12 @@ def test_split_range(backend, frames, cols, rows):
     assert np.all(np.isnan(got[6])) and np.array_equal(got[5], np.where(w[:, 2] < 0, -np.inf, np.inf).astype(np.float32))
 
 
+@pytest.mark.parametrize("cols", [100, 101, 196])
 @pytest.mark.parametrize("value", [2.0**21, 2.0**-90, np.inf])
-def test_weights_outside_the_planes(backend, value):
+def test_weights_outside_the_planes(backend, value, cols):
     rng = np.random.default_rng(1)
-    x = rng.standard_normal((200, 100)).astype(np.float32)
-    w = rng.standard_normal((130, 100)).astype(np.float32)
+    x = rng.standard_normal((200, cols)).astype(np.float32)
+    w = rng.standard_normal((130, cols)).astype(np.float32)
     w[4] = np.float32(value) * (np.sign(w[4]) if np.isfinite(value) else 1)
     got = run(backend, x, w)
     if np.isfinite(value):
@@ -163,13 +164,14 @@ def test_planes_memory(backend, rows, cols, value, planes):
     check(run(backend, x, w), x, w)
 
 
+@pytest.mark.parametrize("cols", [100, 101, 196])
 @pytest.mark.parametrize("value,partner", [(2.0**-135, 2.0**80), (2.0**-125, 2.0**100), (2.0**-118, 2.0**60)])
-def test_tiny_weight_beside_ordinary_ones(backend, value, partner):
+def test_tiny_weight_beside_ordinary_ones(backend, value, partner, cols):
     """An element that the planes do not hold, in a row of ordinary ones, against
     frames that are large there and zero elsewhere."""
     rng = np.random.default_rng(4)
-    x = rng.standard_normal((70, 100)).astype(np.float32)
-    w = rng.standard_normal((130, 100)).astype(np.float32)
+    x = rng.standard_normal((70, cols)).astype(np.float32)
+    w = rng.standard_normal((130, cols)).astype(np.float32)
     w[9, 6] = np.float32(value * 1.2345678)
     x[[3, 40]] = 0
     x[[3, 40], 6] = np.float32(partner)
