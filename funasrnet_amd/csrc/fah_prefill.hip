@@ -398,6 +398,162 @@ __global__ __launch_bounds__(64 * WF * WR) void q8_gemm_kernel(GemmArgs g) {
   }
 }
 
+// The same sums, plain outputs, for short rows and for large products with fp32
+// scales (gemm_is_short). A wave owns a (16 TR rows) x (16 TF frames) tile of
+// 16x16 MFMA tiles, a workgroup of 2 x 2 waves (32 TR) x (32 TF). Operands move
+// through LDS in stages of four blocks (128 bytes of every tile row, 16 bytes a
+// lane): the next stage's global loads are in flight in registers while the
+// current stage is computed, then written to the other LDS buffer. The 16-byte
+// chunk c of tile row t sits at slot c ^ (t & 7), so that the 16 rows of an MFMA
+// operand read spread over the banks. Bound by the launch and the first loads
+// for small products, by the ordered fp32 steps (four VALU operations a row,
+// frame and block) for large ones.
+constexpr int kGT = 256;  // threads per workgroup
+constexpr int kStageBlocks = 4;
+template <int TR, int TF>
+constexpr int kShortStage = (32 * TR + 32 * TF) * (32 + 4) * kStageBlocks;  // rows and frames, then their scales as fp32
+
+template <class Scale, int TR, int TF>
+__global__ __launch_bounds__(kGT) void q8_gemm_short_kernel(GemmArgs g) {
+  constexpr int RW = 16 * TR, FW = 16 * TF;  // wave tile
+  constexpr int RT = 2 * RW, FT = 2 * FW;    // workgroup tile
+  constexpr int kRowBytes = 32 * kStageBlocks, kOperandBytes = (RT + FT) * kRowBytes;
+  __shared__ __attribute__((aligned(16))) char stage_s[2][kShortStage<TR, TF>];
+  const int B = g.K >> 5;
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+  const int wr = wave & 1, wf = wave >> 1;
+  const int row0 = blockIdx.x * RT, f0 = blockIdx.y * FT;
+
+  // Stage loads: piece j of a stage is tile rows 8j..8j+7 (rows [0, RT) are
+  // weight rows, [RT, RT + FT) frames); lane l takes row 8j + l/8, chunk
+  // (l%8) ^ (row & 7), and writes it to slot l%8. Rows past the matrix and
+  // frames past the input load the first one, with a scale of 0: never stored.
+  constexpr int kPerWave = (RT + FT) / 32;
+  const int8_t* src[kPerWave];
+#pragma unroll
+  for (int i = 0; i < kPerWave; ++i) {
+    const int t = 8 * (wave + 4 * i) + (lane >> 3), chunk = (lane & 7) ^ (t & 7);
+    const int r = row0 + t, f = f0 + t - RT;
+    src[i] = (t < RT ? g.w + (size_t)(r < g.rows ? r : 0) * g.K : g.xq + (size_t)(f < g.frames ? f : 0) * g.K) + 16 * chunk;
+  }
+  // Scales of a stage: thread t takes block t % 4 of row t / 4 and of frame t / 4.
+  using ST = typename Scale::type;
+  static_assert(RT <= 64 && FT <= 64, "one row scale and one frame scale per thread");
+  const int sblk = tid & 3, srow = tid >> 2;
+  const bool row_live = srow < RT && row0 + srow < g.rows, frame_live = srow < FT && f0 + srow < g.frames;
+  const ST* wsrc = reinterpret_cast<const ST*>(g.ws) + (size_t)(row_live ? row0 + srow : 0) * B + sblk;
+  const float* xsrc = g.xs + (size_t)(frame_live ? f0 + srow : 0) * B + sblk;
+  v4i pending[kPerWave];
+  ST wraw;
+  float xraw;
+  auto fetch = [&](int st) {  // stage st: blocks [4 st, 4 st + 4)
+#pragma unroll
+    for (int i = 0; i < kPerWave; ++i) pending[i] = *reinterpret_cast<const v4i*>(src[i] + (size_t)st * kRowBytes);
+    wraw = wsrc[kStageBlocks * st];
+    xraw = xsrc[kStageBlocks * st];
+  };
+  auto put = [&](int st) {
+    char* base = stage_s[st & 1];
+#pragma unroll
+    for (int i = 0; i < kPerWave; ++i) *reinterpret_cast<v4i*>(base + (wave + 4 * i) * 1024 + 16 * lane) = pending[i];
+    float* sc = reinterpret_cast<float*>(base + kOperandBytes);  // [4][RT] rows, then [4][FT] frames
+    if (srow < RT) sc[sblk * RT + srow] = row_live ? Scale::get(wraw) : 0.0f;
+    if (srow < FT) sc[kStageBlocks * RT + sblk * FT + srow] = frame_live ? xraw : 0.0f;
+  };
+  const int stages = B / kStageBlocks;
+  fetch(0);
+  put(0);
+  fetch(min(1, stages - 1));
+  lds_barrier();
+
+  // MFMA operand of lane l: 8 bytes of row (frame) l % 16 at byte 8 (l / 16)
+  // of the block; result register j of lane l: row 4 (l / 16) + j, frame l % 16.
+  const int l16 = lane & 15, kq = lane >> 4;
+  int a_at[TR], b_at[TF];  // byte offsets of this lane's operand rows in a stage
+#pragma unroll
+  for (int tr = 0; tr < TR; ++tr) a_at[tr] = (wr * RW + 16 * tr + l16) * kRowBytes;
+#pragma unroll
+  for (int tf = 0; tf < TF; ++tf) b_at[tf] = (RT + wf * FW + 16 * tf + l16) * kRowBytes;
+  // Chunk 2 blk + kq/2 of row t sits at slot (2 blk + kq/2) ^ (t & 7); every
+  // operand row of this lane has t & 7 == l16 & 7.
+  auto at = [&](int row_at, int blk) { return row_at + 16 * ((2 * blk + (kq >> 1)) ^ (l16 & 7)) + 8 * (kq & 1); };
+  const v4i zero4 = {0, 0, 0, 0};
+  float acc[TR][TF][4];
+#pragma unroll
+  for (int tr = 0; tr < TR; ++tr)
+#pragma unroll
+    for (int tf = 0; tf < TF; ++tf)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) acc[tr][tf][j] = 0.0f;
+
+  for (int st = 0; st < stages; ++st) {
+    const char* sa = stage_s[st & 1];
+    const float* ws_s = reinterpret_cast<const float*>(sa + kOperandBytes);  // [4][RT]
+    const float* xs_s = ws_s + kStageBlocks * RT;                           // [4][FT]
+    // Four-tile waves keep two blocks in flight (fewer registers, more waves
+    // a SIMD); single-tile waves all four.
+    constexpr int kBlkUnroll = TR * TF >= 4 ? 2 : kStageBlocks;
+#pragma unroll kBlkUnroll
+    for (int blk = 0; blk < kStageBlocks; ++blk) {
+      long av[TR], bv[TF];
+#pragma unroll
+      for (int tr = 0; tr < TR; ++tr) av[tr] = *reinterpret_cast<const long*>(sa + at(a_at[tr], blk));
+#pragma unroll
+      for (int tf = 0; tf < TF; ++tf) bv[tf] = *reinterpret_cast<const long*>(sa + at(b_at[tf], blk));
+      v4i d[TR][TF];
+#pragma unroll
+      for (int tr = 0; tr < TR; ++tr)
+#pragma unroll
+        for (int tf = 0; tf < TF; ++tf) d[tr][tf] = __builtin_amdgcn_mfma_i32_16x16x32_i8(av[tr], bv[tf], zero4, 0, 0, 0);
+      // The reference's ((float)dot * w_scale) * x_scale, added in block order.
+      float4 w4[TR];
+      float xv[TF];
+#pragma unroll
+      for (int tr = 0; tr < TR; ++tr) w4[tr] = *reinterpret_cast<const float4*>(ws_s + blk * RT + wr * RW + 16 * tr + 4 * kq);
+#pragma unroll
+      for (int tf = 0; tf < TF; ++tf) xv[tf] = xs_s[blk * FT + wf * FW + 16 * tf + l16];
+#pragma unroll
+      for (int tr = 0; tr < TR; ++tr) {
+        const float w[4] = {w4[tr].x, w4[tr].y, w4[tr].z, w4[tr].w};
+#pragma unroll
+        for (int tf = 0; tf < TF; ++tf)
+#pragma unroll
+          for (int j = 0; j < 4; ++j) acc[tr][tf][j] = fadd(acc[tr][tf][j], fmul(fmul((float)d[tr][tf][j], w[j]), xv[tf]));
+      }
+    }
+    // Stage st + 1 into the other buffer (last read at stage st - 1, before
+    // the previous barrier), then stage st + 2's loads into the registers
+    // (past the last stage: the last one again, unused).
+    put(st + 1);
+    fetch(min(st + 2, stages - 1));
+    lds_barrier();
+  }
+
+#pragma unroll
+  for (int tf = 0; tf < TF; ++tf) {
+    const int f = f0 + wf * FW + 16 * tf + l16;
+    if (f >= g.frames) continue;
+#pragma unroll
+    for (int tr = 0; tr < TR; ++tr) {
+      const int r = row0 + wr * RW + 16 * tr + 4 * kq;
+      float v[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        v[j] = acc[tr][tf][j];
+        if (g.bias && r + j < g.rows) v[j] = fadd(g.bias[r + j], v[j]);
+      }
+      float* o = g.out + (size_t)f * g.out_stride + r;
+      if (r + 3 < g.rows && ((g.out_stride | r) & 3) == 0) {
+        *reinterpret_cast<float4*>(o) = make_float4(v[0], v[1], v[2], v[3]);
+      } else {
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+          if (r + j < g.rows) o[j] = v[j];
+      }
+    }
+  }
+}
+
 // RMSNorm (when norm_w is set) and activation quantisation of one row per
 // workgroup: the GEMV prologue's arithmetic (TensorMath.Elementwise.cs:26-100,
 // TensorMath.cs:378-412), four values per thread per 1024-value chunk.
@@ -1184,6 +1340,20 @@ static hipError_t launch_gemm_tiles(const GemmArgs& g, hipStream_t s) {
   return hipGetLastError();
 }
 
+// Largest wave tile that still gives the chip about two waves per SIMD.
+template <class Scale>
+static hipError_t launch_gemm_short(const GemmArgs& g, hipStream_t s) {
+  const auto waves = [&](int rows, int frames) {
+    return (long)((g.rows + rows - 1) / rows) * ((g.frames + frames - 1) / frames);
+  };
+  const auto grid = [&](int rows, int frames) { return dim3((g.rows + rows - 1) / rows, (g.frames + frames - 1) / frames); };
+  constexpr long kWant = 2048;
+  if (waves(32, 32) >= kWant) q8_gemm_short_kernel<Scale, 2, 2><<<grid(64, 64), kGT, 0, s>>>(g);
+  else if (waves(32, 16) >= kWant) q8_gemm_short_kernel<Scale, 2, 1><<<grid(64, 32), kGT, 0, s>>>(g);
+  else q8_gemm_short_kernel<Scale, 1, 1><<<grid(32, 32), kGT, 0, s>>>(g);
+  return hipGetLastError();
+}
+
 // The largest tile that still loads the chip. Measured, us (64 x 64, 32 x 64,
 // 32 x 32 with stages of eight blocks; frames x K -> rows): 750 x 1024 -> 4096
 // 20.7 25.1 27.7; 500 x 2944 -> 6000 44.8 55.3 63.0; 375 x 1024 -> 4096 14.6 13.5
@@ -1192,18 +1362,47 @@ static hipError_t launch_gemm_tiles(const GemmArgs& g, hipStream_t s) {
 // the gate and up rows of 32 outputs (a prefill of all layers, ms: 750 rows 5.49
 // 5.61 5.75, 300 rows 2.94 3.04 3.03, 203 rows 2.51 2.45 2.52, 28 rows 1.96 1.88
 // 1.82; the third a 32 x 64 tile with stages of eight).
+enum GemmTile { k64x64, k32x64, k32x32 };
+template <int OUT>
+static GemmTile gemm_tile(const GemmArgs& g) {
+  const auto tiles = [&](int frames, int rows) { return ((g.frames + frames - 1) / frames) * ((g.rows + rows - 1) / rows); };
+  if (OUT == kGemmSwiGLU) return tiles(64, 32) >= 480 ? k64x64 : tiles(32, 32) >= 448 ? k32x64 : k32x32;
+  return tiles(64, 64) >= 512 ? k64x64 : tiles(32, 64) >= 448 ? k32x64 : k32x32;
+}
+
+// Where q8_gemm_short_kernel is the quicker one. Its prologue is shorter, which
+// counts for rows of few stages, it pads none to stages of eight blocks, and its
+// waves hold half the registers, which the fourth VALU operation of fp32 scales
+// needs. Measured over 3 to 750 frames and 300 to 6144 rows, time of
+// q8_gemm_kernel over that of q8_gemm_short_kernel (32 x 32 tiles, at most one a
+// CU; more; 32 x 64; 64 x 64): K of 128 1.2-1.5, 384 1.05-1.2 for all; 512 0.91-1.05,
+// 1.04-1.15, 0.93-1.07, 0.98-1.16; 640 0.93-1.12, 1.0-1.27, 0.97-1.17, 1.02-1.16; 768
+// 0.92-1.02, 0.97-1.2, 0.91-1.07, 0.97-1.09; 896 0.92-1.01, 1.0-1.15, 0.94-1.08,
+// 0.97-1.08; 1024 0.85-0.92, 0.87-1.11, 0.91-0.98, 0.94-1.05; 1152 0.91-1.01, 0.97-1.21,
+// 0.94-1.02, 0.95-1.07; 1280 0.84-0.97, 0.94-1.13, 0.91-1.0, 0.92-1.03; 2048 0.75-0.9,
+// 0.87-0.99, 0.88-0.96, 0.89-1.0. With fp32 scales the last is 1.05-1.38 for every K
+// from 2048 tiles of 32 x 32 on (450 x 2944 -> 4096, with 1920, 0.88).
+template <class Scale>
+static bool gemm_is_short(const GemmArgs& g) {
+  const int B = g.K / 32, small = ((g.frames + 31) / 32) * ((g.rows + 31) / 32);
+  if (B < 16 || B == 20) return true;
+  const bool half = sizeof(typename Scale::type) == 2;
+  switch (gemm_tile<kGemmPlain>(g)) {
+    case k64x64: return B < 24 || (!half && small >= 2048);
+    case k32x64: return B < 32 && !half;
+    default: return small > 256 && B <= 40 && B != 32;
+  }
+}
+
 template <class Scale, int OUT>
 static hipError_t launch_gemm_out(const GemmArgs& g, hipStream_t s) {
-  const auto tiles = [&](int frames, int rows) { return ((g.frames + frames - 1) / frames) * ((g.rows + rows - 1) / rows); };
-  if constexpr (OUT == kGemmSwiGLU) {
-    if (tiles(64, 32) >= 480) return launch_gemm_tiles<Scale, OUT, 2, 2, 2, 2, 4>(g, s);
-    if (tiles(32, 32) >= 448) return launch_gemm_tiles<Scale, OUT, 2, 2, 1, 2, 4>(g, s);
-    return launch_gemm_tiles<Scale, OUT, 2, 2, 1, 2, 8>(g, s);
-  } else {
-    if (tiles(64, 64) >= 512) return launch_gemm_tiles<Scale, OUT, 2, 2, 2, 2, 4>(g, s);
-    if (tiles(32, 64) >= 448) return launch_gemm_tiles<Scale, OUT, 2, 2, 1, 2, 4>(g, s);
-    return launch_gemm_tiles<Scale, OUT, 2, 2, 1, 1, 8>(g, s);
+  if constexpr (OUT == kGemmPlain) {
+    if (gemm_is_short<Scale>(g)) return launch_gemm_short<Scale>(g, s);
   }
+  const GemmTile tile = gemm_tile<OUT>(g);
+  if (tile == k64x64) return launch_gemm_tiles<Scale, OUT, 2, 2, 2, 2, 4>(g, s);
+  if (tile == k32x64) return launch_gemm_tiles<Scale, OUT, 2, 2, 1, 2, 4>(g, s);
+  return launch_gemm_tiles<Scale, OUT, 2, 2, 1, OUT == kGemmSwiGLU ? 2 : 1, 8>(g, s);
 }
 
 template <class Scale>

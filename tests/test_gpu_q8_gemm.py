@@ -25,12 +25,29 @@ def scales(rng, kind, rows, blocks):
     return s * np.float32(1.0001) if kind == "fp32" else s
 
 
-# Tiles of 32 x 32, 32 x 64 from 448 of them on, 64 x 64 from 512 on; stages of
-# eight blocks with four left over (K = 128, 384, 640).
+# Tiles of 32 x 32, 32 x 64 from 448 of them on, 64 x 64 from 512 on. Rows of less
+# than 512 and of 640 are q8_gemm_short_kernel's at any size, in tiles by the number of
+# waves.
 @pytest.mark.parametrize("frames,cols,rows", [(4, 128, 1), (31, 384, 33), (33, 640, 31), (65, 1024, 65), (225, 256, 3969),
                                               (449, 384, 2047), (513, 128, 4033), (1023, 640, 2049)])
 @pytest.mark.parametrize("kind", ["fp16", "fp32", "odd"])
 def test_tiles(backend, oracle_lib, frames, cols, rows, kind):
+    check_tiles(backend, oracle_lib, frames, cols, rows, kind)
+
+
+# Longer rows: stages of eight blocks with four left over (896, 1152, 1408) and
+# whole, up to 256 tiles of 32 x 32 and more (up to 1280 short rows, from 1408 on
+# not), 32 x 64 (short rows at 896 with fp32 scales) and 64 x 64 (with fp32 scales
+# from 2048 waves of 32 x 32 on).
+@pytest.mark.parametrize("frames,cols,rows", [(33, 896, 31), (512, 768, 512), (513, 768, 512), (300, 1280, 1000),
+                                              (300, 1408, 1000), (225, 896, 3969), (225, 1152, 3969), (513, 512, 4033),
+                                              (513, 768, 4033), (449, 768, 4033)])
+@pytest.mark.parametrize("kind", ["fp16", "fp32", "odd"])
+def test_longer_rows(backend, oracle_lib, frames, cols, rows, kind):
+    check_tiles(backend, oracle_lib, frames, cols, rows, kind)
+
+
+def check_tiles(backend, oracle_lib, frames, cols, rows, kind):
     from funasrnet_amd.model import Q8Tensor
     rng = np.random.default_rng(frames + cols)
     x = rng.standard_normal((frames, cols)).astype(np.float32)
@@ -50,7 +67,7 @@ def test_tiles(backend, oracle_lib, frames, cols, rows, kind):
 
 # Last scales that are infinite or overflow with the dot, where the last stage
 # of eight blocks has four left over, and where it has none.
-@pytest.mark.parametrize("cols", [128, 256, 384, 896])
+@pytest.mark.parametrize("cols", [128, 256, 384, 896, 1024, 1152])
 def test_last_scales(backend, oracle_lib, cols):
     from funasrnet_amd.model import Q8Tensor
     rng = np.random.default_rng(cols)
