@@ -509,10 +509,10 @@ __global__ __launch_bounds__(64 * WN * KS) void f32_split_gemm_kernel(
 // LDS reads. One order per shape: the same bits whichever entry point runs it.
 constexpr int kGK = 64;
 
-template <int BI, int BJ>
+template <int BI, int BJ, bool RELU>
 __global__ __launch_bounds__(256) void f32_gemm_kernel(const float* __restrict__ x, const float* __restrict__ w,
                                                        const float* __restrict__ bias, float* __restrict__ out, int M,
-                                                       int N, int K, int relu) {
+                                                       int N, int K) {
   constexpr int TM = 32 * BI, TN = 32 * BJ;              // workgroup tile
   constexpr int ROW = kGK + 4, KQ = kGK / 4;              // LDS row (floats); k values per lane group
   constexpr int PER_ROW = kGK / 4, ROWS = 256 / PER_ROW;  // 16-byte loads per row; rows per pass
@@ -599,7 +599,7 @@ __global__ __launch_bounds__(256) void f32_gemm_kernel(const float* __restrict__
         const int f = f0 + wm + 16 * i + 4 * lq + r;
         if (f < M) {
           float v = acc[i][j][r] + b;
-          if (relu) v = v < 0.0f ? 0.0f : v;  // (-0 and NaN pass, as the reference's `v < 0 ? 0 : v`)
+          if (RELU) v = v < 0.0f ? 0.0f : v;  // (-0 and NaN pass, as the reference's `v < 0 ? 0 : v`)
           out[(size_t)f * N + n] = v;
         }
       }
@@ -1502,11 +1502,12 @@ static hipError_t launch_f32_gemm(const float* x, const float* w, const float* b
   const int64_t big_cost = (int64_t)((big + 255) / 256) * 2, small_cost = (small + 255) / 256;
   const dim3 grid((N + 63) / 64, (M + 31) / 32);
   if (big_cost <= small_cost)
-    f32_gemm_kernel<2, 2><<<dim3((N + 63) / 64, (M + 63) / 64), 256, 0, s>>>(x, w, bias, out, M, N, K, relu);
+    (relu ? f32_gemm_kernel<2, 2, true> : f32_gemm_kernel<2, 2, false>)<<<dim3((N + 63) / 64, (M + 63) / 64), 256, 0, s>>>(
+        x, w, bias, out, M, N, K);
   else if (small <= 256 && K >= 256)
     f32_gemm_wavek_kernel<<<grid, 256, 0, s>>>(x, w, bias, out, M, N, K, relu);
   else
-    f32_gemm_kernel<1, 2><<<grid, 256, 0, s>>>(x, w, bias, out, M, N, K, relu);
+    (relu ? f32_gemm_kernel<1, 2, true> : f32_gemm_kernel<1, 2, false>)<<<grid, 256, 0, s>>>(x, w, bias, out, M, N, K);
   return hipGetLastError();
 }
 
@@ -1552,7 +1553,13 @@ hipError_t launch_f32_linear(const float* x, const float* w, const void* weight_
   // -> 50000 64 87; 333 x 192 -> 1100 7.4 5.8, 1000 x 128 -> 512 6.0 4.9, 64 x 64 ->
   // 2048 5.6 3.8, 64 x 224 -> 1100 6.5 6.4, 9 x 192 -> 2048 4.8 5.4, 2000 x 192 -> 2048
   // 16.7 24.3. (Odd K has no such tile: 333 x 65 -> 512 6.3 10.2.)
-  const bool tall = M <= 32 && N >= 28672, narrow = K <= 64 ? (int64_t)M * N <= 4000000 : K <= 192 && M > 16 && (int64_t)M * N <= 2100000;
+  // The latter up to 256 tiles of 64 x 128, and up to 64 columns also where they leave
+  // much of their last round idle (two a CU): of 64 -> 2048 1280 frames, 320 tiles, 9.8
+  // 9.5, 1500, 384 tiles, 9.8 12.6, 2560, 640 tiles, 16.3 17.8; of 64 -> 3072 1500, 576
+  // tiles, 16.6 13.9; 40 of 64 -> 50000 8.8 11.3.
+  const int64_t wide = (int64_t)((M + 63) / 64) * ((N + 127) / 128);
+  const bool tall = M <= 32 && N >= 28672;
+  const bool narrow = wide <= 256 ? K <= 64 || (K <= 192 && M > 16) : K <= 64 && (wide <= 320 || (wide > 512 && wide <= 600));
   if (!weight_planes || (K % 4 == 0 && (tall || narrow)))
     return launch_f32_gemm(x, w, bias, out, M, N, K, relu, s);
   const uint4* planes = static_cast<const uint4*>(weight_planes);
@@ -1572,7 +1579,6 @@ hipError_t launch_f32_linear(const float* x, const float* w, const void* weight_
   // 57.5 63.4 82.4; 4000 x 512 -> 2048 68.9 55.9 74.6 91.7; 1000 x 512 -> 1536
   // 17.2 17.5 16.3 20.5; 333 x 560 -> 1536 18.8 18.0 12.1 12.9; 300 x 1023 ->
   // 700 40.5 38.9 21.3 19.0; 20 x 512 -> 1024 14.4 14.2 8.2 7.1.
-  const int wide = tiles(64, 128);
   if (wide > 256) FAH_SPLIT(4, 1, 2, 1, 1, 2);
   else if (wide >= 224) FAH_SPLIT(4, 2, 2, 1, 2, 2);
   else if (tiles(32, 64) >= 128) FAH_SPLIT(2, 2, 1, 1, 2, 2);

@@ -44,12 +44,13 @@ def test_split_tiles(backend, frames, cols, rows, biased):
 
 
 # The same tiles above 192 columns and at odd widths, and either side of the sizes
-# that fp32 MFMA takes: up to 64 columns and 4,000,000 results, up to 192 and
-# 2,100,000 from 17 frames on, and up to 32 frames of 28,672 rows or more.
+# that fp32 MFMA takes: up to 256 tiles of 64 x 128 of 192 columns from 17 frames on,
+# up to 320 and 513 to 600 of 64 columns, and up to 32 frames of 28,672 rows or more.
 @pytest.mark.parametrize("frames,cols,rows", [(9, 193, 33), (31, 200, 31), (33, 257, 33), (64, 260, 65), (511, 196, 500),
                                               (513, 225, 511), (1023, 196, 1793), (2100, 199, 1100), (17, 65, 40),
                                               (16, 192, 31), (17, 192, 31), (1000, 192, 2100), (1001, 192, 2100),
-                                              (2000, 64, 2000), (2001, 64, 2000), (32, 196, 28672), (33, 196, 28672)])
+                                              (2000, 64, 2000), (1280, 64, 2048), (1281, 64, 2048), (2048, 64, 2048),
+                                              (2049, 64, 2048), (2432, 64, 2000), (1300, 64, 3600), (32, 196, 28672), (33, 196, 28672)])
 def test_gemm_choice(backend, frames, cols, rows):
     rng = np.random.default_rng(cols)
     x = rng.standard_normal((frames, cols)).astype(np.float32)
