@@ -403,10 +403,11 @@ struct fah_weight {
   DeviceBuffer q, s;
   int group_rows = 1;
   // FP32 weight (Weight.Values): `f` holds [rows][cols] floats
-  // (fah::f32_weight_bytes), `planes` their bf16 planes (empty where there are
-  // none), q/s unused.
+  // (fah::f32_weight_bytes) and after them their bf16 planes, if it has any
+  // (`planes`), q/s unused.
   bool f32 = false;
-  DeviceBuffer f, planes;
+  DeviceBuffer f;
+  void* planes = nullptr;
 };
 
 struct DeviceMatrix {
@@ -1613,7 +1614,7 @@ int fah_weight_release(fah_weight* w) {
 }
 
 int64_t fah_weight_device_bytes(const fah_weight* w) {
-  return w ? (int64_t)(w->q.bytes + w->s.bytes + w->f.bytes + w->planes.bytes) : 0;
+  return w ? (int64_t)(w->q.bytes + w->s.bytes + w->f.bytes) : 0;
 }
 
 int fah_weight_f32_upload(fah_context* h, const float* values, int rows, int cols, fah_weight** out) {
@@ -1631,17 +1632,28 @@ int fah_weight_f32_upload(fah_context* h, const float* values, int rows, int col
     w->rows = rows;
     w->cols = cols;
     w->f32 = true;
-    w->f.allocate(fah::f32_weight_bytes(rows, cols));
+    // Without planes (no memory left for them, among others) the weight runs on fp32
+    // MFMA. One allocation for both: releasing one of a few MiB takes 240 us.
+    const size_t held = fah::f32_weight_bytes(rows, cols), planes = fah::f32_planes_bytes(rows, cols);
+    if (planes && w->f.try_allocate(held + planes)) w->planes = w->f.as<char>() + held;
+    else w->f.allocate(held);
     check(hipMemcpyAsync(w->f.ptr, values, (size_t)rows * cols * 4, hipMemcpyHostToDevice, c->stream), "H2D weight");
-    // Without planes (no memory left for them, among others) the weight runs on fp32 MFMA.
     int outside = 0;
-    if (w->planes.try_allocate(fah::f32_planes_bytes(rows, cols))) {
-      check(fah::launch_f32_split(w->f.as<float>(), rows, cols, w->planes.ptr, c->stream), "split weight");
+    if (w->planes) {
+      check(fah::launch_f32_split(w->f.as<float>(), rows, cols, w->planes, c->stream), "split weight");
       check(hipMemcpyAsync(&outside, fah::f32_weight_outside(w->f.as<float>(), rows, cols), 4, hipMemcpyDeviceToHost, c->stream),
             "D2H range");
     }
     check(hipStreamSynchronize(c->stream), "hipStreamSynchronize");
-    if (outside) w->planes.release();
+    if (outside) {
+      w->planes = nullptr;
+      DeviceBuffer alone;
+      if (alone.try_allocate(held)) {
+        check(hipMemcpyAsync(alone.ptr, w->f.ptr, held, hipMemcpyDeviceToDevice, c->stream), "D2D weight");
+        check(hipStreamSynchronize(c->stream), "hipStreamSynchronize");
+        w->f = std::move(alone);
+      }
+    }
     *out = w.release();
     return FAH_OK;
   });
@@ -1836,7 +1848,7 @@ int fah_linear_many(fah_context* h, const float* input, int frames, const fah_we
       // through the same kernel as fah_linear, so the bits equal separate calls.
       size_t at = 0;
       for (int i = 0; i < count; ++i) {
-        check(fah::launch_f32_linear(c->in.as<float>(), weights[i]->f.as<float>(), weights[i]->planes.ptr, nullptr,
+        check(fah::launch_f32_linear(c->in.as<float>(), weights[i]->f.as<float>(), weights[i]->planes, nullptr,
                                      c->out.as<float>() + at, frames, weights[i]->rows, cols, false, c->stream),
               "f32 linear");
         at += (size_t)frames * weights[i]->rows;
@@ -1900,7 +1912,7 @@ int fah_linear(fah_context* h, const float* input, int frames, const fah_weight*
       check(hipMemcpyAsync(dbias, bias, (size_t)w->rows * 4, hipMemcpyHostToDevice, c->stream), "H2D bias");
     }
     meter.kernels_begin();
-    check(fah::launch_f32_linear(c->in.as<float>(), w->f.as<float>(), w->planes.ptr, dbias, c->out.as<float>(), frames,
+    check(fah::launch_f32_linear(c->in.as<float>(), w->f.as<float>(), w->planes, dbias, c->out.as<float>(), frames,
                                  w->rows, w->cols, false, c->stream),
           "f32 linear");
     meter.kernels_end();
@@ -1923,7 +1935,7 @@ int fah_linear_device(fah_context* h, const float* x, int frames, const fah_weig
     if (c->disposed) return fail(FAH_ERROR_DISPOSED, "context disposed");
     check(hipSetDevice(c->device), "hipSetDevice");
     DeviceWork work(*c);
-    check(fah::launch_f32_linear(x, w->f.as<float>(), w->planes.ptr, bias, out, frames, w->rows, w->cols, false, c->stream),
+    check(fah::launch_f32_linear(x, w->f.as<float>(), w->planes, bias, out, frames, w->rows, w->cols, false, c->stream),
           "f32 linear");
     return FAH_OK;
   });
@@ -1963,9 +1975,9 @@ int fah_relu_projection(fah_context* h, const float* input, int frames, const fa
     float* dout = reinterpret_cast<float*>(c->out.as<char>() + mid_bytes);
     // The intermediate stays on the device (IReluProjectionBackend.cs:4-16).
     meter.kernels_begin();
-    check(fah::launch_f32_linear(c->in.as<float>(), first->f.as<float>(), first->planes.ptr, d1, mid, frames, H, K, true, c->stream),
+    check(fah::launch_f32_linear(c->in.as<float>(), first->f.as<float>(), first->planes, d1, mid, frames, H, K, true, c->stream),
           "f32 linear + ReLU");
-    check(fah::launch_f32_linear(mid, second->f.as<float>(), second->planes.ptr, d2, dout, frames, N, H, false, c->stream), "f32 linear");
+    check(fah::launch_f32_linear(mid, second->f.as<float>(), second->planes, d2, dout, frames, N, H, false, c->stream), "f32 linear");
     meter.kernels_end();
     check(hipMemcpyAsync(output, dout, out_bytes, hipMemcpyDeviceToHost, c->stream), "D2H output");
     work.release();  // enqueued: other contexts may enqueue while this stream drains

@@ -250,11 +250,11 @@ hipError_t launch_session_embed(const int8_t* q, const void* scales, bool half_s
                                 const SessionRef* sessions, int count, float* x, hipStream_t s);
 
 
-// FP32 weights [N][K]: an allocation of f32_weight_bytes that holds the values
-// first, and one of f32_planes_bytes (0: none for such widths) for their bf16
+// FP32 weights [N][K]: f32_weight_bytes of memory (a multiple of 16) that holds the
+// values first, and f32_planes_bytes (0: none for such widths) for their bf16
 // planes. launch_f32_split fills in the planes and the word that
-// f32_weight_outside points to (on the device; not 0: the planes do not hold
-// the values and are not to be used).
+// f32_weight_outside points to (on the device; not 0: the planes do not hold the
+// values and are not to be used).
 size_t f32_weight_bytes(int64_t rows, int cols);
 size_t f32_planes_bytes(int64_t rows, int cols);
 const int* f32_weight_outside(const float* w, int64_t rows, int cols);
