@@ -54,11 +54,11 @@ typedef float floatx4_any __attribute__((ext_vector_type(4), aligned(4)));
 // .. + 7; result register r of lane l: row 8 (r / 4) + 4 (l / 32) + r % 4,
 // column l % 32.
 //
-// Measured against the fp32 MFMA kernel before it (fp32 sums of 64 x 64 tiles),
-// us: 1000 x 512 -> 2048 25.3 -> 19.5, 333 x 560 -> 1536 17.2 -> 11.8, 4000 x
-// 2048 -> 512 84.7 -> 54.1, 300 x 1023 -> 700 170 -> 19.2; error against 64 bits
+// Measured against the fp32 MFMA kernel for all weights (fp32 sums of 64 x 64 tiles),
+// us: 1000 x 512 -> 2048 25.4 -> 18.6, 333 x 560 -> 1536 17.2 -> 11.5, 4000 x
+// 2048 -> 512 85 -> 52, 300 x 1023 -> 700 77 -> 18; error against 64 bits
 // (2-norm) 4.0e-7 -> 0.97e-7, 4.2e-7 -> 1.0e-7, 8.1e-7 -> 1.9e-7, 5.7e-7 ->
-// 1.0e-7. Of the 19.5, the MFMAs take 6.2 (at the 2.0 GHz seen), the 8 MB of
+// 1.0e-7. Of the 18.6, the MFMAs take 6.2 (at the 2.0 GHz seen), the 8 MB of
 // stores 3, the launch, first loads and epilogue the rest.
 //
 // Range: a weight is split only if its values, but zeros, lie in [kSplitTiny,
@@ -1181,8 +1181,8 @@ __global__ __launch_bounds__(256) void f32_attention_mfma_kernel(const float* __
 // cycles) and, for short inputs, by launches and first loads. One wave a SIMD
 // (402 registers at 128: eight operand groups, 1 to 1.5 us of MFMAs, are on
 // their way; four measured 176 us where eight take 169). Measured against
-// attention_tile_f32 for all: 4096 frames of 4 x 128 569 -> 169 us, 1864 133 ->
-// 54, 1000 44 -> 32, 1100 of 8 x 96 984 -> 43 (it ran on the VALU); error against
+// attention_tile_f32 for all: 4096 frames of 4 x 128 569 -> 171 us, 1864 133 ->
+// 57, 1000 42 -> 30, 1100 of 8 x 96 945 -> 45 (it ran on the VALU); error against
 // 64 bits 7.2e-7 -> 4.1e-7 (4096), 5.0e-7 -> 1.7e-7 (1000).
 //
 // Values outside [2^-100, 2^60] in magnitude, but zero, set the head's word in

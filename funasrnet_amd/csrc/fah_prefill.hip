@@ -54,8 +54,9 @@ __device__ __forceinline__ int gate_up_row(int r, int kind, int base, int extra)
 // tiles, a workgroup WF x WR of them. SwiGLU waves hold 8 TJ gate rows (tiles
 // 0 .. TJ / 2 - 1) and the matching up rows.
 //
-// What bounds it: the ordered fp32 steps, at three VALU operations a row, frame
-// and block. The dots' MFMA starts from 0x4b400000, the bits of 1.5 2^23, so
+// What bounds it: at the largest sizes the VALU, mostly with the ordered fp32
+// steps, three operations a row, frame and block; below, the serial block chain
+// of a wave. The dots' MFMA starts from 0x4b400000, the bits of 1.5 2^23, so
 // that its integer result is, as a float, 1.5 2^23 + dot exactly; with c =
 // -1.5 2^23 w_scale (exact: w_scale has 11 bits), fma(result, w_scale, c) is
 // dot w_scale rounded once, what (float)dot * w_scale is, without the
@@ -72,10 +73,11 @@ __device__ __forceinline__ int gate_up_row(int r, int kind, int base, int extra)
 //
 // Measured against the four-operation kernel with rows as the MFMA's rows, us:
 // 28 x 2048 -> 1024 9.2 -> 7.2, 100 x 3072 -> 1024 12.9 -> 9.6, 375 x 3072 -> 1024
-// 15.7 -> 13.8, 375 x 1024 -> 4096 13.9 -> 13.5, 500 x 2944 -> 6000 50.5 -> 44.8. At
-// the largest the VALU is busy for two thirds of the CU's time and the MFMAs
-// for a sixth; below, the serial block chain of a wave (about 110 cycles a
-// block of 16 x 16) is what is left. Weights read straight from memory in the
+// 15.7 -> 13.8, 500 x 2944 -> 6000 50.5 -> 44.8; 375 x 1024 -> 4096 is unchanged (16.0
+// with the quantisation before it). At the largest the VALU is busy for two thirds
+// of the CU's time and the MFMAs for a sixth; for a few hundred frames the VALU's
+// share is 35 to 60% (375 x 1024 -> 4096: 42% of 14.3 us), and the block chain of a
+// wave (about 110 cycles a block of 16 x 16) is what is left. Weights read straight from memory in the
 // operand's order (32 bytes a row and load) took two to three times as long.
 constexpr int kMagicBits = 0x4b400000;
 constexpr float kMagic = 12582912.0f;  // 1.5 2^23
@@ -1418,8 +1420,8 @@ hipError_t launch_gemm_scaled(const GemmArgs& g, int out, hipStream_t s) {
 }  // namespace
 
 hipError_t launch_gemm(const GemmArgs& g, bool half_scales, int out, hipStream_t s) {
-  // Operands and scales move through LDS in stages of four blocks, so K only
-  // bounds the int32 offsets; 3072 is the widest decoder matrix.
+  // Operands and scales move through LDS in stages of four or eight blocks, so K
+  // only bounds the int32 offsets; 3072 is the widest decoder matrix.
   if (g.K % 128 != 0 || g.K > 3072 || g.rows < 1 || g.frames < 1) return hipErrorInvalidValue;
   if (out == kGemmSwiGLU && !g.gu_map && (g.split_base < 1 || g.split_extra < 0)) return hipErrorInvalidValue;
   if (g.out_q && (out != kGemmSwiGLU || g.rows % 32 != 0 || !g.out_s)) return hipErrorInvalidValue;
@@ -1537,9 +1539,10 @@ hipError_t launch_attn_prefill(const PrefillAttnArgs& args, hipStream_t s) {
   // Many rows of one cache (a prefill): blocks of rows share K/V reads.
   if (!a.sessions && a.heads == 2 * a.kv_heads && a.frames >= 2 * kRowBlock && rows_lds_bytes(n) <= kStageLds) {
     // Up to two workgroups a CU, the time is that of the last rows' workgroup,
-    // which eight waves shorten (375 rows: 49.5 -> 39 us a layer); with more, two
-    // workgroups of four waves a CU fill each other's waits (prefill of 750 rows
-    // 5.6 ms against 6.3; 500 rows, 504 workgroups, 4.76 and 4.68).
+    // which eight waves shorten; with more, two workgroups of four waves a CU fill
+    // each other's waits. A prefill with eight and with four waves, ms: 200 rows 2.36
+    // 2.44, 375 3.26 3.48, 500 (504 workgroups) 3.77 3.84, 520 4.49 4.45, 600 4.83 4.67,
+    // 750 5.83 5.34.
     return a.kv_heads * ((a.frames + kRowBlock - 1) / kRowBlock) <= 512 ? launch_attn_rows<512>(a, n, s)
                                                                         : launch_attn_rows<256>(a, n, s);
   }
