@@ -1445,10 +1445,14 @@ static int few_rows(int rows, int K, int frames, int out) {
 // took 61 us for 151936 rows of 1024, staged in LDS with 128-byte reads of a row
 // 44 (16 sessions 1.011 -> 0.994 ms a step, 8 0.864 -> 0.843). Fewer frames are
 // quicker in q8_gemm_few_kernel (7 sessions 0.827 and 0.829, 2 0.766 and 0.772),
-// and so are the layers' projections, whose 256 to 384 tiles leave the chip idle.
-constexpr int kHeadRows = 128;
+// and so are the layers' projections, whose 256 to 384 tiles leave the chip idle,
+// and small vocabularies (a step of one layer and the head with 8 and 16 sessions, GEMM and
+// few-frame kernel: 1024 -> 4096 59.5 55.5, 67.8 64.3; -> 8192 59.6 56.0, 68.2 68.3;
+// -> 12288 59.5 57.0, 68.5 68.7; -> 16384 60.6 58.2, 69.5 75.3).
+constexpr int kHeadRows = 128, kHeadLeastRows = 12288;
 static int head_groups(int rows, int K, int frames, int out) {
   if (out != kGemmGreedy || frames < 8 || frames > 16 || K % 128 != 0 || K > 3072 || rows < 16) return 0;
+  if (rows < kHeadLeastRows && K <= kFewMaxK && few_rows(rows, K, frames, out)) return 0;
   return (rows + kHeadRows - 1) / kHeadRows;
 }
 

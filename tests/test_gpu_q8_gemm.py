@@ -86,10 +86,10 @@ def test_last_scales(backend, oracle_lib, cols):
     assert np.array_equal(out[~nan].view(np.uint32), expected[~nan].view(np.uint32))
 
 
-# The lm_head of lock-step sessions: the few-frame kernel up to seven, the GEMM
-# from eight on; vocabularies that end inside a workgroup's 128 rows.
+# The lm_head of lock-step sessions: the few-frame kernel up to seven and below
+# 12,288 rows, else the GEMM; vocabularies that end inside a workgroup's 128 rows.
 @pytest.mark.parametrize("count", [7, 8, 13, 16])
-@pytest.mark.parametrize("vocab", [33, 4001])
+@pytest.mark.parametrize("vocab", [33, 4001, 12287, 12288, 12389])
 def test_session_heads(backend, count, vocab):
     from funasrnet_amd import model
     from funasrnet_amd.hip import HipDecoder
